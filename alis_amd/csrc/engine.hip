@@ -47,13 +47,6 @@ int fail(const std::string &what)
 
 #define HIPCHECK(call) do { hipError_t e_ = (call); if (e_ != hipSuccess) return fail(#call, e_); } while (0)
 
-#ifndef TPB_TILE
-#define TPB_TILE 1
-#endif
-#ifndef K_SHUFFLE
-#define K_SHUFFLE true       // k_curl: k neighbours passed between lanes (see curl_cell.inc, KSH)
-#endif
-constexpr int ROW_ALIGN_BYTES = 128;
 constexpr int MAXPOLE = ALIS_DEV_MAXPOLES;
 
 // Index map of one device array: (i - i0)*si + (j - j0)*sj + (k - k0) + koff.
@@ -83,16 +76,6 @@ template<class T> struct Quad;
 template<> struct Quad<float> { typedef float V __attribute__((vector_size(16))); };
 template<> struct Quad<double> { typedef double V __attribute__((vector_size(32))); };
 
-template<class T> struct CurlFace {
-	T *pa, *pb;                 // the two auxiliary components of this face
-	T *qa, *qb;                 // where their new values go (the same arrays but in k_step
-	                            // and k_fix, which write the world's other set of arrays)
-	const T *bc;                // recursion coefficients (b, ca, cb, 0) along the face axis
-	                            // (index - MIN), four to an index for one vector load
-	Lay L;
-	int lo, hi, on;
-};
-
 // A dispersive object as the kernels see it (device memory, one table per world):
 // its box clipped to the grid, the compact layout of its arrays, pole coefficients,
 // fill factors on the staggered E positions and the J/K currents per real/imaginary part.
@@ -117,29 +100,6 @@ template<class T> struct PhsZ {
 };
 constexpr int MAXZS = 4;
 
-template<class T> struct CurlArgs {
-	T *F0, *F1, *F2;
-	T *O0, *O1, *O2;            // where the new values go (F* but in k_step and k_fix)
-	const T *G0, *G1, *G2;
-	const T *C0, *C1, *C2;
-	const typename Quad<T>::V *seg;  // k_curl E: per 64-cell row segment (tile), 1/eps
-	                            // (x, y, z, 1) when the segment holds one triple, else 0s
-	const T *dtx, *dty, *dtz;   // dt/d along each axis, index - MIN
-	Lay L;
-	int iMIN, jMIN, kMIN, ni, nj, nk;
-	int alt;                    // +1: E from H, -1: H from E
-	CurlFace<T> face[6];        // xMin yMin zMin xMax yMax zMax
-	const ObjDev<T> *obj;       // dispersive objects (E: scaling and -sum J before the curl;
-	int nobj, m;                //  H: current update on the new E), part m
-	const ObjDev<T> *objOut;    // the table whose currents receive the new values (obj but
-	                            //  in k_step and k_fix)
-	const int *otStart;         // per 64 x 4 tile (k_curl's tiles): its objects are
-	const int *otList;          //  otList[otStart[t] .. otStart[t+1]) ascending; null: all
-	int flatPitch;              // batched launches of packed short rows: row length with ghosts
-	int nzs;                    // H launches of k_curl: phaser z faces to sample (see PhsZ)
-	PhsZ<T> zs[MAXZS];
-};
-
 // Fields and coefficients live in global memory, but to the compiler a pointer that a kernel
 // loads from memory (the batched launches' argument tables) is generic, and generic (flat)
 // accesses cost more than global ones (about 20 % on a batched 256^3 curl): the cell update
@@ -153,186 +113,8 @@ template<class T> __device__ inline __attribute__((address_space(1))) T *glb(T *
 	return (__attribute__((address_space(1))) T *)p;
 }
 
-// Streaming access: arrays touched once per launch (the updated field, 1/eps, CPML psi)
-// are read and written non-temporally so they do not displace the other field's rows and
-// planes, which neighbouring workgroups read again from L2.
-template<bool NT, class T> __device__ inline T ldS(const T *p)
-{
-	if (NT) return __builtin_nontemporal_load(glb(p));
-	return *glb(p);
-}
-template<bool NT, class T> __device__ inline void stS(T *p, T v)
-{
-	if (NT) __builtin_nontemporal_store(v, glb(p));
-	else *glb(p) = v;
-}
-
-// Curl update of one half step plus the CPML slabs (src/update.c:48-125).  One thread per
-// cell; 64 lanes along z, 4 rows along y per workgroup, one x plane per grid z index.
-// NT: non-temporal access to the single-use arrays; NTG also to the centre values of the
-// other field.
-// BY: rows along y per workgroup (64 x BY threads).  ROWS: a one-dimensional grid that
-// deals rows (the tiles along k of one block of BY rows in one x plane) to the 8 XCDs in turn,
-// every tile of a row on one XCD in consecutive slots, so that the line a tile reads beyond
-// its last k is fetched into the L2 that the next tile reads it from (the dispatcher deals
-// consecutive workgroup ids to XCDs in turn; with the plain grid the tiles of a row land on
-// different XCDs).  Measured on the 256^3 nanoblock: H 139.8 -> 137.1 us, E unchanged
-// (149 us either way, so E keeps the plain grid); groups of 2 or 4 rows per XCD, which would
-// also keep the j+1 row local, lose 5-11 %.
-
-template<class T, int CM, bool NT = true, bool NTG = false, bool MZ = false, bool PC = false>
-__device__ __forceinline__ void curlAt(const CurlArgs<T> &a, int i, int j, int k, T (&coef)[6]);
-template<class T, int CM, bool NT, bool MZ>
-__device__ __forceinline__ void curlAtGiven(const CurlArgs<T> &a, int i, int j, int k, const T (&coef)[6]);
-
-// Cell (bx, by, bz) of a 64 x 4 tile, of part a (PAIR: then of part *b, the imaginary part of
-// the same world).
-template<class T, int CM, bool PAIR>
-__device__ __forceinline__ void curlCell(const CurlArgs<T> &a, const CurlArgs<T> *b, int bx, int by, int bz)
-{
-	const int k = a.kMIN + bx * 64 + (int)threadIdx.x;
-	const int j = a.jMIN + by * 4 + (int)threadIdx.y;
-	const int i = a.iMIN + bz;
-	if (k >= a.kMIN + a.nk || j >= a.jMIN + a.nj) return;
-	T coef[6];
-	curlAt<T, CM>(a, i, j, k, coef);
-	if (PAIR) curlAtGiven<T, CM, true, false>(*b, i, j, k, coef);
-}
-
-// The update of cell (i, j, k) in batched launches: the CPML faces reuse the curl's
-// neighbour values, and the psi slabs go through the cache (the short rows of small worlds
-// cover a slab with partial lines that neighbouring tiles complete).  Measured on 64 k-point
-// worlds: 5 % (E) and 14 % (H) faster than reloading and streaming; slower in k_curl.
-template<class T, int CM, bool NT, bool NTG, bool MZ, bool PC>
-__device__ __forceinline__ void curlAt(const CurlArgs<T> &a, int i, int j, int k, T (&coef)[6])
-{
-	constexpr bool SHARE = true, NTP = false, MERGEZ = MZ, UNI = !MZ, SEP = false, wr = true, NTC = NT && !PC;
-	constexpr int KSH = 0;
-#include "curl_cell.inc"
-	coef[0] = dx, coef[1] = dy, coef[2] = dz, coef[3] = cx, coef[4] = cy, coef[5] = cz;
-}
-
-// The same for the imaginary part of a Bloch world in the thread that updated the real part:
-// dt/d and 1/eps are the real part's (coef), not loaded again.
-template<class T, int CM, bool NT, bool MZ>
-__device__ __forceinline__ void curlAtGiven(const CurlArgs<T> &a, int i, int j, int k, const T (&coef)[6])
-{
-	constexpr bool NTG = false, SHARE = true, NTP = false, MERGEZ = MZ, UNI = !MZ, SEP = false, wr = true, NTC = NT;
-	constexpr int KSH = 0;
-#define CURL_COEF
-#include "curl_cell.inc"
-#undef CURL_COEF
-}
-
-template<class T, int CM, bool ROWS, bool NT = true, bool NTG = false, int BY = 4, bool ZS = false, bool KSHUF = K_SHUFFLE>
-__global__ __launch_bounds__(64 * BY) void k_curl(CurlArgs<T> a)
-{
-	int bx = (int)blockIdx.x, by = (int)blockIdx.y, bz = (int)blockIdx.z;
-	if (ROWS) {
-		// workgroup w: XCD w % 8, its slot s = w / 8; row r = (s / nkb) * 8 + w % 8
-		const int nkb = (a.nk + 63) / 64, njb = (a.nj + BY - 1) / BY;
-		const int w = (int)blockIdx.x, s = w >> 3, r = (s / nkb) * 8 + (w & 7);
-		if (r >= njb * a.ni) return;
-		bx = s % nkb, by = r % njb, bz = r / njb;
-	}
-	const int k = a.kMIN + bx * 64 + (int)threadIdx.x;
-	const int j = a.jMIN + by * BY + (int)threadIdx.y;
-	const int i = a.iMIN + bz;
-	if (k >= a.kMIN + a.nk || j >= a.jMIN + a.nj) return;
-	constexpr bool SHARE = false, NTP = NT, MERGEZ = false, UNI = true, SEP = false, wr = true, NTC = NT;
-	// E only: the H launch (previous lane, lane 0 loading) measured 137.8 -> 145.7 us with it,
-	// the E launch 147.8 -> 146.6 us (256^3 nanoblock)
-	constexpr int KSH = KSHUF && !ROWS ? 1 : 0;
-#include "curl_cell.inc"
-	// H: the samples of the phasers' z faces from the values at hand -- the new H here and at
-	// k + 1 (the next lane: the host takes faces whose k + 1 lies in the same wavefront) and E,
-	// final after its end-of-half-step program -- in place of k_phs_sample reading a strided
-	// plane (the host takes faces that the H program does not change)
-	if (ZS && ROWS) {
-		for (int z = 0; z < a.nzs; z++) {
-			const PhsZ<T> &Z = a.zs[z];
-			// the wavefront's row and 64 cells (bx) hold a sampled cell of the face: the same
-			// for all its lanes, so only these waves exchange values
-			if (i < Z.si0 || i > Z.si1 || j < Z.sj0 || j > Z.sj1 || (Z.k - a.kMIN) >> 6 != bx) continue;
-			const T hx1 = __shfl_down(fx, 1), hy1 = __shfl_down(fy, 1);
-			if (k != Z.k) continue;
-			const long t = Z.base + (long)(i - Z.i0) * (Z.j1 - Z.j0 + 1) + (j - Z.j0);
-			T *const q = Z.slot;
-			q[t] = gx, q[Z.cells + t] = gy, q[2 * Z.cells + t] = fx + hx1, q[3 * Z.cells + t] = fy + hy1;
-		}
-	}
-}
-
-// The entry owning workgroup b of a batch launch: start[] is increasing; every wave finds it
-// with one load per lane and a ballot (no chain of dependent loads).
-__device__ __forceinline__ int batchEntry(const int *start, int n, int b)
-{
-	int e = 0;
-	for (int c = 0; c < n; c += 64) {
-		const int q = c + (int)__lane_id();
-		const unsigned long long m = __ballot(q < n && start[q] <= b);
-		if (!m) break;
-		e = c + __popcll(m) - 1;
-		if (__popcll(m) < 64) break;
-	}
-	return __builtin_amdgcn_readfirstlane(e);
-}
-
-// Several worlds (and real/imaginary parts) in one launch: entry e owns workgroups
-// [start[e], start[e+1]) of a one-dimensional grid; each workgroup updates TPB consecutive
-// tiles of its entry (tiles as in k_curl).
-// FLAT: 1 or 0 when every entry of the launch has packed rows or none has; CM: 2 when every
-// entry takes 1/eps from its per-segment table (and arrays where a segment is mixed), 1 when
-// every entry reads 1/eps arrays, 0 when none does; -1 to decide per entry.  Specialised
-// launches compile to leaner code (64 k-point worlds: E curl 380 -> 332 us); the host runs
-// one launch per class of entries.  H launches (alt < 0), which read the next plane of E, run each entry's
-// tiles in descending order, so that plane was read as a centre just before (64 k-point
-// worlds: H curl 331 -> 306 us; the 256^3 k_curl shows no difference).
-// PAIR: every entry is both parts of a Bloch world (arguments 2e and 2e + 1, one geometry):
-// each thread updates its cell of the real part and then of the imaginary part, which reads
-// the same 1/eps values again, from the cache (the real part loads them cached).
-template<class T, int TPB, int FLAT = -1, int CM = -1, bool PAIR = false>
-__global__ __launch_bounds__(256) void k_curl_batch(const CurlArgs<T> *__restrict__ args, const int *__restrict__ start, int n)
-{
-	const int b = (int)blockIdx.x;
-	const int e = batchEntry(start, n, b);
-	const CurlArgs<T> &a = args[PAIR ? 2 * e : e];
-	if (FLAT == 1 || (FLAT < 0 && a.flatPitch)) {
-		// packed rows shorter than a wavefront: a tile is 256 consecutive cells of one x
-		// plane from the plane's first (ghost) row on (ghost rows, row ghosts and plane
-		// padding included, their lanes idle), so the lanes of a wavefront stay busy across
-		// row ends; planes are padded to 256 bytes, so every wavefront's access is aligned
-		const int pitch = a.flatPitch, per = (int)((a.L.si + 255) / 256), tiles = per * a.ni;
-		const int lid = (int)(threadIdx.y * 64 + threadIdx.x);
-		for (int t0 = (b - start[e]) * TPB, t1 = min(t0 + TPB, tiles); t0 < t1; t0++) {
-			const int t = a.alt < 0 ? tiles - 1 - t0 : t0;
-			const int off = (t % per) * 256 + lid, jj = off / pitch - 1, kk = off - (jj + 1) * pitch;
-			if (jj < 0 || jj >= a.nj || kk < 1 || kk > a.nk) continue;
-			const int i = a.iMIN + t / per, j = a.jMIN + jj, k = a.kMIN - 1 + kk;
-			T coef[6];
-			const int cm = CM >= 0 ? CM : a.seg ? 2 : a.C0 ? 1 : 0;
-			if (cm == 2) curlAt<T, 2, true, false, true, PAIR>(a, i, j, k, coef);
-			else if (cm == 1) curlAt<T, 1, true, false, true, PAIR>(a, i, j, k, coef);
-			else curlAt<T, 0, true, false, true, PAIR>(a, i, j, k, coef);
-			if (PAIR) {
-				// the imaginary part: the same world's dt/d and 1/eps
-				const CurlArgs<T> &a1 = args[2 * e + 1];
-				if (cm == 2) curlAtGiven<T, 2, true, true>(a1, i, j, k, coef);
-				else if (cm == 1) curlAtGiven<T, 1, true, true>(a1, i, j, k, coef);
-				else curlAtGiven<T, 0, true, true>(a1, i, j, k, coef);
-			}
-		}
-		return;
-	}
-	const int nkb = (a.nk + 63) / 64, njb = (a.nj + 3) / 4, tiles = nkb * njb * a.ni;
-	for (int t0 = (b - start[e]) * TPB, t1 = min(t0 + TPB, tiles); t0 < t1; t0++) {
-		const int t = a.alt < 0 ? tiles - 1 - t0 : t0;
-		const int bx = t % nkb, by = (t / nkb) % njb, bz = t / (nkb * njb);
-		if (CM == 2 || (CM < 0 && a.seg)) curlCell<T, 2, PAIR>(a, args + 2 * e + 1, bx, by, bz);
-		else if (CM == 1 || (CM < 0 && a.C0)) curlCell<T, 1, PAIR>(a, args + 2 * e + 1, bx, by, bz);
-		else curlCell<T, 0, PAIR>(a, args + 2 * e + 1, bx, by, bz);
-	}
-}
+#include "curl_quads.inc"
+#include "objects.inc"
 
 __device__ inline void boxCell(long t, int ni, int nj, int nk, int &di, int &dj, int &dk)
 {
@@ -341,135 +123,6 @@ __device__ inline void boxCell(long t, int ni, int nj, int nk, int &di, int &dj,
 	dj = (int)(r % nj);
 	di = (int)(r / nj);
 	(void)ni;
-}
-
-// One time step of a world in one pass (the curl halves of src/update.c:275-341): the E
-// update and then the H update on the new E, read from the world's current set of arrays
-// (fields, CPML psi, dispersive currents) and written to its other set, so that no
-// workgroup overwrites a value another one still reads.  A workgroup sweeps a chunk of x
-// planes for R rows (each wave one row, all of its k cells, NC per lane): per plane it
-// updates E, passes the new values through LDS, then updates H from them, so each field
-// element comes from HBM once and goes back once per step (the separate half steps read
-// the other field a second time).  The E values H needs beyond the workgroup's cells -- row
-// j0 - 1 (wave 0) and plane i0 - 1 (the sweep's first iteration) -- are computed again and
-// not stored; outside the update range the arrays' values are read (cells no step writes).
-// The end-of-E-half program (strips, sources, ghosts) runs afterwards on the new set, and
-// k_fix recomputes H on the cells whose E inputs it changed.
-// Workgroups are dealt to the 8 XCDs by chunk: all row groups of a chunk run on one XCD,
-// side by side, so the rows one group reads of its neighbour's come from that XCD's L2.
-template<class T> struct StepArgs {
-	CurlArgs<T> e, h;           // the two halves (alt +1 and -1): F, G, psi and currents of
-	                            // the current set; O*, qa/qb and objOut of the other
-};
-
-// sa: the halves' arguments (device memory, read as needed rather than held in registers
-// across the sweep); R rows per group; wave (c, w) of the workgroup (threadIdx.y, .z) owns
-// the 64 cells from kMIN + 64 c of row j0 - 1 + w, so every wave has one cell per lane per
-// half step and plane, as in k_curl; P = 64 * ceil(nk / 64) + 1 values per LDS row and
-// component, whose slot 0 holds k = kMIN - 1.  LDS: two planes (this one and the one
-// before, alternating) of R + 1 rows of the three E components, so one barrier per plane
-// separates the E writes from the H reads.  The values a plane's E update streams from the
-// current set -- E and H at the cell, H one cell up along each axis -- are loaded into
-// registers a plane ahead (H at the cell two planes ahead: it is the next plane's i + 1
-// neighbour first), so their latency passes while the plane before is updated.
-template<class T, int CME>
-__global__ __launch_bounds__(1024, sizeof(T) == 4 ? 8 : 4) void k_step(const StepArgs<T> *__restrict__ sa, int R, int P, int chunk, int nchunk, int ngroup)
-{
-	extern __shared__ __align__(16) unsigned char stepLds[];
-	const int lane = (int)threadIdx.x, c = (int)threadIdx.y, w = (int)threadIdx.z;
-	const int b = (int)blockIdx.x, slot = b >> 3;
-	const int g = slot % ngroup, q = (b & 7) + 8 * (slot / ngroup);
-	if (q >= nchunk) return;
-	const int iMIN = sa->e.iMIN, jMIN = sa->e.jMIN, kMIN = sa->e.kMIN, nj = sa->e.nj, nk = sa->e.nk;
-	const int j = jMIN + g * R - 1 + w, k = kMIN + c * 64 + lane, x = 1 + c * 64 + lane;
-	const int ib = iMIN + q * chunk, ie = min(ib + chunk, iMIN + sa->e.ni) - 1;
-	const bool rowIn = j >= jMIN && j < jMIN + nj, live = j < jMIN + nj && k < kMIN + nk;
-	const int plane = (R + 1) * 3 * P;
-	const Lay L = sa->e.L;
-	const T *const E0 = sa->e.F0, *const E1 = sa->e.F1, *const E2 = sa->e.F2;
-	const T *const H0 = sa->e.G0, *const H1 = sa->e.G1, *const H2 = sa->e.G2;
-	// pipeline: e (E at plane i), h (H at i), u (H at i + 1), n (H x, z at j + 1 and x, y at
-	// k + 1, plane i), s (E at k = kMIN - 1, plane i; lane x == 1); the next plane's in p*
-	T e0 = 0, e1 = 0, e2 = 0, h0 = 0, h1 = 0, h2 = 0, u0 = 0, u1 = 0, u2 = 0;
-	T n0 = 0, n1 = 0, n2 = 0, n3 = 0, s0 = 0, s1 = 0, s2 = 0;
-	auto loadE = [&](int ii, T &a0, T &a1, T &a2) {
-		const long id = L.at(ii, j, k);
-		a0 = ldS<true>(E0 + id), a1 = ldS<true>(E1 + id), a2 = ldS<true>(E2 + id);
-	};
-	auto loadH = [&](int ii, T &a0, T &a1, T &a2) {
-		const long id = L.at(ii, j, k);
-		a0 = *glb(H0 + id), a1 = *glb(H1 + id), a2 = *glb(H2 + id);
-	};
-	auto loadN = [&](int ii, T &a0, T &a1, T &a2, T &a3) {
-		const long id = L.at(ii, j, k);
-		a0 = *glb(H0 + id + L.sj), a1 = *glb(H2 + id + L.sj), a2 = *glb(H0 + id + 1), a3 = *glb(H1 + id + 1);
-	};
-	auto loadS = [&](int ii, T &a0, T &a1, T &a2) {
-		const long id = L.at(ii, j, kMIN - 1);
-		a0 = *glb(E0 + id), a1 = *glb(E1 + id), a2 = *glb(E2 + id);
-	};
-	if (live) {
-		loadE(ib - 1, e0, e1, e2);
-		if (x == 1) loadS(ib - 1, s0, s1, s2);
-		if (rowIn) {
-			loadH(ib - 1, h0, h1, h2), loadH(ib, u0, u1, u2), loadN(ib - 1, n0, n1, n2, n3);
-		}
-	}
-	for (int i = ib - 1; i <= ie; i++) {
-		T pe0 = 0, pe1 = 0, pe2 = 0, pu0 = 0, pu1 = 0, pu2 = 0, pn0 = 0, pn1 = 0, pn2 = 0, pn3 = 0, ps0 = 0, ps1 = 0, ps2 = 0;
-		if (live && i < ie) {
-			loadE(i + 1, pe0, pe1, pe2);
-			if (x == 1) loadS(i + 1, ps0, ps1, ps2);
-			if (rowIn) {
-				loadN(i + 1, pn0, pn1, pn2, pn3);
-				if (i + 2 <= ie + 1) loadH(i + 2, pu0, pu1, pu2);
-			}
-		}
-		T *const mine = (T *)stepLds + (i & 1) * plane + w * 3 * P;
-		const bool own = w > 0 && rowIn && i >= ib;
-		if (live) {
-			T ex = e0, ey = e1, ez = e2;
-			if (rowIn && i >= iMIN) {
-				const T given0 = e0, given1 = e1, given2 = e2;
-				const T gx = h0, gy = h1, gz = h2;
-				const T g0j = n0, g2j = n1, g0k = n2, g1k = n3, g1i = u1, g2i = u2;
-				const CurlArgs<T> &a = sa->e;
-				const bool wr = own;
-				constexpr int CM = CME;
-				constexpr bool NT = true, NTG = false, SHARE = true, NTP = true, MERGEZ = false, UNI = true, SEP = true, NTC = true;
-				constexpr int KSH = 0;
-#define CURL_GIVEN
-#define CURL_GIVEN_F
-#include "curl_cell.inc"
-#undef CURL_GIVEN_F
-#undef CURL_GIVEN
-				ex = fx, ey = fy, ez = fz;
-			}
-			mine[x] = ex, mine[P + x] = ey, mine[2 * P + x] = ez;
-			if (x == 1) mine[0] = s0, mine[P] = s1, mine[2 * P] = s2;
-		}
-		__syncthreads();
-		if (own && live) {
-			const T *const below = mine - 3 * P;
-			const T *const before = (T *)stepLds + ((i + 1) & 1) * plane + w * 3 * P;   // plane i - 1
-			const T given0 = h0, given1 = h1, given2 = h2;
-			const T gx = mine[x], gy = mine[P + x], gz = mine[2 * P + x];
-			const T g0k = mine[x - 1], g1k = mine[P + x - 1];
-			const T g0j = below[x], g2j = below[2 * P + x];
-			const T g1i = before[P + x], g2i = before[2 * P + x];
-			const CurlArgs<T> &a = sa->h;
-			constexpr int CM = 0;
-			constexpr bool NT = true, NTG = false, SHARE = true, NTP = true, MERGEZ = false, UNI = true, SEP = true, wr = true, NTC = true;
-			constexpr int KSH = 0;
-#define CURL_GIVEN
-#define CURL_GIVEN_F
-#include "curl_cell.inc"
-#undef CURL_GIVEN_F
-#undef CURL_GIVEN
-		}
-		e0 = pe0, e1 = pe1, e2 = pe2, h0 = u0, h1 = u1, h2 = u2, u0 = pu0, u1 = pu1, u2 = pu2;
-		n0 = pn0, n1 = pn1, n2 = pn2, n3 = pn3, s0 = ps0, s1 = ps1, s2 = ps2;
-	}
 }
 
 // Cells copied from one set of a world's arrays to the other (see the carry lists of
@@ -496,34 +149,6 @@ __global__ __launch_bounds__(256) void k_carry(CarryArgs<T> a)
 	boxCell(t - a.off[q], B.i1 - B.i0 + 1, B.j1 - B.j0 + 1, B.k1 - B.k0 + 1, di, dj, dk);
 	const long id = a.L.at(B.i0 + di, B.j0 + dj, B.k0 + dk);
 	a.dst[q][id] = a.src[q][id];
-}
-
-// H again on the cells whose E inputs the end-of-E-half program changed after k_step (the
-// boxes of its operations, one cell further up each axis): from the old set's H, psi and
-// currents and the new set's final E, into the new set -- the values the separate half
-// steps give.  One thread per cell of a list of boxes.
-constexpr int MAXFIX = 16;
-struct FixBoxes {
-	Box b[MAXFIX];
-	long off[MAXFIX + 1];       // first thread of each box; off[n] = all
-	int n;
-};
-
-template<class T>
-__global__ __launch_bounds__(256) void k_fix(CurlArgs<T> a, FixBoxes f)
-{
-	const long t0 = (long)blockIdx.x * 256 + threadIdx.x;
-	if (t0 >= f.off[f.n]) return;
-	int q = 0;
-	while (q + 1 < f.n && f.off[q + 1] <= t0) q++;
-	const Box &B = f.b[q];
-	int di, dj, dk;
-	boxCell(t0 - f.off[q], B.i1 - B.i0 + 1, B.j1 - B.j0 + 1, B.k1 - B.k0 + 1, di, dj, dk);
-	const int i = B.i0 + di, j = B.j0 + dj, k = B.k0 + dk;
-	constexpr int CM = 0;
-	constexpr bool NT = false, NTG = false, SHARE = true, NTP = false, MERGEZ = false, UNI = false, SEP = true, wr = true, NTC = false;
-	constexpr int KSH = 0;
-#include "curl_cell.inc"
 }
 
 // The end of a half step in one launch: TF/SF strips and sources (additive operations,
@@ -559,10 +184,6 @@ template<class T> struct PostOp {
 constexpr int MAXSRC = 128;     // sources per chain (E or H) of one world
 constexpr int MAXCHAIN = 24;    // copies per launch
 constexpr int MAXPOST = 48;     // operations per launch
-constexpr int CURL_TPB = 2;     // tiles per workgroup of a batched curl launch (measured best of 1..16)
-constexpr int CURL_TPB_PAIR = 1;  // the same for entries of both parts of a Bloch world
-constexpr int CURL_TPB_TILE = TPB_TILE;  // the same for entries of 64 x 4 tiles (rows of 64 cells or more)
-
 constexpr int POST_WG = 64;     // threads (cells) per workgroup of k_post: one wavefront (64 k-point
                                 // worlds: H program 84 -> 79 us, E 35 -> 31 us against 256)
 
@@ -579,6 +200,8 @@ template<class T> struct PostArgs {
 	const PostOp<T> *ops;
 	const PostPiece *pieces;    // per workgroup of the launch: the piece it runs
 	long total;
+	int post;                   // workgroups of the program; those after them run `ade`
+	ObjArgs<T> ade;
 	unsigned strips;            // TF/SF boxes whose strips apply this half step (bit s)
 	unsigned src[MAXSRC / 32];  // sources active this half step
 	T wave[MAXSRC];             // their scalar wave values
@@ -592,18 +215,18 @@ template<class T> __device__ inline bool opOn(const PostArgs<T> &a, const PostOp
 }
 
 // F(i,j,k) + dt/ds G_aux (1/eps), or F + amplitude wave, as the reference evaluates them.
-template<class T> __device__ inline T addOne(const PostArgs<T> &a, const PostOp<T> &o, T f, int i, int j, int k)
+template<class T, class O> __device__ inline T addTo(O &o, T f, int i, int j, int k, T wave)
 {
 	if (o.kind == OP_STRIP) {
 		int ia = i + o.di, ja = j + o.dj;
 		if (o.exX && ia > o.auxIMAX) ia = o.auxIMAX + o.altX;
 		if (o.exY && ja > o.auxJMAX) ja = o.auxJMAX + o.altY;
-		const T g = o.A[o.LA.at(ia, ja, k + o.dk)];
-		return o.C ? f + o.c * g * o.C[o.LC.at(i, j, k)] : f + o.c * g;
+		const T g = glb(o.A)[layAt(o.LA, ia, ja, k + o.dk)];
+		return o.C ? f + o.c * g * glb(o.C)[layAt(o.LC, i, j, k)] : f + o.c * g;
 	}
-	const long c = o.LC.at(i, j, k);
-	const T amp = o.C ? o.C[c] : o.c;
-	const T w = o.W ? o.W[c] : a.wave[o.slot];
+	const long c = layAt(o.LC, i, j, k);
+	const T amp = o.C ? glb(o.C)[c] : o.c;
+	const T w = o.W ? glb(o.W)[c] : wave;
 	return f + amp * w;
 }
 
@@ -613,22 +236,23 @@ template<class T> __device__ inline T addOne(const PostArgs<T> &a, const PostOp<
 // dependent loads (piece, operation, cell) where a search of the pieces added about seven
 // (measured with 256-thread workgroups: 64 k-point worlds' H program 95 -> 84 us; 256^3
 // nanoblock H program 17.5 -> 16.1 us).
+// (tid: the thread's place in the workgroup.)
 template<class T>
-__device__ __forceinline__ void postBlock(const PostArgs<T> &a, int blk)
+__device__ __forceinline__ void postCells(const PostArgs<T> &a, const PostOp<T> *ops, const PostPiece *pieces, int blk, int tid)
 {
-	const PostPiece &P = a.pieces[blk];
+	const PostPiece &P = pieces[blk];
 	const int ni = P.b.i1 - P.b.i0 + 1, nj = P.b.j1 - P.b.j0 + 1, nk = P.b.k1 - P.b.k0 + 1;
-	const int t = blk * POST_WG + (int)threadIdx.x - (int)P.off;
+	const int t = blk * POST_WG + tid - (int)P.off;
 	if (t >= ni * nj * nk) return;
 	const int dk = t % nk, r = t / nk, dj = r % nj, di = r / nj;
 	const int i = P.b.i0 + di, j = P.b.j0 + dj, k = P.b.k0 + dk;
-	const PostOp<T> &o = a.ops[P.list[0]];
+	const PostOp<T> &o = ops[P.list[0]];
 	const long d = o.LF.at(i, j, k);
 	if (P.kind == OP_COPY) {
 		const long s = o.LF.at(i + P.si, j + P.sj, k + P.sk);
 		T f = o.F[s], g = o.G ? o.G[s] : T(0);
 		for (int u = P.n - 1; u >= 0; u--) {
-			const PostOp<T> &r = a.ops[P.list[u]];
+			const PostOp<T> &r = ops[P.list[u]];
 			if (o.G) {
 				const T fs = f, gs = g;
 				f = r.c * fs + r.s * gs;
@@ -643,12 +267,19 @@ __device__ __forceinline__ void postBlock(const PostArgs<T> &a, int blk)
 	bool on = false;
 	T f = T(0);
 	for (int u = 0; u < P.n; u++) {
-		const PostOp<T> &r = a.ops[P.list[u]];
+		const PostOp<T> &r = ops[P.list[u]];
 		if (!opOn(a, r)) continue;
 		if (!on) f = o.F[d], on = true;
-		f = addOne(a, r, f, i, j, k);
+		f = addTo(r, f, i, j, k, r.kind == OP_SOURCE ? a.wave[r.slot] : T(0));
 	}
 	if (on) o.F[d] = f;
+}
+
+template<class T>
+__device__ __forceinline__ void postBlock(const PostArgs<T> &a, int blk)
+{
+	if (blk < a.post) postCells(a, a.ops, a.pieces, blk, (int)threadIdx.x);
+	else if (a.ade.blocks) adeBlock(a.ade, blk - a.post);
 }
 
 template<class T>
@@ -665,6 +296,9 @@ __global__ __launch_bounds__(POST_WG) void k_post_batch(const PostArgs<T> *__res
 	const int e = batchEntry(start, n, b);
 	postBlock(args[e], b - start[e]);
 }
+
+#include "step_kernel.inc"
+#include "aux_curl.inc"
 
 // Phaser running DFT (src/phaser.c:83-110): one thread per face cell and block of PHS_QPT
 // frequencies (the frequency blocks multiply the threads, so even a small phaser box fills
@@ -1232,10 +866,10 @@ inline void launchEv(void (*k)(P...), dim3 grid, dim3 block, size_t lds, hipStre
 
 struct DevSlab {
 	bool on = false;
-	int lo = 0, hi = -1;
+	int lo = 0, hi = -1, first = 0;   // first: the face's place in the axis's shared array (SlabPair)
 	Lay L{};
 	Box b{};                    // host extents of the slab array
-	long n = 0;                 // elements of each array
+	long n = 0;                 // elements of each array (0: a max face sharing its min face's)
 	void *p[2][2] = {};         // [m][a/b]
 	void *alt[2][2] = {};       // the other set (k_step), allocated at the first fused step
 };
@@ -1244,12 +878,12 @@ struct DevObj {
 	Box box{};                  // object box (C->iMin[n]..C->iMax[n] ...)
 	Box clip{};                 // box clipped to the grid [MIN..MAX]
 	Lay LO{};
+	long n = 0;                 // elements of each array
 	int NJ = 0, NK = 0;
 	float a[3] = {};
 	float JJ[3][MAXPOLE] = {}, JK[3][MAXPOLE] = {}, JE[3][MAXPOLE] = {}, KJ[3][MAXPOLE] = {}, KK[3][MAXPOLE] = {}, KE[3][MAXPOLE] = {};
 	void *fill[3] = {};
 	void *J[2][3][MAXPOLE] = {}, *K[2][3][MAXPOLE] = {};
-	void *Jalt[2][3][MAXPOLE] = {}, *Kalt[2][3][MAXPOLE] = {};   // the other set (k_step)
 };
 
 struct DevSrc {
@@ -1329,7 +963,6 @@ struct alis_dev_world {
 	DevSlab slab[2][6];
 	std::vector<DevObj> obj;
 	void *objTab = nullptr;     // ObjDev<T>[obj.size()] in device memory
-	void *objTile = nullptr;    // int[]: per-tile object lists (see objectTiles) or null
 	std::vector<DevSrc> src[2];
 	std::vector<DevTfsf> tf;
 	// end-of-half-step programs (k_post launches), built at the first ghosts call after the
@@ -1356,26 +989,39 @@ struct alis_dev_world {
 	double evMs[3] = {0, 0, 0};
 	long evCount[3] = {0, 0, 0};
 	// Fused steps (k_step): the world holds a second set of the arrays a step updates and
-	// alternates between the sets; an E half step is deferred until its H half arrives.
-	int fuseState = 0;          // 0 not decided yet, 1 fused steps allowed, -1 not
+	// alternates between the sets; a step is deferred until its H half is complete.
+	int fuseState = 0;          // 0 not decided yet, 1 fused steps possible, -1 not
 	bool isAux = false;         // the TF/SF auxiliary world of another world
+	alis_dev_world *mainOf = nullptr;   // that world
 	int inBatch = 0;            // live batches whose launch arguments name this world's arrays
-	int pendE = 0;              // 1: E curl deferred; 2: and its end-of-half-step program
+	int pendE = 0;              // 1: E core deferred; 2: and its ghosts; 3: and the H core
+	// A small auxiliary world's half step in the main world's launches (k_curl_aux): main world:
+	// 1 + h while its core of half step h waits for its ghosts; auxiliary world: its core and its
+	// ghosts of half step h wait for them too.
+	int pendMain = 0, pendCore = 0, pendGhosts = 0;
+	int foldState = 0;          // main world: 0 not decided yet, 1 its auxiliary world can, -1 cannot
+	int pendH = 0;              // auxiliary world: its H core (1) and ghosts (2) wait for the
+	                            //  main world's deferred step, which reads the old H
 	bool altReady = false;      // the other set exists
 	bool altStale = false;      // cells no step writes may differ between the sets
 	int par = 0;                // which set is current (0: the one allocated at commit)
 	void *Falt[2][2][3] = {};
-	void *objTabAlt = nullptr;  // the object table naming the other set's currents
 	std::vector<PostSeg> postAlt[2];  // end-of-half-step programs of the other set
-	bool postBuiltAlt = false;
-	void *stepArgs = nullptr;   // StepArgs<T>[2 sets][2 parts]: k_step's arguments per current set
+	std::vector<PostSeg> copies, copiesAlt;  // both halves' ghost copies alone, per set (fused steps)
+	bool copiesBuilt = false, copiesBuiltAlt = false, postBuiltAlt = false;
+	void *stepArgs = nullptr;   // StepArgs<T>[2 parts][2 sets]: k_step's arguments per current set
+	void *objStart = nullptr, *objOver = nullptr;   // tables of the objects' launches (ObjArgs)
+	int objWgs = 0;             // workgroups of one component of one part
+	bool pendAde = false;       // the current update of the last H core is still to run
+	struct AddRef { int kind, slot; };
+	std::vector<AddRef> adds[2][2];   // [part][half]: the additive operations of k_step's lists
+	void *addTab[2][2] = {}, *addAt[2][2] = {};   // their tables on the device (StepAdd<T>, bits per plane)
 	struct Carry { int axis; Box b; };
-	std::vector<Carry> carry[2];  // cells a fused step's end-of-half programs take from the other set
-	bool carryDue[2] = {false, false};
+	std::vector<Carry> carry[2];  // cells a fused step's ghost copies take from the other set
 	std::vector<Box> hWrites;   // the boxes the end-of-H-half program writes
-	std::vector<Box> fix;       // boxes k_fix recomputes after the E program
-	bool fixOk = false;         // every additive operation lies in the update range and the
-	                            //  boxes fit one k_fix launch
+	std::vector<Box> hCopies;   // those of its ghost copies
+	bool addsInside = false;    // every additive operation lies in the update range and their
+	                            //  lists fit k_step's
 };
 
 namespace {
@@ -1394,7 +1040,7 @@ int devAlloc(alis_dev_world *D, void **p, size_t bytes)
 template<class T>
 int upload1(alis_dev_world *D, void **dst, const float *src, int n)
 {
-	if (devAlloc(D, dst, n * sizeof(T))) return -1;
+	if (devAlloc(D, dst, (n + 16 / sizeof(T)) * sizeof(T))) return -1;   // k_step reads whole quads
 	std::vector<T> tmp(n);
 	for (int a = 0; a < n; a++) tmp[a] = (T)src[a];
 	HIPCHECK(hipMemcpyAsync(*dst, tmp.data(), n * sizeof(T), hipMemcpyHostToDevice, D->st));
@@ -1460,29 +1106,30 @@ int downloadSubBox(alis_dev_world *D, const void *src, const Lay &L, const Box &
 	return 0;
 }
 
-// Field arrays: rows along k.  Rows are padded and shifted so that k = kMIN starts on a
-// 128-byte boundary, except rows (ghosts included) no longer than a wavefront: those are
-// packed end to end, where the padding and the ghost cell would cost a partly used sector
-// per row and array, and the batched curl runs them in flat tiles across row ends, its
-// planes padded to 256 bytes so that the tiles, which start at plane origins, keep every
-// wavefront's access aligned (64 k-point worlds: E curl 17 % faster than unpadded planes
-// tiled from the first active row).  (Longer rows lose when packed: 64-194-cell rows of the
-// serving worlds ran 14 % slower.)
+// Field arrays: rows along k, end to end.  A row is kNUM + 2 values rounded up to quads
+// (16 bytes): k = kMIN starts on a quad, and the ghost below it is the last value of the row
+// before.  k_step's wavefronts run across row ends, so short rows fill them as well as long
+// ones; planes are padded to 256 bytes, and one such line lies before the first row (its lower
+// ghost) and after the last.
 Lay fieldLayout(const alis_dev_world *D)
 {
-	const int align = ROW_ALIGN_BYTES / (int)D->esz;
-	int koff = align;
-	const int nkTot = koff + D->kNUM + 1;                      // offsets 0..koff+kNUM used
-	long SK = ((nkTot + align - 1) / align) * align;
-	if (D->kNUM + 2 <= 64) koff = 1, SK = D->kNUM + 2;
+	const long quad = 16 / (long)D->esz, line = 256 / (long)D->esz;
 	Lay L;
-	L.i0 = D->iMIN - 1, L.j0 = D->jMIN - 1, L.k0 = D->kMIN, L.koff = koff;
-	L.sj = SK;
-	L.si = (long)(D->jNUM + 2) * SK;
-	if (koff == 1) {
-		const long plane = 256 / (long)D->esz;
-		L.si = (L.si + plane - 1) / plane * plane;
-	}
+	L.i0 = D->iMIN - 1, L.j0 = D->jMIN - 1, L.k0 = D->kMIN, L.koff = (int)line;
+	L.sj = (D->kNUM + 2 + quad - 1) / quad * quad;
+	L.si = ((long)(D->jNUM + 2) * L.sj + line - 1) / line * line;
+	return L;
+}
+
+// A compact layout over box b whose rows start and end on quads of the world's rows, so that a
+// quad of the grid is one quad here.
+Lay quadLayout(const alis_dev_world *D, const Box &b)
+{
+	const int quad = 16 / (int)D->esz, k0 = D->kMIN + (b.k0 - D->kMIN) / quad * quad;
+	Lay L;
+	L.i0 = b.i0, L.j0 = b.j0, L.k0 = k0, L.koff = 0;
+	L.sj = (b.k1 - k0 + quad) / quad * quad;
+	L.si = (long)(b.j1 - b.j0 + 1) * L.sj;
 	return L;
 }
 
@@ -1730,44 +1377,10 @@ int rowSegments(alis_dev_world *D)
 	return 0;
 }
 
-// Per-tile object lists for worlds with more dispersive objects than OBJ_SCAN: for every
-// 64 x 4 tile of the curl (an x plane, 4 rows, 64 cells along k) the objects whose clipped
-// box meets it, in ascending order, so that a cell visits only those (and adds their
-// currents in the same order as a scan of all objects would).  Layout: ntile + 1 starts,
-// then the lists.
-constexpr int OBJ_SCAN = 2;
-
-int objectTiles(alis_dev_world *D)
-{
-	if ((int)D->obj.size() <= OBJ_SCAN) return 0;
-	const int njb = (D->jNUM + 3) / 4, nkb = (D->kNUM + 63) / 64;
-	const long ntile = (long)D->iNUM * njb * nkb;
-	std::vector<int> start(ntile + 1, 0);
-	auto each = [&](const Box &b, auto &&f) {
-		if (b.i1 < b.i0 || b.j1 < b.j0 || b.k1 < b.k0) return;
-		for (int i = b.i0; i <= b.i1; i++)
-			for (int jb = (b.j0 - D->jMIN) / 4; jb <= (b.j1 - D->jMIN) / 4; jb++)
-				for (int kb = (b.k0 - D->kMIN) / 64; kb <= (b.k1 - D->kMIN) / 64; kb++)
-					f(((long)(i - D->iMIN) * njb + jb) * nkb + kb);
-	};
-	for (const DevObj &O : D->obj) each(O.clip, [&](long t) { start[t + 1]++; });
-	for (long t = 0; t < ntile; t++) start[t + 1] += start[t];
-	std::vector<int> table(start.begin(), start.end());
-	table.resize(ntile + 1 + start[ntile]);
-	std::vector<int> fill(start.begin(), start.end() - 1);
-	for (int n = 0; n < (int)D->obj.size(); n++)
-		each(D->obj[n].clip, [&](long t) { table[ntile + 1 + fill[t]++] = n; });
-	if (devAlloc(D, &D->objTile, table.size() * sizeof(int))) return -1;
-	HIPCHECK(hipMemcpyAsync(D->objTile, table.data(), table.size() * sizeof(int), hipMemcpyHostToDevice, D->st));
-	HIPCHECK(hipStreamSynchronize(D->st));
-	return 0;
-}
-
 // Commit: allocate and upload everything of the descriptor.
-// The device table of D's dispersive objects (ObjDev<T>), naming the currents of its
-// commit-time set (alt false) or of its other set (alt true, see k_step).
+// The device table of D's dispersive objects (ObjDev<T>).
 template<class T>
-int uploadObjTable(alis_dev_world *D, bool alt, void **dst)
+int uploadObjTable(alis_dev_world *D, void **dst)
 {
 	std::vector<ObjDev<T>> tab(D->obj.size());
 	for (size_t n = 0; n < D->obj.size(); n++) {
@@ -1785,8 +1398,8 @@ int uploadObjTable(alis_dev_world *D, bool alt, void **dst)
 				t.JJ[c][p] = (T)O.JJ[c][p], t.JK[c][p] = (T)O.JK[c][p], t.JE[c][p] = (T)O.JE[c][p];
 				t.KJ[c][p] = (T)O.KJ[c][p], t.KK[c][p] = (T)O.KK[c][p], t.KE[c][p] = (T)O.KE[c][p];
 				for (int m = 0; m <= D->cplx; m++) {
-					t.J[m][c][p] = (T *)(alt ? O.Jalt : O.J)[m][c][p];
-					t.K[m][c][p] = (T *)(alt ? O.Kalt : O.K)[m][c][p];
+					t.J[m][c][p] = (T *)O.J[m][c][p];
+					t.K[m][c][p] = (T *)O.K[m][c][p];
 				}
 			}
 		}
@@ -1802,7 +1415,7 @@ int commitWorld(alis_dev_world *D)
 {
 	const alis_dev_world_desc *W = &D->W;
 	D->L = fieldLayout(D);
-	D->fsize = (long)(D->iNUM + 2) * D->L.si;
+	D->fsize = (long)(D->iNUM + 2) * D->L.si + 2 * D->L.koff;
 	const Box fb = fieldBox(D);
 
 	for (int h = 0; h < 2; h++)
@@ -1857,21 +1470,41 @@ int commitWorld(alis_dev_world *D)
 			if (ax == 1) b.j0 = S.lo, b.j1 = S.hi;
 			if (ax == 2) b.k0 = S.lo, b.k1 = S.hi;
 			S.b = b;
-			if (ax == 2) S.L = compactLayout(b);
-			else {
-				S.L = D->L;
-				S.L.i0 = b.i0, S.L.j0 = b.j0;
-				S.L.si = (long)(b.j1 - b.j0 + 1) * D->L.sj;
+		}
+		// the min and max face of an axis in one array, the max face's cells after the min
+		// face's along the axis (see SlabPair); along z whole quads, one of them shared where
+		// both faces lie in it
+		for (int ax = 0; ax < 3; ax++) {
+			DevSlab *pair[2] = {&D->slab[h][ax], &D->slab[h][ax + 3]};
+			const int quad = 16 / (int)sizeof(T);
+			long cells[2] = {0, 0};     // their extents along the axis; z: in elements of whole quads
+			for (int s = 0; s < 2; s++) {
+				if (!pair[s]->on) continue;
+				pair[s]->L = ax == 2 ? quadLayout(D, pair[s]->b) : D->L;
+				cells[s] = ax == 2 ? pair[s]->L.sj : pair[s]->hi - pair[s]->lo + 1;
 			}
-			const long n = (long)(b.i1 - b.i0 + 1) * S.L.si;
-			S.n = n;
-			for (int m = 0; m <= D->cplx; m++)
-				for (int s2 = 0; s2 < 2; s2++) {
-					float ***hostp = W->slab[h][m][f][s2];
-					if (!hostp) return fail("CPML slab missing on the host");
-					if (devAlloc(D, &S.p[m][s2], n * sizeof(T))) return -1;
-					if (uploadBox<T>(D, S.p[m][s2], S.L, b, hostBlock(hostp, b))) return -1;
-				}
+			const bool share = ax == 2 && pair[0]->on && pair[1]->on && (pair[0]->hi - D->kMIN) / quad == (pair[1]->lo - D->kMIN) / quad;
+			if (share) cells[0] -= quad;
+			const long sj = ax == 2 ? cells[0] + cells[1] : D->L.sj;
+			const long rows = ax == 1 ? cells[0] + cells[1] : D->jNUM, si = rows * sj, n = (ax == 0 ? cells[0] + cells[1] : D->iNUM) * si;
+			void *shared[2][2] = {};
+			for (int s = 0; s < 2; s++) {
+				DevSlab &S = *pair[s];
+				if (!S.on) continue;
+				const long before = s ? cells[0] : 0;
+				S.L.i0 = S.b.i0, S.L.j0 = S.b.j0, S.L.sj = sj, S.L.si = si;
+				S.L.koff = (int)(before * (ax == 0 ? si : ax == 1 ? sj : 1));
+				S.first = (int)(ax == 2 ? before / quad : before);
+				S.n = shared[0][0] ? 0 : n;
+				for (int m = 0; m <= D->cplx; m++)
+					for (int s2 = 0; s2 < 2; s2++) {
+						float ***hostp = W->slab[h][m][ax + 3 * s][s2];
+						if (!hostp) return fail("CPML slab missing on the host");
+						if (!shared[m][s2] && devAlloc(D, &shared[m][s2], n * sizeof(T))) return -1;
+						S.p[m][s2] = shared[m][s2];
+						if (uploadBox<T>(D, S.p[m][s2], S.L, S.b, hostBlock(hostp, S.b))) return -1;
+					}
+			}
 		}
 	}
 
@@ -1883,7 +1516,7 @@ int commitWorld(alis_dev_world *D)
 		O.clip = Box{std::max(D->iMIN, A.i0), std::min(D->iMAX, A.i1),
 		             std::max(D->jMIN, A.j0), std::min(D->jMAX, A.j1),
 		             std::max(D->kMIN, A.k0), std::min(D->kMAX, A.k1)};
-		O.LO = compactLayout(O.box);
+		O.LO = quadLayout(D, O.box);
 		O.NJ = A.nj, O.NK = A.nk;
 		if (O.NK > MAXPOLE || O.NJ > O.NK) return fail("bad pole counts");
 		for (int c = 0; c < 3; c++) {
@@ -1893,7 +1526,7 @@ int commitWorld(alis_dev_world *D)
 				if (p >= O.NJ) O.JK[c][p] = A.JK[c][p], O.KJ[c][p] = A.KJ[c][p], O.KK[c][p] = A.KK[c][p], O.KE[c][p] = A.KE[c][p];
 			}
 		}
-		const long n3 = O.box.count();
+		const long n3 = O.n = (long)(O.box.i1 - O.box.i0 + 1) * O.LO.si;
 		for (int c = 0; c < 3; c++) {
 			if (devAlloc(D, &O.fill[c], n3 * sizeof(T))) return -1;
 			if (uploadBox<T>(D, O.fill[c], O.LO, O.box, hostBlock(A.fill[c], O.box))) return -1;
@@ -1911,8 +1544,20 @@ int commitWorld(alis_dev_world *D)
 		D->obj.push_back(O);
 	}
 	if (!D->obj.empty()) {
-		if (uploadObjTable<T>(D, false, &D->objTab)) return -1;
-		if (objectTiles(D)) return -1;
+		std::vector<int> start, over(2 * D->obj.size() + 1);
+		for (const DevObj &O : D->obj) start.push_back(D->objWgs), D->objWgs += (int)blocksFor(O.n / Quads<T>::N, OBJ_WG);
+		for (size_t n = 0; n < D->obj.size(); n++)
+			for (size_t q = 0; q <= D->obj.size(); q++) {
+				if (q == 0) over[2 * n] = (int)over.size();
+				if (q == n) over[2 * n + 1] = (int)over.size();
+				if (q < D->obj.size() && q != n && boxesMeet(D->obj[q].clip, D->obj[n].clip)) over.push_back((int)q);
+			}
+		over[2 * D->obj.size()] = (int)over.size();
+		if (devAlloc(D, &D->objStart, start.size() * sizeof(int)) || devAlloc(D, &D->objOver, over.size() * sizeof(int))) return -1;
+		HIPCHECK(hipMemcpyAsync(D->objStart, start.data(), start.size() * sizeof(int), hipMemcpyHostToDevice, D->st));
+		HIPCHECK(hipMemcpyAsync(D->objOver, over.data(), over.size() * sizeof(int), hipMemcpyHostToDevice, D->st));
+		HIPCHECK(hipStreamSynchronize(D->st));
+		if (uploadObjTable<T>(D, &D->objTab)) return -1;
 	}
 
 	// sources
@@ -1952,38 +1597,67 @@ int commitWorld(alis_dev_world *D)
 }
 
 template<class T>
-CurlArgs<T> curlArgs(alis_dev_world *D, int h, int m)
+HalfArgs<T> halfArgs(alis_dev_world *D, int h, int m)
 {
-	CurlArgs<T> a{};
-	a.F0 = (T *)D->F[h][m][0], a.F1 = (T *)D->F[h][m][1], a.F2 = (T *)D->F[h][m][2];
-	a.O0 = a.F0, a.O1 = a.F1, a.O2 = a.F2;
-	a.G0 = (const T *)D->F[1-h][m][0], a.G1 = (const T *)D->F[1-h][m][1], a.G2 = (const T *)D->F[1-h][m][2];
-	if (h == 0) a.C0 = (const T *)D->C[0], a.C1 = (const T *)D->C[1], a.C2 = (const T *)D->C[2];
+	constexpr int N = Quads<T>::N;
+	HalfArgs<T> a{};
+	for (int c = 0; c < 3; c++) {
+		a.F[c] = (T *)D->F[h][m][c], a.G[c] = (const T *)D->F[1-h][m][c];
+		if (h == 0) a.C[c] = (const T *)D->C[c];
+	}
 	if (h == 0) a.seg = (const typename Quad<T>::V *)D->seg;
 	a.dtx = (const T *)D->dt[h][0], a.dty = (const T *)D->dt[h][1], a.dtz = (const T *)D->dt[h][2];
 	a.L = D->L;
 	a.iMIN = D->iMIN, a.jMIN = D->jMIN, a.kMIN = D->kMIN;
 	a.ni = D->iNUM, a.nj = D->jNUM, a.nk = D->kNUM;
-	a.alt = h ? -1 : 1;
-	for (int f = 0; f < 6; f++) {
-		const DevSlab &S = D->slab[h][f];
-		CurlFace<T> &P = a.face[f];
-		P.on = S.on;
-		if (!S.on) continue;
-		const int ax = f % 3;
-		P.pa = (T *)S.p[m][0], P.pb = (T *)S.p[m][1];
-		P.qa = P.pa, P.qb = P.pb;
-		P.bc = (const T *)D->cpk[h][ax];
-		P.L = S.L, P.lo = S.lo, P.hi = S.hi;
+	a.pq = (int)(D->L.sj / N);
+	a.tiles = (a.nj * a.pq + CURL_WG - 1) / CURL_WG;
+	a.inv = a.pq == 1 ? 0xffffffffu : (unsigned)(((1ull << 32) + a.pq - 1) / a.pq);
+	for (int ax = 0; ax < 3; ax++) {
+		SlabPair<T> &P = a.slab[ax];
+		for (int side = 0; side < 2; side++) {
+			const DevSlab &S = D->slab[h][ax + 3 * side];
+			P.lo[side] = INT_MAX, P.hi[side] = INT_MIN;
+			if (!S.on) continue;
+			P.lo[side] = S.lo, P.hi[side] = S.hi, P.first[side] = S.first;
+			P.q0[side] = (S.lo - D->kMIN) / N;
+			P.pa = (T *)S.p[m][0], P.pb = (T *)S.p[m][1];
+			P.si = S.L.si, P.sj = S.L.sj;
+			P.bc = (const T *)D->cpk[h][ax];
+			P.b = (const T *)D->cp[h][ax][0], P.ca = (const T *)D->cp[h][ax][1], P.cb = (const T *)D->cp[h][ax][2];
+		}
 	}
-	a.obj = a.objOut = (const ObjDev<T> *)D->objTab;
-	a.nobj = (int)D->obj.size();
-	if (D->objTile) {
-		const long ntile = (long)D->iNUM * ((D->jNUM + 3) / 4) * ((D->kNUM + 63) / 64);
-		a.otStart = (const int *)D->objTile, a.otList = (const int *)D->objTile + ntile + 1;
-	}
-	a.m = m;
 	return a;
+}
+
+// D's objects in launches of their own (objects.inc), and the workgroups these take.
+template<class T>
+ObjArgs<T> objArgs(const alis_dev_world *D)
+{
+	ObjArgs<T> A{};
+	A.obj = (const ObjDev<T> *)D->objTab, A.start = (const int *)D->objStart, A.over = (const int *)D->objOver;
+	A.nobj = (int)D->obj.size(), A.blocks = D->objWgs;
+	A.L = D->L;
+	for (int m = 0; m <= D->cplx; m++)
+		for (int c = 0; c < 3; c++) A.E[m][c] = (T *)D->F[0][m][c];
+	return A;
+}
+
+int objBlocks(const alis_dev_world *D) { return D->objWgs * 3 * (1 + D->cplx); }
+
+// Make D use the stream of `to` (reference counted; the last user destroys a stream).
+int joinStream(alis_dev_world *D, alis_dev_world *to)
+{
+	if (D->st == to->st) return 0;
+	HIPCHECK(hipStreamSynchronize(D->st));
+	if (--*D->streamRefs == 0) {
+		HIPCHECK(hipStreamDestroy(D->st));
+		delete D->streamRefs;
+	}
+	D->st = to->st;
+	D->streamRefs = to->streamRefs;
+	++*to->streamRefs;
+	return 0;
 }
 
 // A pair of timing events of D: reused ones where alis_dev_timing_read has read them.
@@ -2003,13 +1677,15 @@ void dropPresamples(alis_dev_world *D)
 }
 
 // The z faces of D's phasers that the H curl can sample (PhsZ): a face whose k + 1 lies in
-// the same wavefront as k (k_curl's waves cover 64 cells from kMIN on), over the rectangle of
+// the same quad as k, over the rectangle of
 // its cells that the end-of-H-half program leaves alone at k and k + 1 (shrunk from the edges
 // its boxes reach: the ghost planes of periodic boundaries), so the values the curl has are
 // the ones the phaser update would read; k_phs_sample samples the other cells.
+// fused: by k_step, which applies the strips and sources itself, so only the ghost copies count.
 template<class T>
-int zSamples(alis_dev_world *D, PhsZ<T> *zs, std::vector<DevPhaser *> &owners)
+int zSamples(alis_dev_world *D, PhsZ<T> *zs, std::vector<DevPhaser *> &owners, bool fused)
 {
+	const int reach = Quads<T>::N;
 	int n = 0;
 	if (!D->postBuilt) return 0;
 	for (DevPhaser &P : D->phs) {
@@ -2020,9 +1696,9 @@ int zSamples(alis_dev_world *D, PhsZ<T> *zs, std::vector<DevPhaser *> &owners)
 			const PhsFaceGeom &g = P.face[f];
 			if (g.kind < 4) continue;
 			const int k = g.fixed;
-			if ((k - D->kMIN) % 64 == 63 || k + 1 > D->kMAX || n == MAXZS) { ok = false; break; }
+			if ((k - D->kMIN) % reach == reach - 1 || k + 1 > D->kMAX || n == MAXZS) { ok = false; break; }
 			int i0 = P.iMin, i1 = P.iMax, j0 = P.jMin, j1 = P.jMax;
-			for (const Box &b : D->hWrites) {
+			for (const Box &b : fused ? D->hCopies : D->hWrites) {
 				if (b.k1 < k || b.k0 > k + 1 || b.i1 < i0 || b.i0 > i1 || b.j1 < j0 || b.j0 > j1) continue;
 				if (b.i1 - b.i0 < b.j1 - b.j0 && b.i1 < (i0 + i1) / 2) i0 = b.i1 + 1;          // a plane at low i
 				else if (b.i1 - b.i0 < b.j1 - b.j0 && b.i0 > (i0 + i1) / 2) i1 = b.i0 - 1;
@@ -2063,32 +1739,36 @@ int zSamples(alis_dev_world *D, PhsZ<T> *zs, std::vector<DevPhaser *> &owners)
 	return n;
 }
 
+// x: an auxiliary world's share of the launch, or null.
 template<class T>
-int coreHalf(alis_dev_world *D, int h)
+int coreHalf(alis_dev_world *D, int h, const AuxCurl<T> *x = nullptr)
 {
 	dropPresamples(D);
 	hipEvent_t e0 = nullptr, e1 = nullptr;
 	if (D->timing) {
 		if (timingEvents(D, e0, e1)) return -1;
 	}
-	// E: grid (k tiles, y tiles, x planes); H: rows dealt to XCDs (k_curl's ROWS), rows
-	// padded to a multiple of 8
-	const long rows = (long)((D->jNUM + 3) / 4) * D->iNUM;
-	const dim3 grid = h == 0 ? dim3((D->kNUM + 63) / 64, (D->jNUM + 3) / 4, D->iNUM)
-	                         : dim3((unsigned)((rows + 7) / 8 * 8 * ((D->kNUM + 63) / 64))), block(64, 4);
 	// timing events are bound to the launches themselves (their start and end), so timing
 	// adds no marker between launches
 	std::vector<DevPhaser *> sampled;
 	for (int m = 0; m <= D->cplx; m++) {
-		CurlArgs<T> a = curlArgs<T>(D, h, m);
-		if (h == 1 && m == 0) a.nzs = zSamples<T>(D, a.zs, sampled);   // phasers sample part 0
+		HalfArgs<T> a = halfArgs<T>(D, h, m);
+		ZFaces<T> z{};
+		const bool aux = x && m == 0;
+		const dim3 grid(a.tiles, a.ni + (aux ? 1 : 0)), block(CURL_WG);
+		if (h == 0 && m == 0 && D->objWgs) k_currents<T><<<objBlocks(D), OBJ_WG, 0, D->st>>>(objArgs<T>(D));
+		if (h == 1 && m == 0) z.n = zSamples<T>(D, z.z, sampled, false);   // phasers sample part 0
 		hipEvent_t s0 = m == 0 ? e0 : nullptr, s1 = m == D->cplx ? e1 : nullptr;
-		if (h == 0 && D->seg) launchEv(k_curl<T, 2, false>, grid, block, 0, D->st, s0, s1, a);
-		else if (h == 0 && D->C[0]) launchEv(k_curl<T, 1, false>, grid, block, 0, D->st, s0, s1, a);
-		else if (h == 0) launchEv(k_curl<T, 0, false>, grid, block, 0, D->st, s0, s1, a);
-		else if (a.nzs) launchEv(k_curl<T, 0, true, true, false, 4, true>, grid, block, 0, D->st, s0, s1, a);
-		else launchEv(k_curl<T, 0, true>, grid, block, 0, D->st, s0, s1, a);
+#define CURL(H, C) (aux ? launchEv(k_curl_aux<T, H, C, false>, grid, block, 0, D->st, s0, s1, a, *x, z) : launchEv(k_curl<T, H, C>, grid, block, 0, D->st, s0, s1, a))
+		if (h == 0 && D->seg) CURL(0, 2);
+		else if (h == 0 && D->C[0]) CURL(0, 1);
+		else if (h == 0) CURL(0, 0);
+		else if (z.n && aux) launchEv(k_curl_aux<T, 1, 0, true>, grid, block, 0, D->st, s0, s1, a, *x, z);
+		else if (z.n) launchEv(k_curl_zs<T>, grid, block, 0, D->st, s0, s1, a, z);
+		else CURL(1, 0);
+#undef CURL
 	}
+	if (h == 1 && D->objWgs) D->pendAde = true;   // with the end of the half step (or flushStep)
 	if (e1) {
 		D->evPairs[h].push_back(e0);
 		D->evPairs[h].push_back(e1);
@@ -2217,61 +1897,82 @@ std::vector<Box> outsideParts(Box b, const Box &r)
 	return out;
 }
 
-// The H cells a fused step computes again after the E program (k_fix): H at a cell reads E
-// there and one cell below along each axis, so each box the program writes, grown by one
-// cell upwards and clipped to the update range.  Boxes that overlap much (the two strips of
-// one TF/SF face) are merged, and then the pairs whose union adds the fewest cells until at
-// most MAXFIX remain; computing H again on a cell the program did not reach reproduces the
-// value k_step wrote.
-std::vector<Box> fixBoxes(const std::vector<Box> &ops, const Box &range)
+// Upload one launch's program (nadd additive operations, then copies) compiled into pieces.
+template<class T>
+int postSegment(alis_dev_world *D, const std::vector<PostOp<T>> &v, int nadd, std::vector<PostPiece> &pieces, PostSeg &seg)
 {
-	std::vector<Box> v;
-	for (Box b : ops) {
-		b = Box{std::max(b.i0, range.i0), std::min(b.i1 + 1, range.i1), std::max(b.j0, range.j0), std::min(b.j1 + 1, range.j1),
-		        std::max(b.k0, range.k0), std::min(b.k1 + 1, range.k1)};
-		if (b.count()) v.push_back(b);
+	pieces.clear();
+	buildPieces(v, nadd, pieces, seg.total);
+	if (pieces.empty()) return 0;
+	if (seg.total >= (1L << 31)) return fail("end-of-half-step launch over 2^31 threads");
+	std::vector<PostPiece> perBlock(seg.total / POST_WG);
+	for (const PostPiece &P : pieces)
+		for (long b = P.off / POST_WG; b < (P.off + P.b.count() + POST_WG - 1) / POST_WG; b++) perBlock[b] = P;
+	if (devAlloc(D, &seg.ops, v.size() * sizeof(PostOp<T>))) return -1;
+	if (devAlloc(D, &seg.pieces, perBlock.size() * sizeof(PostPiece))) return -1;
+	HIPCHECK(hipMemcpyAsync(seg.ops, v.data(), v.size() * sizeof(PostOp<T>), hipMemcpyHostToDevice, D->st));
+	HIPCHECK(hipMemcpyAsync(seg.pieces, perBlock.data(), perBlock.size() * sizeof(PostPiece), hipMemcpyHostToDevice, D->st));
+	HIPCHECK(hipStreamSynchronize(D->st));   // the host vectors end with the caller
+	return 0;
+}
+
+// Group copies, in order, into launches that read no cell they write.
+template<class T>
+std::vector<std::vector<PostOp<T>>> copyGroups(const std::vector<PostOp<T>> &copies)
+{
+	std::vector<std::vector<PostOp<T>>> out;
+	std::vector<PostOp<T>> group;
+	const std::vector<PostOp<T>> none;
+	for (const PostOp<T> &o : copies) {
+		std::vector<PostOp<T>> trial = group;
+		trial.push_back(o);
+		if (!group.empty() && (trial.size() > (size_t)MAXCHAIN || postConflict(none, trial))) {
+			out.push_back(group);
+			group.assign(1, o);
+		}
+		else group.swap(trial);
 	}
-	auto unite = [](const Box &a, const Box &b) {
-		return Box{std::min(a.i0, b.i0), std::max(a.i1, b.i1), std::min(a.j0, b.j0), std::max(a.j1, b.j1),
-		           std::min(a.k0, b.k0), std::max(a.k1, b.k1)};
-	};
-	for (bool merged = true; merged;) {
-		merged = false;
-		for (size_t x = 0; x < v.size() && !merged; x++)
-			for (size_t y = x + 1; y < v.size() && !merged; y++)
-				if (unite(v[x], v[y]).count() * 10 <= (v[x].count() + v[y].count()) * 11) {
-					v[x] = unite(v[x], v[y]);
-					v.erase(v.begin() + y);
-					merged = true;
-				}
+	if (!group.empty()) out.push_back(group);
+	return out;
+}
+
+template<class T>
+void dropEmpty(std::vector<PostOp<T>> &v)
+{
+	v.erase(std::remove_if(v.begin(), v.end(), [](const PostOp<T> &o) { return o.b.count() == 0; }), v.end());
+}
+
+// The ghost copies of half step h, in call order.
+template<class T>
+std::vector<PostOp<T>> copyOps(const alis_dev_world *D, int h)
+{
+	std::vector<PostOp<T>> copies;
+	for (const CopySpec &c : ghostSchedule(&D->W, h)) {
+		PostOp<T> o{};
+		o.kind = OP_COPY;
+		o.F = (T *)D->F[h][0][c.axis];
+		o.G = D->cplx ? (T *)D->F[h][1][c.axis] : nullptr;
+		o.LF = D->L;
+		o.b = c.b;
+		o.di = c.di, o.dj = c.dj, o.dk = c.dk;
+		o.c = (T)c.c, o.s = (T)c.s;
+		copies.push_back(o);
 	}
-	while (v.size() > (size_t)MAXFIX) {
-		size_t bx = 0, by = 1;
-		long best = -1;
-		for (size_t x = 0; x < v.size(); x++)
-			for (size_t y = x + 1; y < v.size(); y++) {
-				const long grow = unite(v[x], v[y]).count() - v[x].count() - v[y].count();
-				if (best < 0 || grow < best) best = grow, bx = x, by = y;
-			}
-		v[bx] = unite(v[bx], v[by]);
-		v.erase(v.begin() + by);
-	}
-	return v;
+	dropEmpty(copies);
+	return copies;
 }
 
 // Build the end-of-half-step programs of D: strips of every TF/SF box, sources of the
 // chain, ghost copies; split into launches where a copy chain would read a cell that its
-// launch writes.
+// launch writes.  For fused steps, whose pass applies the strips and sources itself: the additive
+// operations' tables.
 template<class T>
 int buildPost(alis_dev_world *D)
 {
 	if ((int)D->tf.size() > 32) return fail("more than 32 TF/SF boxes in one world");
-	std::vector<std::vector<PostOp<T>>> segOps[2];
-	std::vector<int> segAdd[2];
 	const Box range{D->iMIN, D->iMAX, D->jMIN, D->jMAX, D->kMIN, D->kMAX};
-	std::vector<Box> eOps;      // the cells the E program writes
-	std::vector<PostOp<T>> copyOps[2];
-	D->fixOk = true;
+	D->addsInside = true;
+	D->copiesBuilt = false;
 	for (int h = 0; h < 2; h++) {
 		if ((int)D->src[h].size() > MAXSRC) return fail("more than 128 sources in one chain");
 		std::vector<PostOp<T>> adds, copies;
@@ -2291,67 +1992,68 @@ int buildPost(alis_dev_world *D)
 			o.c = (T)S.amp;
 			adds.push_back(o);
 		}
-		for (const CopySpec &c : ghostSchedule(&D->W, h)) {
-			PostOp<T> o{};
-			o.kind = OP_COPY;
-			o.F = (T *)D->F[h][0][c.axis];
-			o.G = D->cplx ? (T *)D->F[h][1][c.axis] : nullptr;
-			o.LF = D->L;
-			o.b = c.b;
-			o.di = c.di, o.dj = c.dj, o.dk = c.dk;
-			o.c = (T)c.c, o.s = (T)c.s;
-			copies.push_back(o);
+		copies = copyOps<T>(D, h);
+		dropEmpty(adds);
+		// k_step applies additive operations to the cells it updates
+		std::vector<StepAdd<T>> list[2];
+		for (PostOp<T> o : adds) {
+			// what an operation adds to cells beyond is lost where a ghost copy overwrites them
+			for (const Box &x : outsideParts(o.b, range)) {
+				bool lost = false;
+				for (const PostOp<T> &t : copies)
+					lost = lost || ((t.F == o.F || t.G == o.F) && x.i0 >= t.b.i0 && x.i1 <= t.b.i1 && x.j0 >= t.b.j0 && x.j1 <= t.b.j1 && x.k0 >= t.b.k0 && x.k1 <= t.b.k1);
+				if (!lost) D->addsInside = false;
+			}
+			o.b = Box{std::max(o.b.i0, range.i0), std::min(o.b.i1, range.i1), std::max(o.b.j0, range.j0), std::min(o.b.j1, range.j1),
+			          std::max(o.b.k0, range.k0), std::min(o.b.k1, range.k1)};
+			if (!o.b.count()) continue;
+			for (int m = 0; m <= D->cplx; m++)
+				for (int a = 0; a < 3; a++)
+					if (o.F == (T *)D->F[h][m][a]) list[m].push_back(StepAdd<T>{o, a});
 		}
-		auto nonEmpty = [](std::vector<PostOp<T>> &v) {
-			v.erase(std::remove_if(v.begin(), v.end(), [](const PostOp<T> &o) { return o.b.count() == 0; }), v.end());
-		};
-		nonEmpty(adds), nonEmpty(copies);
-		// fused steps keep the two sets equal on the cells no step writes, which an additive
-		// operation outside the update range (applied on some steps only) would break
-		for (const PostOp<T> &o : adds)
-			if (o.b.i0 < range.i0 || o.b.i1 > range.i1 || o.b.j0 < range.j0 || o.b.j1 > range.j1 || o.b.k0 < range.k0 || o.b.k1 > range.k1)
-				D->fixOk = false;
-		if (h == 0) {
-			for (const PostOp<T> &o : adds) eOps.push_back(o.b);
-			for (const PostOp<T> &o : copies) eOps.push_back(o.b);
+		for (int m = 0; m <= D->cplx; m++) {
+			D->adds[m][h].clear();
+			D->addTab[m][h] = D->addAt[m][h] = nullptr;
+			if (list[m].size() > (size_t)MAXADD) D->addsInside = false;
+			if (!D->addsInside || list[m].empty()) continue;
+			std::vector<unsigned long long> at(D->iNUM, 0ull);
+			for (size_t u = 0; u < list[m].size(); u++) {
+				const PostOp<T> &o = list[m][u].o;
+				D->adds[m][h].push_back({o.kind, o.slot});
+				for (int i = o.b.i0; i <= o.b.i1; i++) at[i - D->iMIN] |= 1ull << u;
+			}
+			if (devAlloc(D, &D->addTab[m][h], list[m].size() * sizeof(StepAdd<T>))) return -1;
+			if (devAlloc(D, &D->addAt[m][h], at.size() * sizeof(at[0]))) return -1;
+			HIPCHECK(hipMemcpyAsync(D->addTab[m][h], list[m].data(), list[m].size() * sizeof(StepAdd<T>), hipMemcpyHostToDevice, D->st));
+			HIPCHECK(hipMemcpyAsync(D->addAt[m][h], at.data(), at.size() * sizeof(at[0]), hipMemcpyHostToDevice, D->st));
+			HIPCHECK(hipStreamSynchronize(D->st));
 		}
-		else {
-			D->hWrites.clear();
+		if (h == 1) {
+			D->hWrites.clear(), D->hCopies.clear();
 			for (const PostOp<T> &o : adds) D->hWrites.push_back(o.b);
-			for (const PostOp<T> &o : copies) D->hWrites.push_back(o.b);
+			for (const PostOp<T> &o : copies) D->hWrites.push_back(o.b), D->hCopies.push_back(o.b);
 		}
-		copyOps[h] = copies;
+		std::vector<std::vector<PostOp<T>>> segOps;
+		std::vector<int> segAdd;
 		if (copies.size() <= (size_t)MAXCHAIN && adds.size() + copies.size() <= (size_t)MAXPOST && !postConflict(adds, copies)) {
 			std::vector<PostOp<T>> all = adds;
 			all.insert(all.end(), copies.begin(), copies.end());
-			if (!all.empty()) segOps[h].push_back(all), segAdd[h].push_back((int)adds.size());
-			continue;
+			if (!all.empty()) segOps.push_back(all), segAdd.push_back((int)adds.size());
 		}
-		for (size_t a0 = 0; a0 < adds.size(); a0 += MAXPOST) {
-			std::vector<PostOp<T>> chunk(adds.begin() + a0, adds.begin() + std::min(adds.size(), a0 + MAXPOST));
-			segOps[h].push_back(chunk), segAdd[h].push_back((int)chunk.size());
-		}
-		std::vector<PostOp<T>> group;
-		const std::vector<PostOp<T>> none;
-		for (const PostOp<T> &o : copies) {
-			std::vector<PostOp<T>> trial = group;
-			trial.push_back(o);
-			if (!group.empty() && (trial.size() > (size_t)MAXCHAIN || postConflict(none, trial))) {
-				segOps[h].push_back(group), segAdd[h].push_back(0);
-				group.assign(1, o);
+		else {
+			for (size_t a0 = 0; a0 < adds.size(); a0 += MAXPOST) {
+				std::vector<PostOp<T>> chunk(adds.begin() + a0, adds.begin() + std::min(adds.size(), a0 + MAXPOST));
+				segOps.push_back(chunk), segAdd.push_back((int)chunk.size());
 			}
-			else group.swap(trial);
+			for (const std::vector<PostOp<T>> &g : copyGroups(copies)) segOps.push_back(g), segAdd.push_back(0);
 		}
-		if (!group.empty()) segOps[h].push_back(group), segAdd[h].push_back(0);
-	}
-	for (int h = 0; h < 2; h++) {
 		D->post[h].clear();
 		D->carry[h].clear();
-		for (size_t g = 0; g < segOps[h].size(); g++) {
-			const std::vector<PostOp<T>> &v = segOps[h][g];
+		for (size_t g = 0; g < segOps.size(); g++) {
+			const std::vector<PostOp<T>> &v = segOps[g];
 			std::vector<PostPiece> pieces;
 			PostSeg seg;
-			buildPieces(v, segAdd[h][g], pieces, seg.total);
+			if (postSegment(D, v, segAdd[g], pieces, seg)) return -1;
 			if (pieces.empty()) continue;
 			// A copy chain starts from a cell no earlier copy of its launch writes.  Where that
 			// cell lies outside the update range and a copy of the program writes it (later:
@@ -2363,7 +2065,7 @@ int buildPost(alis_dev_world *D)
 				int axis = -1;
 				for (int a = 0; a < 3; a++) if (o.F == (T *)D->F[h][0][a]) axis = a;
 				const Box base{P.b.i0 + P.si, P.b.i1 + P.si, P.b.j0 + P.sj, P.b.j1 + P.sj, P.b.k0 + P.sk, P.b.k1 + P.sk};
-				for (const PostOp<T> &t : copyOps[h]) {
+				for (const PostOp<T> &t : copies) {
 					if (t.F != o.F) continue;
 					for (const Box &part : outsideParts(t.b, range)) {
 						const Box x{std::max(base.i0, part.i0), std::min(base.i1, part.i1), std::max(base.j0, part.j0),
@@ -2372,67 +2074,145 @@ int buildPost(alis_dev_world *D)
 					}
 				}
 			}
-			if (seg.total >= (1L << 31)) return fail("end-of-half-step launch over 2^31 threads");
-			std::vector<PostPiece> perBlock(seg.total / POST_WG);
-			for (const PostPiece &P : pieces)
-				for (long b = P.off / POST_WG; b < (P.off + P.b.count() + POST_WG - 1) / POST_WG; b++) perBlock[b] = P;
-			if (devAlloc(D, &seg.ops, v.size() * sizeof(PostOp<T>))) return -1;
-			if (devAlloc(D, &seg.pieces, perBlock.size() * sizeof(PostPiece))) return -1;
-			HIPCHECK(hipMemcpyAsync(seg.ops, v.data(), v.size() * sizeof(PostOp<T>), hipMemcpyHostToDevice, D->st));
-			HIPCHECK(hipMemcpyAsync(seg.pieces, perBlock.data(), perBlock.size() * sizeof(PostPiece), hipMemcpyHostToDevice, D->st));
-			HIPCHECK(hipStreamSynchronize(D->st));   // the host vectors end with this iteration
 			D->post[h].push_back(seg);
 		}
 	}
 	HIPCHECK(hipStreamSynchronize(D->st));
 	D->postBuilt = true;
-	D->fix = fixBoxes(eOps, range);
-	long fixCells = 0;
-	for (const Box &b : D->fix) fixCells += b.count();
-	if (D->fix.size() > (size_t)MAXFIX || fixCells * 4 > range.count()) D->fixOk = false;   // not worth it
-	for (int h = 0; h < 2; h++)
-		if (D->carry[h].size() * (1 + D->cplx) > (size_t)MAXCARRY) D->fixOk = false;
+	if ((D->carry[0].size() + D->carry[1].size()) * (1 + D->cplx) > (size_t)MAXCARRY) D->addsInside = false;
 	return 0;
 }
 
-// Run the end of half step h: the recorded strips and sources, then the ghost copies.
+// For fused steps: the ghost copies of both halves as a program of their own.  E's copies write E
+// alone and H's H alone, so one launch takes both where they fit.
 template<class T>
-int postHalf(alis_dev_world *D, int h)
+int buildCopies(alis_dev_world *D)
 {
-	if (!D->postBuilt && buildPost<T>(D)) return -1;
-	if (D->carryDue[h]) {
-		D->carryDue[h] = false;
-		CarryArgs<T> c{};
-		for (const alis_dev_world::Carry &x : D->carry[h])
-			for (int m = 0; m <= D->cplx; m++) {
-				c.src[c.n] = (const T *)D->Falt[h][m][x.axis], c.dst[c.n] = (T *)D->F[h][m][x.axis];
-				c.b[c.n] = x.b, c.off[c.n + 1] = c.off[c.n] + x.b.count();
-				c.n++;
-			}
-		c.L = D->L;
-		if (c.n) {
-			k_carry<T><<<blocksFor(c.off[c.n]), 256, 0, D->st>>>(c);
-			HIPCHECK(hipGetLastError());
-		}
+	std::vector<PostOp<T>> both = copyOps<T>(D, 0), copies = copyOps<T>(D, 1);
+	both.insert(both.end(), copies.begin(), copies.end());
+	D->copies.clear();
+	for (const std::vector<PostOp<T>> &g : copyGroups(both)) {
+		std::vector<PostPiece> pieces;
+		PostSeg seg;
+		if (postSegment(D, g, 0, pieces, seg)) return -1;
+		if (!pieces.empty()) D->copies.push_back(seg);
 	}
-	PostArgs<T> a{};
-	a.strips = D->pendStrips[h];
-	for (size_t w = 0; w < D->pendSrc[h].size(); w++) a.src[w] = D->pendSrc[h][w];
-	for (size_t q = 0; q < D->pendWave[h].size(); q++) a.wave[q] = (T)D->pendWave[h][q];
-	// Strips read the auxiliary fields of the other kind, which the auxiliary world's half
-	// steps write on its own stream: they wait for its last half step, and its next one
-	// waits for them.  Both events are bound to the worlds' last post launches, so the
-	// ordering adds no marker to either stream.
-	auto sideStream = [&](size_t s) { return ((a.strips >> s) & 1u) && D->tf[s].aux->st != D->st; };
+	HIPCHECK(hipStreamSynchronize(D->st));
+	D->copiesBuilt = true;
+	return 0;
+}
+
+int flushE(alis_dev_world *D);
+
+// Make D's stream wait for the last half step of the auxiliary worlds (on other streams) whose
+// strips apply.
+int waitForAux(alis_dev_world *D, unsigned strips)
+{
 	for (size_t s = 0; s < D->tf.size(); s++) {
-		if (!sideStream(s)) continue;
 		alis_dev_world *X = D->tf[s].aux;
+		if (!((strips >> s) & 1u)) continue;
+		if (X->st == D->st) continue;
 		if (!X->halfDone) {
 			HIPCHECK(hipEventCreateWithFlags(&X->halfDone, hipEventDisableTiming));
 			HIPCHECK(hipEventRecord(X->halfDone, X->st));
 		}
 		HIPCHECK(hipStreamWaitEvent(D->st, X->halfDone, 0));
 	}
+	return 0;
+}
+
+// The current update of the last H core, where no end-of-half-step launch took it along.
+template<class T>
+int flushAde(alis_dev_world *D)
+{
+	if (!D->pendAde) return 0;
+	D->pendAde = false;
+	k_ade<T><<<objBlocks(D), POST_WG, 0, D->st>>>(objArgs<T>(D));
+	HIPCHECK(hipGetLastError());
+	return 0;
+}
+
+// What the end of half step h applies: the recorded strips and sources, which are done with.
+template<class T>
+PostArgs<T> postArgs(alis_dev_world *D, int h)
+{
+	PostArgs<T> a{};
+	a.strips = D->pendStrips[h];
+	for (size_t w = 0; w < D->pendSrc[h].size(); w++) a.src[w] = D->pendSrc[h][w];
+	for (size_t q = 0; q < D->pendWave[h].size(); q++) a.wave[q] = (T)D->pendWave[h][q];
+	D->pendStrips[h] = 0;
+	std::fill(D->pendSrc[h].begin(), D->pendSrc[h].end(), 0u);
+	return a;
+}
+
+// Whether the half steps of D's auxiliary world run in D's launches (see k_curl_aux).
+template<class T>
+int foldsAux(alis_dev_world *D, bool &on)
+{
+	on = false;
+	if (D->tf.empty() || D->foldState < 0) return 0;
+	alis_dev_world *A = D->tf[0].aux;
+	if (!D->foldState) {
+		D->foldState = -1;
+		if (D->tf.size() != 1 || !A || A->mainOf != D || A == D || !A->tf.empty() || !A->obj.empty()) return 0;
+		if (!A->postBuilt && buildPost<T>(A)) return -1;
+		const long tiles = ((long)A->jNUM * (A->L.sj / Quads<T>::N) + CURL_WG - 1) / CURL_WG * A->iNUM * (1 + A->cplx);
+		if (tiles > AUX_TILES) return 0;
+		for (int h = 0; h < 2; h++) {
+			if (A->post[h].empty() || A->post[h].size() > (size_t)AUX_SEGS + 1) return 0;
+			for (size_t g = 0; g + 1 < A->post[h].size(); g++)
+				if (A->post[h][g].total > AUX_UNITS * (long)POST_WG) return 0;
+		}
+		if (joinStream(A, D)) return -1;
+		D->foldState = 1;
+	}
+	on = !A->timing && A->st == D->st && A->par == 0;
+	return 0;
+}
+
+template<class T>
+int postHalf(alis_dev_world *D, int h, const PostArgs<T> *x = nullptr);
+
+// A half step of D and of its auxiliary world, both waiting: two launches (three with objects, or a
+// main program of several).
+template<class T>
+int foldedHalf(alis_dev_world *D, int h)
+{
+	alis_dev_world *A = D->tf[0].aux;
+	D->pendMain = A->pendCore = A->pendGhosts = 0;
+	dropPresamples(A);
+	if (!A->postBuilt && buildPost<T>(A)) return -1;
+	AuxCurl<T> x{};
+	static_assert(sizeof(HalfArgs<T>) + sizeof x + sizeof(ZFaces<T>) <= 4096 && 2 * sizeof(PostArgs<T>) <= 4096, "kernel arguments");
+	x.parts = 1 + A->cplx;
+	for (int m = 0; m <= A->cplx; m++) x.part[m] = halfArgs<T>(A, h, m);
+	x.post = postArgs<T>(A, h);
+	for (size_t g = 0; g + 1 < A->post[h].size(); g++) {
+		const PostSeg &G = A->post[h][g];
+		x.seg[x.segs].ops = (const PostOp<T> *)G.ops, x.seg[x.segs].pieces = (const PostPiece *)G.pieces;
+		x.seg[x.segs++].n = (int)blocksFor(G.total, POST_WG);
+	}
+	if (coreHalf<T>(D, h, &x)) return -1;
+	PostArgs<T> last = x.post;
+	const PostSeg &G = A->post[h].back();
+	last.ops = (const PostOp<T> *)G.ops, last.pieces = (const PostPiece *)G.pieces;
+	last.total = G.total, last.post = (int)blocksFor(G.total, POST_WG);
+	return postHalf<T>(D, h, &last);
+}
+
+// Run the end of half step h: the recorded strips and sources, then the ghost copies.
+// x: an auxiliary world's launch to take along, or null.
+template<class T>
+int postHalf(alis_dev_world *D, int h, const PostArgs<T> *x)
+{
+	if (!D->postBuilt && buildPost<T>(D)) return -1;
+	PostArgs<T> a = postArgs<T>(D, h);
+	// Strips read the auxiliary fields of the other kind, which the auxiliary world's half
+	// steps write on its own stream: they wait for its last half step, and its next one
+	// waits for them.  Both events are bound to the worlds' last post launches, so the
+	// ordering adds no marker to either stream.
+	auto sideStream = [&](size_t s) { return ((a.strips >> s) & 1u) && D->tf[s].aux->st != D->st; };
+	if (waitForAux(D, a.strips)) return -1;
 	// the end of this program: an event the auxiliary world's stream waits for (a world with
 	// strips on another stream), or the main world's (an auxiliary world)
 	bool bind = D->isAux;
@@ -2445,16 +2225,22 @@ int postHalf(alis_dev_world *D, int h)
 		if (!G.total) continue;
 		a.ops = (const PostOp<T> *)G.ops;
 		a.pieces = (const PostPiece *)G.pieces;
-		a.total = G.total;
-		if (g == last) launchEv(k_post<T>, dim3(blocksFor(G.total, POST_WG)), dim3(POST_WG), 0, D->st, nullptr, bind ? D->halfDone : nullptr, a);
-		else k_post<T><<<blocksFor(G.total, POST_WG), POST_WG, 0, D->st>>>(a);
+		a.total = G.total, a.post = (int)blocksFor(G.total, POST_WG);
+		unsigned blocks = a.post;
+		if (g == last && h == 1 && D->pendAde) a.ade = objArgs<T>(D), blocks += objBlocks(D), D->pendAde = false;
+		if (g == last && x) launchEv(k_post_aux<T>, dim3(blocks + x->post), dim3(POST_WG), 0, D->st, nullptr, bind ? D->halfDone : nullptr, a, *x, (int)blocks);
+		else if (g == last) launchEv(k_post<T>, dim3(blocks), dim3(POST_WG), 0, D->st, nullptr, bind ? D->halfDone : nullptr, a);
+		else k_post<T><<<blocks, POST_WG, 0, D->st>>>(a);
+		HIPCHECK(hipGetLastError());
+	}
+	if (last < 0 && flushAde<T>(D)) return -1;
+	if (last < 0 && x) {
+		k_post<T><<<x->post, POST_WG, 0, D->st>>>(*x);
 		HIPCHECK(hipGetLastError());
 	}
 	if (last < 0 && bind) HIPCHECK(hipEventRecord(D->halfDone, D->st));
 	for (size_t s = 0; s < D->tf.size(); s++)
 		if (sideStream(s)) HIPCHECK(hipStreamWaitEvent(D->tf[s].aux->st, D->halfDone, 0));
-	D->pendStrips[h] = 0;
-	std::fill(D->pendSrc[h].begin(), D->pendSrc[h].end(), 0u);
 	return 0;
 }
 
@@ -2490,12 +2276,9 @@ void swapSets(alis_dev_world *D)
 	for (int h = 0; h < 2; h++)
 		for (DevSlab &S : D->slab[h])
 			for (int m = 0; m < 2; m++) std::swap(S.p[m][0], S.alt[m][0]), std::swap(S.p[m][1], S.alt[m][1]);
-	for (DevObj &O : D->obj)
-		for (int m = 0; m < 2; m++)
-			for (int c = 0; c < 3; c++)
-				for (int p = 0; p < MAXPOLE; p++) std::swap(O.J[m][c][p], O.Jalt[m][c][p]), std::swap(O.K[m][c][p], O.Kalt[m][c][p]);
-	std::swap(D->objTab, D->objTabAlt);
 	for (int h = 0; h < 2; h++) std::swap(D->post[h], D->postAlt[h]);
+	std::swap(D->copies, D->copiesAlt);
+	std::swap(D->copiesBuilt, D->copiesBuiltAlt);
 	std::swap(D->postBuilt, D->postBuiltAlt);
 	D->par ^= 1;
 }
@@ -2512,17 +2295,12 @@ int ensureAlt(alis_dev_world *D)
 					if (devAlloc(D, &D->Falt[h][m][a], D->fsize * sizeof(T))) return -1;
 		for (int h = 0; h < 2; h++)
 			for (DevSlab &S : D->slab[h])
-				for (int m = 0; S.on && m <= D->cplx; m++)
+				for (int m = 0; S.n && m <= D->cplx; m++)
 					for (int x = 0; x < 2; x++)
 						if (devAlloc(D, &S.alt[m][x], S.n * sizeof(T))) return -1;
-		for (DevObj &O : D->obj)
-			for (int m = 0; m <= D->cplx; m++)
-				for (int c = 0; c < 3; c++)
-					for (int p = 0; p < O.NK; p++) {
-						if (devAlloc(D, &O.Jalt[m][c][p], O.box.count() * sizeof(T))) return -1;
-						if (p >= O.NJ && devAlloc(D, &O.Kalt[m][c][p], O.box.count() * sizeof(T))) return -1;
-					}
-		if (!D->obj.empty() && uploadObjTable<T>(D, true, &D->objTabAlt)) return -1;
+		for (int h = 0; h < 2; h++)
+			for (int a = 0; a < 3; a++)       // a max face in its min face's array
+				if (D->slab[h][a + 3].on && !D->slab[h][a + 3].n) memcpy(D->slab[h][a + 3].alt, D->slab[h][a].alt, sizeof D->slab[h][a].alt);
 		D->altReady = true, D->altStale = true;
 	}
 	if (D->altStale) {
@@ -2534,88 +2312,93 @@ int ensureAlt(alis_dev_world *D)
 				for (int a = 0; a < 3; a++) HIPCHECK(copy(D->Falt[h][m][a], D->F[h][m][a], D->fsize));
 		for (int h = 0; h < 2; h++)
 			for (DevSlab &S : D->slab[h])
-				for (int m = 0; S.on && m <= D->cplx; m++)
+				for (int m = 0; S.n && m <= D->cplx; m++)
 					for (int x = 0; x < 2; x++) HIPCHECK(copy(S.alt[m][x], S.p[m][x], S.n));
-		for (DevObj &O : D->obj)
-			for (int m = 0; m <= D->cplx; m++)
-				for (int c = 0; c < 3; c++)
-					for (int p = 0; p < O.NK; p++) {
-						HIPCHECK(copy(O.Jalt[m][c][p], O.J[m][c][p], O.box.count()));
-						if (p >= O.NJ) HIPCHECK(copy(O.Kalt[m][c][p], O.K[m][c][p], O.box.count()));
-					}
 		D->altStale = false;
 	}
 	return 0;
 }
 
-// Launch shape of k_step for D: NC waves per row (64 cells each), R rows per group and the
-// row below them (R + 1 = 16 / NC rows, at most 9, fewer where the two planes of LDS rows
-// would pass 64 KiB), P values per LDS row and component, x planes per chunk (8;
-// ALIS_STEP_CHUNK and ALIS_STEP_ROWS override).
-struct StepShape { int NC, R, P, chunk, ngroup, nchunk; size_t lds; };
+// Launch shape of k_step for one part of D.
+struct StepShape { int pq, zq, own, ntile, chunk, nchunk; long blocks; size_t lds; };
 
 StepShape stepShape(const alis_dev_world *D)
 {
 	StepShape s{};
-	s.NC = (D->kNUM + 63) / 64;
-	s.P = 64 * s.NC + 1;
-	const size_t row = 2 * 3 * (size_t)s.P * D->esz;
-	s.R = std::min({8, 16 / std::max(s.NC, 1) - 1, (int)(65536 / row) - 1});
-	if (const char *e = getenv("ALIS_STEP_ROWS")) s.R = std::min(s.R, atoi(e));
-	if (s.R < 1) s.R = 1;
-	s.lds = (s.R + 1) * row;
-	s.ngroup = (D->jNUM + s.R - 1) / s.R;
+	const int quad = 16 / (int)D->esz;
+	s.pq = (int)(D->L.sj / quad);
+	for (int h = 0; h < 2; h++) {
+		int z = 0;
+		for (int f : {2, 5}) if (D->slab[h][f].on) z = D->slab[h][f].first + (D->slab[h][f].hi - D->kMIN) / quad - (D->slab[h][f].lo - D->kMIN) / quad + 1;
+		s.zq = std::max(s.zq, z);
+	}
+	s.lds = (4 * STEP_THREADS + 2 * s.pq + 6 * s.zq) * 16 + 32 * D->esz;
+	s.own = STEP_THREADS - s.pq;
+	if (s.own < 1) return s;
+	s.ntile = (D->jNUM * s.pq + s.own - 1) / s.own;
 	s.chunk = 8;
 	if (const char *e = getenv("ALIS_STEP_CHUNK")) s.chunk = std::max(1, atoi(e));
 	s.nchunk = (D->iNUM + s.chunk - 1) / s.chunk;
+	s.blocks = 8L * s.ntile * ((s.nchunk + 7) / 8);
 	return s;
 }
 
-// Whether D's steps run fused: decided once per world (again after a TF/SF link).  Off
-// unless ALIS_FUSE is 1 (worlds that give k_step two workgroups per CU and at least 3 rows
-// per group) or force (every world whose results it can reproduce): on the 256^3 nanoblock
-// k_step takes 560 us against 286 us for the two separate curl launches.
+// Whether D's steps run fused: possible worlds are decided once (again after a TF/SF link).  Off
+// unless ALIS_FUSE is 1 (worlds that give every CU a workgroup of k_step) or force (every world whose
+// results it can reproduce).
 template<class T>
 int fusedSteps(alis_dev_world *D, bool &on)
 {
 	on = false;
 	if (D->isAux || D->inBatch) return 0;
+	const char *env = getenv("ALIS_FUSE");
+	const bool force = env && !strcmp(env, "force");
+	if (!force && !(env && !strcmp(env, "1"))) return 0;
 	if (!D->fuseState) {
 		D->fuseState = -1;
-		const char *env = getenv("ALIS_FUSE");
 		for (const DevTfsf &t : D->tf)
-			if (!t.aux) return 0;           // its programs cannot be built yet
+			if (!t.aux || !t.aux->tf.empty()) return 0;   // not linked yet, or an auxiliary world of its own
 		if (!D->postBuilt && buildPost<T>(D)) return -1;
-		const StepShape s = stepShape(D);
-		const bool force = env && !strcmp(env, "force");   // every world where the results allow it
-		const bool on = force || (env && !strcmp(env, "1"));
-		if (on && D->fixOk && s.NC <= 8 && (force || (s.R >= 3 && (long)s.ngroup * s.nchunk >= 512)))
-			D->fuseState = 1;
+		const StepShape z = stepShape(D);
+		// rows of at most half a workgroup
+		if (!D->addsInside || 2 * z.pq > STEP_THREADS || z.blocks >= (1L << 31) || z.lds > 65536) return 0;
+		// the other set takes as much memory again: without it the halves stay apart
+		const size_t na = D->allocs.size();
+		const long nb = D->bytes;
+		if (ensureAlt<T>(D)) {
+			(void)hipGetLastError();
+			HIPCHECK(hipStreamSynchronize(D->st));
+			for (size_t a = na; a < D->allocs.size(); a++) HIPCHECK(hipFree(D->allocs[a]));
+			D->allocs.resize(na), D->bytes = nb;
+			return 0;
+		}
+		D->fuseState = 1;
 	}
-	on = D->fuseState > 0;
+	const StepShape z = stepShape(D);
+	on = D->fuseState > 0 && (force || (long)z.ntile * z.nchunk >= 256);
 	return 0;
 }
 
-// Point the results of a half's arguments (built on the current set) at the other set.
-template<class T>
-void toOtherSet(alis_dev_world *D, int h, int m, CurlArgs<T> &a)
-{
-	a.O0 = (T *)D->Falt[h][m][0], a.O1 = (T *)D->Falt[h][m][1], a.O2 = (T *)D->Falt[h][m][2];
-	for (int f = 0; f < 6; f++)
-		if (a.face[f].on) a.face[f].qa = (T *)D->slab[h][f].alt[m][0], a.face[f].qb = (T *)D->slab[h][f].alt[m][1];
-	a.objOut = (const ObjDev<T> *)D->objTabAlt;
-}
-
-// k_step's argument table: for each set as the current one, each part.
+// k_step's argument table: for each part, each set as the current one.
 template<class T>
 int stepTable(alis_dev_world *D)
 {
 	StepArgs<T> t[2][2] = {};
+	const StepShape z = stepShape(D);
 	for (int pass = 0; pass < 2; pass++) {
 		for (int m = 0; m <= D->cplx; m++) {
-			StepArgs<T> &s = t[D->par][m];
-			s.e = curlArgs<T>(D, 0, m), s.h = curlArgs<T>(D, 1, m);
-			toOtherSet<T>(D, 0, m, s.e), toOtherSet<T>(D, 1, m, s.h);
+			StepArgs<T> &s = t[m][D->par];
+			s.e = halfArgs<T>(D, 0, m), s.h = halfArgs<T>(D, 1, m);
+			for (int h = 0; h < 2; h++) {
+				for (int c = 0; c < 3; c++) {
+					s.O[h][c] = (T *)D->Falt[h][m][c];
+					for (int f : {c, c + 3})
+						if (D->slab[h][f].on) s.qa[h][c] = (T *)D->slab[h][f].alt[m][0], s.qb[h][c] = (T *)D->slab[h][f].alt[m][1];
+				}
+				s.add[h] = (const StepAdd<T> *)D->addTab[m][h], s.addAt[h] = (const unsigned long long *)D->addAt[m][h];
+				s.nadd[h] = (int)D->adds[m][h].size();
+			}
+			s.zq = z.zq, s.own = z.own, s.chunk = z.chunk, s.nchunk = z.nchunk, s.ntile = z.ntile;
 		}
 		swapSets(D);
 	}
@@ -2625,81 +2408,166 @@ int stepTable(alis_dev_world *D)
 	return 0;
 }
 
-// A whole step of D after its deferred E half: k_step from the current set into the other,
-// the sets exchanged, the E half's end-of-step program on the new set, H again where that
-// program changed E (k_fix: old H, psi and currents, final E).
+// The operations of part m switched on this step.
+template<class T>
+StepDyn<T> stepDyn(const alis_dev_world *D, int m)
+{
+	StepDyn<T> d{};
+	d.par = D->par;
+	for (int h = 0; h < 2; h++)
+		for (size_t u = 0; u < D->adds[m][h].size(); u++) {
+			const alis_dev_world::AddRef &r = D->adds[m][h][u];
+			const bool on = r.kind == OP_STRIP ? (D->pendStrips[h] >> r.slot) & 1u : (D->pendSrc[h][r.slot >> 5] >> (r.slot & 31)) & 1u;
+			if (on) d.on[h] |= 1ull << u;
+			if (on && r.kind == OP_SOURCE) d.wave[h][u] = (T)D->pendWave[h][r.slot];
+		}
+	return d;
+}
+
+// Run D's deferred step: k_step from the current set into the other, the sets exchanged, the
+// ghost copies of both halves.  The auxiliary worlds have made their E half step; their H half
+// waits for k_step, which reads their old H (auxHalves).
+template<class T>
+int auxHalves(alis_dev_world *D);
+
 template<class T>
 int fusedStep(alis_dev_world *D)
 {
-	dropPresamples(D);
+	D->pendE = 0;
 	if (ensureAlt<T>(D)) return -1;
+	if (!D->postBuilt && buildPost<T>(D)) return -1;
 	if (!D->stepArgs && stepTable<T>(D)) return -1;
+	dropPresamples(D);
 	hipEvent_t e0 = nullptr, e1 = nullptr;
 	if (D->timing && timingEvents(D, e0, e1)) return -1;
+	const unsigned strips = D->pendStrips[0] | D->pendStrips[1];
+	if (waitForAux(D, strips)) return -1;
+	bool side = false;
+	for (size_t s = 0; s < D->tf.size(); s++) side = side || (((strips >> s) & 1u) && D->tf[s].aux->st != D->st);
+	if (side && !D->halfDone) HIPCHECK(hipEventCreateWithFlags(&D->halfDone, hipEventDisableTiming));
+	// the objects' currents, into the set that this step replaces
+	if (D->objWgs) k_currents<T><<<objBlocks(D), OBJ_WG, 0, D->st>>>(objArgs<T>(D));
 	const StepShape z = stepShape(D);
-	const dim3 grid((unsigned)(8 * z.ngroup * ((z.nchunk + 7) / 8))), block(64, z.NC, z.R + 1);
+	const dim3 grid((unsigned)z.blocks), block(STEP_THREADS);
+	const size_t lds = z.lds;
+	std::vector<DevPhaser *> sampled;
 	for (int m = 0; m <= D->cplx; m++) {
-		const StepArgs<T> *sa = (const StepArgs<T> *)D->stepArgs + 2 * D->par + m;
-		hipEvent_t s0 = m == 0 ? e0 : nullptr, s1 = m == D->cplx ? e1 : nullptr;
-		if (D->seg) hipExtLaunchKernelGGL(k_step<T, 2>, grid, block, z.lds, D->st, s0, s1, 0, sa, z.R, z.P, z.chunk, z.nchunk, z.ngroup);
-		else if (D->C[0]) hipExtLaunchKernelGGL(k_step<T, 1>, grid, block, z.lds, D->st, s0, s1, 0, sa, z.R, z.P, z.chunk, z.nchunk, z.ngroup);
-		else hipExtLaunchKernelGGL(k_step<T, 0>, grid, block, z.lds, D->st, s0, s1, 0, sa, z.R, z.P, z.chunk, z.nchunk, z.ngroup);
+		const StepArgs<T> *sa = (const StepArgs<T> *)D->stepArgs + 2 * m;
+		StepDyn<T> d = stepDyn<T>(D, m);
+		if (m == 0) d.nzs = zSamples<T>(D, d.zs, sampled, true);   // phasers sample part 0
+		hipEvent_t s0 = m == 0 ? e0 : nullptr, s1 = m == D->cplx ? e1 ? e1 : side ? D->halfDone : nullptr : nullptr;
+#define STEP(C) (d.nzs ? launchEv(k_step<T, C, true>, grid, block, lds, D->st, s0, s1, sa, d) : launchEv(k_step<T, C, false>, grid, block, lds, D->st, s0, s1, sa, d))
+		if (D->seg) STEP(2);
+		else if (D->C[0]) STEP(1);
+		else STEP(0);
+#undef STEP
 		HIPCHECK(hipGetLastError());
 	}
 	if (e1) {
 		D->evPairs[2].push_back(e0);
 		D->evPairs[2].push_back(e1);
+		if (side) HIPCHECK(hipEventRecord(D->halfDone, D->st));
 	}
 	swapSets(D);
-	D->pendE = 0;
-	D->carryDue[0] = D->carryDue[1] = true;   // both programs of this step run on the new set
-	if (postHalf<T>(D, 0)) return -1;
-	if (D->fix.empty()) return 0;
-	FixBoxes f{};
-	f.n = (int)D->fix.size();
-	for (int q = 0; q < f.n; q++) f.b[q] = D->fix[q], f.off[q + 1] = f.off[q] + D->fix[q].count();
-	for (int m = 0; m <= D->cplx; m++) {
-		CurlArgs<T> a = curlArgs<T>(D, 1, m);       // the new set: results, and the final E
-		a.O0 = a.F0, a.O1 = a.F1, a.O2 = a.F2;
-		a.F0 = (T *)D->Falt[1][m][0], a.F1 = (T *)D->Falt[1][m][1], a.F2 = (T *)D->Falt[1][m][2];
-		for (int g = 0; g < 6; g++)
-			if (a.face[g].on) {
-				CurlFace<T> &P = a.face[g];
-				P.qa = P.pa, P.qb = P.pb;
-				P.pa = (T *)D->slab[1][g].alt[m][0], P.pb = (T *)D->slab[1][g].alt[m][1];
+	if (!D->postBuilt && buildPost<T>(D)) return -1;     // the other set's programs, once
+	if (!D->copiesBuilt && buildCopies<T>(D)) return -1;
+	CarryArgs<T> c{};
+	for (int h = 0; h < 2; h++)
+		for (const alis_dev_world::Carry &x : D->carry[h])
+			for (int m = 0; m <= D->cplx; m++) {
+				c.src[c.n] = (const T *)D->Falt[h][m][x.axis], c.dst[c.n] = (T *)D->F[h][m][x.axis];
+				c.b[c.n] = x.b, c.off[c.n + 1] = c.off[c.n] + x.b.count();
+				c.n++;
 			}
-		a.objOut = a.obj;
-		a.obj = (const ObjDev<T> *)D->objTabAlt;
-		k_fix<T><<<blocksFor(f.off[f.n]), 256, 0, D->st>>>(a, f);
+	c.L = D->L;
+	if (c.n) {
+		k_carry<T><<<blocksFor(c.off[c.n]), 256, 0, D->st>>>(c);
 		HIPCHECK(hipGetLastError());
+	}
+	D->pendAde = D->objWgs > 0;
+	PostArgs<T> a{};
+	for (const PostSeg &G : D->copies) {
+		a.ops = (const PostOp<T> *)G.ops;
+		a.pieces = (const PostPiece *)G.pieces;
+		a.total = G.total, a.post = (int)blocksFor(G.total, POST_WG);
+		unsigned blocks = a.post;
+		a.ade = ObjArgs<T>{};
+		if (D->pendAde) a.ade = objArgs<T>(D), blocks += objBlocks(D), D->pendAde = false;
+		k_post<T><<<blocks, POST_WG, 0, D->st>>>(a);
+		HIPCHECK(hipGetLastError());
+	}
+	if (flushAde<T>(D)) return -1;
+	for (int h = 0; h < 2; h++) {
+		D->pendStrips[h] = 0;
+		std::fill(D->pendSrc[h].begin(), D->pendSrc[h].end(), 0u);
+	}
+	for (size_t s = 0; side && s < D->tf.size(); s++)
+		if (((strips >> s) & 1u) && D->tf[s].aux->st != D->st) HIPCHECK(hipStreamWaitEvent(D->tf[s].aux->st, D->halfDone, 0));
+	for (DevPhaser *P : sampled) P->pre = true, P->preSlot = P->pend;
+	return auxHalves<T>(D);
+}
+
+// The H halves of D's auxiliary worlds that waited for D's deferred step.
+template<class T>
+int auxHalves(alis_dev_world *D)
+{
+	for (const DevTfsf &t : D->tf) {
+		if (!t.aux || !t.aux->pendH) continue;
+		const int p = t.aux->pendH;
+		t.aux->pendH = 0;
+		if (coreHalf<T>(t.aux, 1) || (p == 2 && postHalf<T>(t.aux, 1))) return -1;
 	}
 	return 0;
 }
 
-// Complete a deferred E half step the separate way (a call that reads or changes the world
-// between its E and H halves).
+// Complete a deferred step the separate way (a call that reads or changes the world between
+// its E and H halves, or that reads an auxiliary world whose H half waits).
 template<class T>
-int flushE(alis_dev_world *D)
+int flushStep(alis_dev_world *D)
 {
+	if (D->pendH && D->mainOf) return flushStep<T>(D->mainOf);
+	if (D->pendCore && D->mainOf) return flushStep<T>(D->mainOf);
+	if (D->pendMain) {
+		const int h = D->pendMain - 1;
+		alis_dev_world *A = D->tf[0].aux;
+		const bool core = A && A->pendCore, ghosts = A && A->pendGhosts;
+		D->pendMain = 0;
+		if (A) A->pendCore = A->pendGhosts = 0;
+		if (coreHalf<T>(D, h)) return -1;
+		if (core && coreHalf<T>(A, h)) return -1;
+		return ghosts ? postHalf<T>(A, h) : 0;
+	}
 	const int p = D->pendE;
-	if (!p) return 0;
+	if (!p) return flushAde<T>(D);
 	D->pendE = 0;
 	if (coreHalf<T>(D, 0)) return -1;
-	return p == 2 ? postHalf<T>(D, 0) : 0;
+	if (p >= 2 && postHalf<T>(D, 0)) return -1;
+	if (p >= 3 && (coreHalf<T>(D, 1) || flushAde<T>(D))) return -1;
+	return auxHalves<T>(D);
 }
 
 int flushE(alis_dev_world *D)
 {
-	return D->fp64 ? flushE<double>(D) : flushE<float>(D);
+	return D->fp64 ? flushStep<double>(D) : flushStep<float>(D);
 }
 
 template<class T>
 int coreEntry(alis_dev_world *D, int h)
 {
-	if (h == 1 && D->pendE == 2) return fusedStep<T>(D);
-	if (flushE<T>(D)) return -1;
+	if (h == 1 && D->pendE == 2) {      // the whole step runs at its alis_dev_ghosts
+		D->pendE = 3;
+		return 0;
+	}
+	if (h == 1 && D->isAux && D->mainOf && D->mainOf->pendE == 3) {
+		D->pendH = 1;
+		return 0;
+	}
+	if (D->mainOf && D->mainOf->pendMain == 1 + h && !D->pendCore && !D->pendGhosts) {
+		D->pendCore = 1 + h;
+		return 0;
+	}
+	if (flushStep<T>(D)) return -1;
 	if (h == 0) {
-		D->carryDue[1] = false;
 		bool on;
 		if (fusedSteps<T>(D, on)) return -1;
 		if (on) {
@@ -2707,7 +2575,34 @@ int coreEntry(alis_dev_world *D, int h)
 			return 0;
 		}
 	}
+	bool fold;
+	if (foldsAux<T>(D, fold)) return -1;
+	if (fold) {                         // with the auxiliary world's half step at alis_dev_ghosts
+		D->pendMain = 1 + h;
+		return 0;
+	}
 	return coreHalf<T>(D, h);
+}
+
+template<class T>
+int ghostsEntry(alis_dev_world *D, int h)
+{
+	if (h == 0 && D->pendE == 1) {      // deferred with its E core
+		D->pendE = 2;
+		return 0;
+	}
+	if (h == 1 && D->pendE == 3) return fusedStep<T>(D);
+	if (D->pendCore == 1 + h && !D->pendGhosts) {
+		D->pendGhosts = 1 + h;
+		return 0;
+	}
+	if (D->pendMain == 1 + h && D->tf[0].aux && D->tf[0].aux->pendGhosts == 1 + h) return foldedHalf<T>(D, h);
+	if (h == 1 && D->pendH == 1) {
+		D->pendH = 2;
+		return 0;
+	}
+	if ((h == 0 || D->pendE || D->pendH || D->pendCore || D->pendMain) && flushStep<T>(D)) return -1;   // (an H program takes its current update along)
+	return postHalf<T>(D, h);
 }
 
 template<class T>
@@ -2966,21 +2861,6 @@ PhsArgs<T> phaserArgs(alis_dev_world *D, DevPhaser &P, int qa, int qn)
 	return a;
 }
 
-// Make D use the stream of `to` (reference counted; the last user destroys a stream).
-int joinStream(alis_dev_world *D, alis_dev_world *to)
-{
-	if (D->st == to->st) return 0;
-	HIPCHECK(hipStreamSynchronize(D->st));
-	if (--*D->streamRefs == 0) {
-		HIPCHECK(hipStreamDestroy(D->st));
-		delete D->streamRefs;
-	}
-	D->st = to->st;
-	D->streamRefs = to->streamRefs;
-	++*to->streamRefs;
-	return 0;
-}
-
 // ---- batches: several worlds stepped in shared launches ----
 
 }  // namespace
@@ -2991,10 +2871,12 @@ struct alis_dev_batch {
 	hipStream_t st = nullptr;
 	void *curl[2] = {};         // CurlArgs<T>[] per half step
 	void *curlStart[2] = {};    // int[] workgroup starts (from 0 within each class)
-	// the entries in classes of one tile kind and one 1/eps source, each class contiguous in
-	// the tables and run by its own specialised launch
-	struct CurlClass { int first, arg, n, blocks, flat, cm, pair; };   // first: start index; arg: argument index
+	// the entries in classes of one 1/eps source, each class contiguous in the tables and run
+	// by its own specialised launch
+	struct CurlClass { int first, arg, n, blocks, cm, pair; };   // first: start index; arg: argument index
 	std::vector<CurlClass> curlClass[2];
+	void *objArgs = nullptr, *objStart = nullptr;   // ObjArgs<T>[] of the worlds with objects
+	int objEntries = 0, objBlocks = 0;
 	bool postReady = false;
 	struct Round {
 		std::vector<int> world;     // index into W
@@ -3027,47 +2909,61 @@ int batchBuildCurl(alis_dev_batch *B)
 {
 	for (int h = 0; h < 2; h++) {
 		// an entry: one part of a world, or both parts of a Bloch world (pair)
-		struct Entry { CurlArgs<T> a[2]; long tiles; int cls; };
+		struct Entry { HalfArgs<T> a[2]; int cls; };
 		const char *pe = getenv("ALIS_BATCH_PAIRS");
 		const bool pairs = !(pe && !strcmp(pe, "0"));
 		std::vector<Entry> all;
 		for (alis_dev_world *D : B->W) {
 			const bool pair = pairs && D->cplx;
 			for (int m = 0; m <= D->cplx; m++) {
-				CurlArgs<T> a = curlArgs<T>(D, h, m);
-				// tiles as k_curl_batch counts them: flat tiles for packed rows shorter than a
-				// wavefront (koff 1: rows end to end), 64 x 4 cells otherwise
-				const bool flat = D->L.koff == 1 && D->kNUM + 2 <= 64;
-				a.flatPitch = flat ? D->kNUM + 2 : 0;
-				const long tiles = flat ? (D->L.si + 255) / 256 * D->iNUM
-				                        : (long)((D->kNUM + 63) / 64) * ((D->jNUM + 3) / 4) * D->iNUM;
+				const HalfArgs<T> a = halfArgs<T>(D, h, m);
 				// 1/eps: 2 per-segment table (and arrays where a segment is mixed), 1 arrays, 0 none
-				const int cm = a.seg ? 2 : a.C0 ? 1 : 0;
+				const int cm = a.seg ? 2 : a.C[0] ? 1 : 0;
 				if (pair && m == 1) all.back().a[1] = a;
-				else all.push_back(Entry{{a, a}, tiles, (pair ? 6 : 0) + (flat ? 3 : 0) + cm});
+				else all.push_back(Entry{{a, a}, (pair ? 3 : 0) + cm});
 			}
 		}
 		std::stable_sort(all.begin(), all.end(), [](const Entry &x, const Entry &y) { return x.cls < y.cls; });
-		std::vector<CurlArgs<T>> args;
+		std::vector<HalfArgs<T>> args;
 		std::vector<int> start;
 		B->curlClass[h].clear();
 		for (const Entry &e : all) {
-			const int pair = e.cls / 6, flat = e.cls / 3 % 2, cm = e.cls % 3;
-			if (B->curlClass[h].empty() || B->curlClass[h].back().pair * 6 + B->curlClass[h].back().flat * 3 + B->curlClass[h].back().cm != e.cls)
-				B->curlClass[h].push_back({(int)start.size(), (int)args.size(), 0, 0, flat, cm, pair});
+			const int pair = e.cls / 3, cm = e.cls % 3;
+			if (B->curlClass[h].empty() || B->curlClass[h].back().pair * 3 + B->curlClass[h].back().cm != e.cls)
+				B->curlClass[h].push_back({(int)start.size(), (int)args.size(), 0, 0, cm, pair});
 			alis_dev_batch::CurlClass &c = B->curlClass[h].back();
 			args.push_back(e.a[0]);
 			if (pair) args.push_back(e.a[1]);
 			start.push_back(c.blocks);
 			c.n++;
-			const int tpb = pair ? CURL_TPB_PAIR : flat ? CURL_TPB : CURL_TPB_TILE;
-			c.blocks += (int)((e.tiles + tpb - 1) / tpb);
+			c.blocks += e.a[0].tiles * e.a[0].ni;
 		}
-		if (batchAlloc(B, &B->curl[h], args.size() * sizeof(CurlArgs<T>))) return -1;
+		if (batchAlloc(B, &B->curl[h], args.size() * sizeof(HalfArgs<T>))) return -1;
 		if (batchAlloc(B, &B->curlStart[h], start.size() * sizeof(int))) return -1;
-		HIPCHECK(hipMemcpyAsync(B->curl[h], args.data(), args.size() * sizeof(CurlArgs<T>), hipMemcpyHostToDevice, B->st));
+		HIPCHECK(hipMemcpyAsync(B->curl[h], args.data(), args.size() * sizeof(HalfArgs<T>), hipMemcpyHostToDevice, B->st));
 		HIPCHECK(hipMemcpyAsync(B->curlStart[h], start.data(), start.size() * sizeof(int), hipMemcpyHostToDevice, B->st));
+		HIPCHECK(hipStreamSynchronize(B->st));   // the host vectors end with this iteration
 	}
+	HIPCHECK(hipStreamSynchronize(B->st));
+	return 0;
+}
+
+template<class T>
+int batchBuildObjects(alis_dev_batch *B)
+{
+	std::vector<ObjArgs<T>> args;
+	std::vector<int> start;
+	for (alis_dev_world *D : B->W) {
+		if (!D->objWgs) continue;
+		args.push_back(objArgs<T>(D));
+		start.push_back(B->objBlocks);
+		B->objBlocks += objBlocks(D);
+	}
+	B->objEntries = (int)args.size();
+	if (args.empty()) return 0;
+	if (batchAlloc(B, &B->objArgs, args.size() * sizeof(ObjArgs<T>)) || batchAlloc(B, &B->objStart, start.size() * sizeof(int))) return -1;
+	HIPCHECK(hipMemcpyAsync(B->objArgs, args.data(), args.size() * sizeof(ObjArgs<T>), hipMemcpyHostToDevice, B->st));
+	HIPCHECK(hipMemcpyAsync(B->objStart, start.data(), start.size() * sizeof(int), hipMemcpyHostToDevice, B->st));
 	HIPCHECK(hipStreamSynchronize(B->st));
 	return 0;
 }
@@ -3090,6 +2986,8 @@ int batchBuildPost(alis_dev_batch *B)
 				R.world.push_back(w), R.seg.push_back((int)r);
 				start.push_back((int)R.blocks);
 				R.blocks += D->post[h][r].total / POST_WG;
+				// the current update runs with a world's last H launch
+				if (h == 1 && r + 1 == D->post[h].size()) R.blocks += objBlocks(D);
 			}
 			if (R.world.empty()) continue;
 			if (batchAlloc(B, &R.start, start.size() * sizeof(int))) return -1;
@@ -3119,43 +3017,31 @@ template<class T>
 int batchCore(alis_dev_batch *B, int h)
 {
 	alis_dev_world *D0 = B->W[0];
-	for (alis_dev_world *W : B->W) dropPresamples(W);
+	for (alis_dev_world *W : B->W) {
+		dropPresamples(W);
+		if (flushStep<T>(W)) return -1;
+		if (h == 1) W->pendAde = W->objWgs > 0;   // with the end of the half step (or flushStep)
+	}
 	hipEvent_t e0 = nullptr, e1 = nullptr;
 	if (D0->timing) {
 		if (timingEvents(D0, e0, e1)) return -1;
 	}
+	if (h == 0 && B->objEntries) {
+		k_currents_batch<T><<<B->objBlocks, OBJ_WG, 0, B->st>>>((const ObjArgs<T> *)B->objArgs, (const int *)B->objStart, B->objEntries);
+		HIPCHECK(hipGetLastError());
+	}
 	const std::vector<alis_dev_batch::CurlClass> &cls = B->curlClass[h];
 	for (size_t q = 0; q < cls.size(); q++) {
 		const alis_dev_batch::CurlClass &c = cls[q];
-		const CurlArgs<T> *args = (const CurlArgs<T> *)B->curl[h] + c.arg;
+		const HalfArgs<T> *args = (const HalfArgs<T> *)B->curl[h] + c.arg;
 		const int *start = (const int *)B->curlStart[h] + c.first;
-		const dim3 grid(c.blocks), block(64, 4);
+		const dim3 grid(c.blocks), block(CURL_WG);
 		hipEvent_t s0 = q == 0 ? e0 : nullptr, s1 = q + 1 == cls.size() ? e1 : nullptr;
-#define CURL_BATCH(F, C) launchEv(k_curl_batch<T, F ? CURL_TPB : CURL_TPB_TILE, F, C>, grid, block, 0, B->st, s0, s1, args, start, c.n)
-#define CURL_PAIR(F, C) launchEv(k_curl_batch<T, CURL_TPB_PAIR, F, C, true>, grid, block, 0, B->st, s0, s1, args, start, c.n)
-		if (c.pair) {
-			if (c.flat) {
-				if (c.cm == 2) CURL_PAIR(1, 2);
-				else if (c.cm == 1) CURL_PAIR(1, 1);
-				else CURL_PAIR(1, 0);
-			}
-			else {
-				if (c.cm == 2) CURL_PAIR(0, 2);
-				else if (c.cm == 1) CURL_PAIR(0, 1);
-				else CURL_PAIR(0, 0);
-			}
-		}
-		else if (c.flat) {
-			if (c.cm == 2) CURL_BATCH(1, 2);
-			else if (c.cm == 1) CURL_BATCH(1, 1);
-			else CURL_BATCH(1, 0);
-		}
-		else {
-			if (c.cm == 2) CURL_BATCH(0, 2);
-			else if (c.cm == 1) CURL_BATCH(0, 1);
-			else CURL_BATCH(0, 0);
-		}
-#undef CURL_PAIR
+#define CURL_BATCH(H, C) (c.pair ? launchEv(k_curl_batch<T, H, C, true>, grid, block, 0, B->st, s0, s1, args, start, c.n) : launchEv(k_curl_batch<T, H, C, false>, grid, block, 0, B->st, s0, s1, args, start, c.n))
+		if (h == 1) CURL_BATCH(1, 0);
+		else if (c.cm == 2) CURL_BATCH(0, 2);
+		else if (c.cm == 1) CURL_BATCH(0, 1);
+		else CURL_BATCH(0, 0);
 #undef CURL_BATCH
 		HIPCHECK(hipGetLastError());
 	}
@@ -3181,7 +3067,8 @@ int batchPost(alis_dev_batch *B, int h)
 			memset(&a[e], 0, sizeof(PostArgs<T>));
 			a[e].ops = (const PostOp<T> *)g.ops;
 			a[e].pieces = (const PostPiece *)g.pieces;
-			a[e].total = g.total;
+			a[e].total = g.total, a[e].post = (int)(g.total / POST_WG);
+			if (h == 1 && R.seg[e] + 1 == (int)D->post[h].size() && D->pendAde) a[e].ade = objArgs<T>(D), D->pendAde = false;
 			a[e].strips = D->pendStrips[h];
 			for (size_t w = 0; w < D->pendSrc[h].size(); w++) a[e].src[w] = D->pendSrc[h][w];
 			for (size_t q = 0; q < D->pendWave[h].size(); q++) a[e].wave[q] = (T)D->pendWave[h][q];
@@ -3194,6 +3081,7 @@ int batchPost(alis_dev_batch *B, int h)
 		HIPCHECK(hipGetLastError());
 	}
 	for (alis_dev_world *D : B->W) {
+		if (h == 1 && flushAde<T>(D)) return -1;     // a world without an H program
 		D->pendStrips[h] = 0;
 		std::fill(D->pendSrc[h].begin(), D->pendSrc[h].end(), 0u);
 	}
@@ -3263,8 +3151,8 @@ int alis_dev_link_tfsf(alis_dev_world *D, int s, alis_dev_world *aux)
 	if (flushE(D) || flushE(aux)) return -1;
 	D->tf[s].aux = aux;
 	D->postBuilt = D->postBuiltAlt = false;
-	D->fuseState = 0;
-	aux->isAux = true;
+	D->fuseState = 0, D->foldState = 0, D->stepArgs = nullptr;
+	aux->isAux = true, aux->mainOf = D;
 	// The auxiliary world keeps its own stream, so its half steps run beside the main
 	// world's curl launches; postHalf orders its strips against them with events.
 	return 0;
@@ -3273,7 +3161,11 @@ int alis_dev_link_tfsf(alis_dev_world *D, int s, alis_dev_world *aux)
 void alis_dev_release(alis_dev_world *D)
 {
 	if (!D) return;
+	if (D->pendMain || D->pendCore) (void)flushE(D);     // an auxiliary world's half step outlives its main world
 	if (D->st) hipStreamSynchronize(D->st);
+	for (DevTfsf &t : D->tf) if (t.aux && t.aux->mainOf == D) t.aux->mainOf = nullptr;
+	if (D->mainOf)
+		for (DevTfsf &t : D->mainOf->tf) if (t.aux == D) t.aux = nullptr, D->mainOf->foldState = 0;
 	for (void *p : D->allocs) hipFree(p);
 	for (int h = 0; h < 2; h++)
 		for (DevSrc &s : D->src[h]) {
@@ -3324,12 +3216,7 @@ int alis_dev_inject(alis_dev_world *D, int h, int index, float wave, const float
 int alis_dev_ghosts(alis_dev_world *D, int h)
 {
 	if (h < 0 || h > 1) return fail("no such half step");
-	if (h == 0 && D->pendE == 1) {      // deferred with its E core (see alis_dev_core)
-		D->pendE = 2;
-		return 0;
-	}
-	if (flushE(D)) return -1;
-	return D->fp64 ? postHalf<double>(D, h) : postHalf<float>(D, h);
+	return D->fp64 ? ghostsEntry<double>(D, h) : ghostsEntry<float>(D, h);
 }
 
 int alis_dev_sync(alis_dev_world *D, int i0, int i1, int j0, int j1, int k0, int k1)
@@ -4136,7 +4023,8 @@ int alis_dev_batch_create(alis_dev_world *const *D, int n, alis_dev_batch **out)
 		if (joinStream(D[w], D[0])) { delete B; return -1; }
 	}
 	B->st = D[0]->st;
-	int rc = B->fp64 ? batchBuildCurl<double>(B) : batchBuildCurl<float>(B);
+	int rc = B->fp64 ? batchBuildCurl<double>(B) || batchBuildObjects<double>(B) : batchBuildCurl<float>(B) || batchBuildObjects<float>(B);
+	if (rc) rc = -1;
 	if (rc) { alis_dev_batch_release(B); return rc; }
 	for (alis_dev_world *W : B->W) W->inBatch++;   // their arrays stay where the arguments name them
 	B->held = true;
@@ -4412,6 +4300,7 @@ double alis_dev_eps_bytes(const alis_dev_world *D)
 
 int alis_dev_timing(alis_dev_world *D, int enable)
 {
+	if (flushE(D)) return -1;
 	HIPCHECK(hipStreamSynchronize(D->st));
 	for (int h = 0; h < 3; h++) {
 		D->evFree.insert(D->evFree.end(), D->evPairs[h].begin(), D->evPairs[h].end());

@@ -4,7 +4,9 @@
         --steps 3 --warmup 1 --no-fp64 --cpu-steps 0 --copy-mib 256
     rocprofv3 --pmc WRITE_SIZE -d DIR_W -o run --output-format csv -- python3 bench.py \\
         --steps 3 --warmup 1 --no-fp64 --cpu-steps 0 --copy-mib 256
-    python3 alis_amd/profile_traffic.py DIR_F DIR_W 256 > profiles/k_curl_nanoblock256_traffic.json
+    python3 alis_amd/profile_traffic.py DIR_F DIR_W 256 16777216 > profiles/k_curl_nanoblock256_traffic.json
+
+The last two arguments are the copy's MiB and the world's cells.
 
 FETCH_SIZE and WRITE_SIZE (KiB per dispatch) are scaled by what they read for the
 device-to-device copy of known size that bench.py makes first (the largest copy dispatch).
@@ -20,13 +22,13 @@ ROOT = Path(__file__).resolve().parent.parent
 
 def kernels_sha256():
     """SHA-256 of the device kernels of the engine (the "Kernels" section of engine.hip and
-    the cell update it includes, alis_amd/csrc/curl_cell.inc): a traffic measurement stays
+    the files of kernels it includes, alis_amd/csrc/*.inc): a traffic measurement stays
     valid while these are unchanged."""
     src = (ROOT / "alis_amd/csrc/engine.hip").read_text()
     a = src.index("// Kernels\n")
     b = src.index("// Device world\n", a)
-    cell = (ROOT / "alis_amd/csrc/curl_cell.inc").read_text()
-    return hashlib.sha256((src[a:b] + cell).encode()).hexdigest()
+    inc = "".join(f.read_text() for f in sorted((ROOT / "alis_amd/csrc").glob("*.inc")))
+    return hashlib.sha256((src[a:b] + inc).encode()).hexdigest()
 
 
 def rows(d):
@@ -35,24 +37,25 @@ def rows(d):
 
 
 def main():
-    dF, dW, mib = sys.argv[1], sys.argv[2], int(sys.argv[3])
+    dF, dW, mib, cells = sys.argv[1], sys.argv[2], int(sys.argv[3]), int(sys.argv[4])
     F, W = rows(dF), rows(dW)
     nbytes = mib << 20
     cF = max(float(r["Counter_Value"]) for r in F if "copyBuffer" in r["Kernel_Name"])
     cW = max(float(r["Counter_Value"]) for r in W if "copyBuffer" in r["Kernel_Name"])
     fs, ws = nbytes / 1024 / cF, nbytes / 1024 / cW
-    cells = max(int(r["Grid_Size"]) for r in F if "k_curl" in r["Kernel_Name"])
     out = {"kernels_sha256": kernels_sha256(),
            "cells": cells, "fields": "fp32",
            "calibration": {"copy_bytes": nbytes, "FETCH_SIZE_kib": cF, "WRITE_SIZE_kib": cW,
                            "fetch_scale": round(fs, 5), "write_scale": round(ws, 5)}}
-    # k_curl<float, CM, ...>: CM 0 is the H launch (no 1/eps), 1 or 2 the E launch
-    # (the largest launches of each kind: the main world, not its TF/SF auxiliary world)
-    for name, pats in (("E", ("k_curl<float, 1", "k_curl<float, 2")), ("H", ("k_curl<float, 0",))):
-        big = max(int(r["Grid_Size"]) for r in F if any(p in r["Kernel_Name"] for p in pats))
+    # k_curl<float, HALF, ...> and k_curl_aux<float, HALF, ...>: HALF 0 is the E launch, 1 H
+    # (the largest launches of each kind: the main world, not an auxiliary world)
+    for name, half in (("E", "<float, 0,"), ("H", "<float, 1,")):
+        def curl(r):
+            return "k_curl" in r["Kernel_Name"] and half in r["Kernel_Name"]
+        big = max(int(r["Grid_Size"]) for r in F if curl(r))
 
         def mine(r):
-            return any(p in r["Kernel_Name"] for p in pats) and int(r["Grid_Size"]) == big
+            return curl(r) and int(r["Grid_Size"]) == big
         f = [float(r["Counter_Value"]) for r in F if mine(r)]
         w = [float(r["Counter_Value"]) for r in W if mine(r)]
         fa, wa = sum(f) / len(f), sum(w) / len(w)

@@ -100,11 +100,14 @@ void alis_dev_release(alis_dev_world *D);
  * (src/update.c:128-158).  Both real and imaginary parts of a Bloch world.
  * Fused steps (opt-in: the environment variable ALIS_FUSE=1 for worlds large enough to
  * fill the GPU, ALIS_FUSE=force for any world; never a TF/SF auxiliary world or a world in a
- * batch): the E core and its alis_dev_ghosts are deferred, and the H core runs both halves
- * in one pass over the grid (k_step) followed by the E half's end-of-step program and a
- * recomputation of H where that program changed E; the results are those of the separate
- * half steps, bit for bit.  Any other call on the world (or on a world that reads it) first
- * completes a deferred E half step the separate way. */
+ * batch): the E half step and the H core are deferred, and the H half's alis_dev_ghosts runs
+ * both halves in one pass over the grid (k_step, strips and sources included) followed by the
+ * ghost copies; the results are those of the separate half steps, bit for bit.
+ * A world with one TF/SF box whose auxiliary world is small defers the core of a half step, and
+ * the auxiliary world its whole half step, to its own alis_dev_ghosts, which runs both in the
+ * same launches.
+ * Any other call on the world (or on a world that reads it) first completes what is deferred
+ * the separate way. */
 int alis_dev_core(alis_dev_world *D, int h);
 
 /* Face-strip corrections of the s-th TF/SF box from its auxiliary world

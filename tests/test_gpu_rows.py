@@ -1,0 +1,75 @@
+"""Rows of every length through the curl kernels' quads (16 bytes of a row per lane): the CPU oracle's
+fields, FP32 bit for bit and FP64 to 1e-12 of the largest value (the bound the parity scenarios
+have), over row lengths that leave every remainder of a quad.  The nanoblock steps its TF/SF box's auxiliary world inside the main
+world's launches and its objects in launches of their own; a read between two calls of a half step
+makes the waiting launches run apart.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+from scenarios import ROOT
+
+pytestmark = pytest.mark.gpu
+
+LIBS = {"hip": ROOT / "alis_amd" / "libalis_workloads.so", "oracle": ROOT / "oracle" / "libwl_oracle.so"}
+ENGINES = {"hip": ROOT / "alis_amd" / "libalis.so", "oracle": ROOT / "oracle" / "liboracle.so"}
+
+
+def _fields(kind, name, cells, bits, steps, parted=False):
+    w, e = ctypes.CDLL(str(LIBS[kind])), ctypes.CDLL(str(ENGINES[kind]))
+    w.wl_create.restype = w.wl_device.restype = ctypes.c_void_p
+    w.wl_create.argtypes = [ctypes.c_char_p] + [ctypes.c_int] * 3
+    w.wl_step.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    w.wl_device.argtypes = w.wl_free.argtypes = [ctypes.c_void_p]
+    w.wl_field.restype = ctypes.c_long
+    w.wl_field.argtypes = [ctypes.c_void_p] + [ctypes.c_int] * 4 + [ctypes.POINTER(ctypes.c_double), ctypes.c_long]
+    for f in (e.alis_dev_core, e.alis_dev_ghosts):
+        f.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    c = w.wl_create(name.encode(), cells, bits, 64)
+    w.wl_step(c, steps)
+    per = (cells + 4) ** 3
+    buf = (ctypes.c_double * per)()
+    out = []
+
+    def read(h):
+        for a in range(3):
+            n = w.wl_field(c, 0, h, 0, a, buf, per)
+            assert n > 0
+            out.append(np.frombuffer(buf, dtype=np.float64, count=n).copy())
+    if parted:
+        dev = w.wl_device(c)
+        for h in range(2):
+            assert e.alis_dev_core(dev, h) == 0
+            read(h)
+            assert e.alis_dev_ghosts(dev, h) == 0
+        w.wl_step(c, 2)
+    read(0), read(1)
+    w.wl_free(c)
+    return np.concatenate(out)
+
+
+def _agree(name, cells, bits, steps, parted=False):
+    print(f"[gpu] {name} {cells}^3 fp{bits}", flush=True)
+    got, ref = _fields("hip", name, cells, bits, steps, parted), _fields("oracle", name, cells, bits, steps, parted)
+    assert got.shape == ref.shape and np.abs(ref).max() > 0
+    if bits == 32:
+        assert np.array_equal(got, ref)
+    else:
+        assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("cells,bits", [(58, 32), (59, 32), (60, 32), (61, 32), (62, 32), (60, 64), (61, 64)])
+def test_dipole_rows(cells, bits):
+    _agree("dipole", cells, bits, 30)
+
+
+@pytest.mark.parametrize("cells,bits", [(108, 32), (109, 32), (110, 32), (111, 32), (109, 64), (110, 64)])
+def test_scatterer_rows(cells, bits):
+    _agree("nanoblock", cells, bits, 12)
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+def test_half_step_in_parts(bits):
+    _agree("nanoblock", 109, bits, 8, parted=True)
