@@ -675,11 +675,17 @@ __global__ __launch_bounds__(256) void k_fill(T *p, long n, T v)
 
 // Probe spectra (the running DFT of writeSpectrum, src/output.c:177-230) in FP64 with
 // compensated (Neumaier) summation.  acc holds, per probe p and frequency bin b, the running
-// sum (re, im) at acc[2 (p nb + b)] and its compensation at acc[2 (p nb + b) + 1]; a thread
-// takes one bin and up to SPEC_PPT probes and adds ns staged samples (tau, v[0..np-1]) in
-// sample order, each with the factor e^{i 2 pi tau (nTop - b)} (one sincos per sample and
-// bin, shared by the thread's probes).
-constexpr int SPEC_PPT = 8;
+// sum (re, im) at acc[2 (p nb + b)] and its compensation at acc[2 (p nb + b) + 1]; ns staged
+// samples (tau, v[0..np-1]) are added in sample order, each with the factor
+// e^{i 2 pi tau (nTop - b)}.
+//
+// What bounds it: latency; a launch has a few hundred sums, each a chain over the samples.  The
+// factors are no part of that chain, so a workgroup (SPEC_BINS bins, up to SPEC_PROBES probes)
+// first computes those of all samples side by side into LDS, one sincos each, and then runs the
+// chains, one real or imaginary sum per thread: additions and LDS reads alone.  256 samples of 8
+// probes and 256 bins: 387 us with the sincos inside the chain (one thread per bin) -> 13 us.
+constexpr int SPEC_RING = 256;      // samples staged per launch
+constexpr int SPEC_BINS = 4, SPEC_PROBES = 16;
 
 __device__ inline void neumaier(double &s, double &c, double x)
 {
@@ -688,34 +694,28 @@ __device__ inline void neumaier(double &s, double &c, double x)
 	s = t;
 }
 
+// LDS: the factors [sample][bin] (cos, sin), then the samples [sample][probe].  Grid: bins, probes.
 __global__ __launch_bounds__(256) void k_spectrum_add(double2 *__restrict__ acc, int np, int nb, int nTop,
                                                       const double *__restrict__ samp, int ns)
 {
-	const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-	const int b = t % nb, p0 = t / nb * SPEC_PPT;
-	if (p0 >= np) return;
-	const int pn = min(SPEC_PPT, np - p0);
-	double2 sum[SPEC_PPT], cmp[SPEC_PPT];
-#pragma unroll
-	for (int u = 0; u < SPEC_PPT; u++)
-		if (u < pn) sum[u] = acc[2 * ((long)(p0 + u) * nb + b)], cmp[u] = acc[2 * ((long)(p0 + u) * nb + b) + 1];
+	extern __shared__ __align__(16) double specLds[];
+	const int b0 = (int)blockIdx.x * SPEC_BINS, p0 = (int)blockIdx.y * SPEC_PROBES, pn = min(SPEC_PROBES, np - p0);
+	double *const f = specLds, *const v = specLds + 2 * SPEC_BINS * ns;
 	const double w = 2 * M_PI;
-	const int harmonic = nTop - b;
-	for (int q = 0; q < ns; q++) {
-		const double *r = samp + (long)q * (1 + np);
-		double sn, cs;
-		sincos(w * r[0] * harmonic, &sn, &cs);
-#pragma unroll
-		for (int u = 0; u < SPEC_PPT; u++)
-			if (u < pn) {
-				const double v = r[1 + p0 + u];
-				neumaier(sum[u].x, cmp[u].x, v * cs);
-				neumaier(sum[u].y, cmp[u].y, v * sn);
-			}
+	for (int t = (int)threadIdx.x; t < ns * SPEC_BINS; t += 256) {
+		const int q = t / SPEC_BINS, harmonic = nTop - (b0 + t % SPEC_BINS);
+		sincos(w * samp[(long)q * (1 + np)] * harmonic, &f[2 * t + 1], &f[2 * t]);
 	}
-#pragma unroll
-	for (int u = 0; u < SPEC_PPT; u++)
-		if (u < pn) acc[2 * ((long)(p0 + u) * nb + b)] = sum[u], acc[2 * ((long)(p0 + u) * nb + b) + 1] = cmp[u];
+	for (int t = (int)threadIdx.x; t < ns * pn; t += 256) v[t] = samp[(long)(t / pn) * (1 + np) + 1 + p0 + t % pn];
+	__syncthreads();
+	// thread: (real, imaginary) of bin of probe
+	const int c = (int)threadIdx.x % (2 * SPEC_BINS), p = (int)threadIdx.x / (2 * SPEC_BINS), b = b0 + c / 2;
+	if (p >= pn || b >= nb) return;
+	double *const a = (double *)(acc + 2 * ((long)(p0 + p) * nb + b)) + c % 2;
+	double sum = a[0], cmp = a[2];
+#pragma unroll 8
+	for (int q = 0; q < ns; q++) neumaier(sum, cmp, v[q * pn + p] * f[q * 2 * SPEC_BINS + c]);
+	a[0] = sum, a[2] = cmp;
 }
 
 // Per-row sums over a plane of a world's fields for the instantaneous Poynting flux
@@ -4152,8 +4152,6 @@ int alis_dev_absorption(alis_dev_world *D, int n, int i0, int i1, int j0, int j1
 
 // ---- probe spectra ----
 
-constexpr int SPEC_RING = 256;  // samples staged per k_spectrum_add launch
-
 struct alis_dev_spectrum {
 	int np = 0, nb = 0, nTop = 0;
 	double2 *acc = nullptr;     // [probe][bin] (sum, compensation)
@@ -4174,8 +4172,9 @@ int spectrumFlush(alis_dev_spectrum *S)
 	if (!S->pend) return 0;
 	const int c = S->cur;
 	HIPCHECK(hipMemcpyAsync(S->stage[c], S->pinned[c], (size_t)S->pend * (1 + S->np) * sizeof(double), hipMemcpyHostToDevice, g_specStream));
-	const long threads = (long)S->nb * ((S->np + SPEC_PPT - 1) / SPEC_PPT);
-	k_spectrum_add<<<blocksFor(threads), 256, 0, g_specStream>>>(S->acc, S->np, S->nb, S->nTop, S->stage[c], S->pend);
+	const dim3 grid((S->nb + SPEC_BINS - 1) / SPEC_BINS, (S->np + SPEC_PROBES - 1) / SPEC_PROBES);
+	const size_t lds = (size_t)S->pend * (2 * SPEC_BINS + std::min(S->np, SPEC_PROBES)) * sizeof(double);   // 48 KiB at most
+	k_spectrum_add<<<grid, 256, lds, g_specStream>>>(S->acc, S->np, S->nb, S->nTop, S->stage[c], S->pend);
 	HIPCHECK(hipGetLastError());
 	HIPCHECK(hipEventRecord(S->done[c], g_specStream));
 	S->cur ^= 1, S->pend = 0;
