@@ -22,6 +22,7 @@
 #include <cstdint>
 #include <cmath>
 #include <algorithm>
+#include <functional>
 #include <map>
 #include <mutex>
 
@@ -113,6 +114,10 @@ template<class T> __device__ inline __attribute__((address_space(1))) T *glb(T *
 	return (__attribute__((address_space(1))) T *)p;
 }
 
+// A value that the whole wavefront reads from a table no kernel of the launch writes: through the
+// scalar cache.
+template<class P> __device__ __forceinline__ const __attribute__((address_space(4))) P *uniform(const P *p) { return (const __attribute__((address_space(4))) P *)p; }
+
 #include "curl_quads.inc"
 #include "objects.inc"
 
@@ -184,22 +189,23 @@ template<class T> struct PostOp {
 constexpr int MAXSRC = 128;     // sources per chain (E or H) of one world
 constexpr int MAXCHAIN = 24;    // copies per launch
 constexpr int MAXPOST = 48;     // operations per launch
-constexpr int POST_WG = 64;     // threads (cells) per workgroup of k_post: one wavefront (64 k-point
-                                // worlds: H program 84 -> 79 us, E 35 -> 31 us against 256)
+constexpr int POST_WG = 64;     // threads per workgroup of k_post: one wavefront (64 k-point worlds:
+                                // H program 84 -> 79 us, E 35 -> 31 us against 256)
+constexpr int POST_U = 4, POST_BLK = POST_WG * POST_U;   // cells per thread, per workgroup
 
 struct PostPiece {
 	int kind;                   // OP_COPY, or OP_STRIP for an additive piece
 	int n;                      // operations in list
 	int si, sj, sk;             // copy piece: base cell - cell
 	Box b;                      // the cells
-	long off;                   // first thread in the launch (a multiple of POST_WG)
+	long off;                   // first cell in the launch (a multiple of POST_BLK)
+	unsigned rk, rj;            // 2^32 over the cells along k, along j (recip32)
 	unsigned char list[MAXPOST];// operation indices (copy piece: its chain, last copy first)
 };
 
 template<class T> struct PostArgs {
 	const PostOp<T> *ops;
 	const PostPiece *pieces;    // per workgroup of the launch: the piece it runs
-	long total;
 	int post;                   // workgroups of the program; those after them run `ade`
 	ObjArgs<T> ade;
 	unsigned strips;            // TF/SF boxes whose strips apply this half step (bit s)
@@ -207,7 +213,7 @@ template<class T> struct PostArgs {
 	T wave[MAXSRC];             // their scalar wave values
 };
 
-template<class T> __device__ inline bool opOn(const PostArgs<T> &a, const PostOp<T> &o)
+template<class A, class O> __device__ inline bool opOn(const A &a, const O &o)
 {
 	if (o.kind == OP_STRIP) return (a.strips >> o.slot) & 1u;
 	if (o.kind == OP_SOURCE) return (a.src[o.slot >> 5] >> (o.slot & 31)) & 1u;
@@ -230,62 +236,95 @@ template<class T, class O> __device__ inline T addTo(O &o, T f, int i, int j, in
 	return f + amp * w;
 }
 
+// t / d for t < 2^31 by r = recip32(d): its rounded-up reciprocal is at most one too large a
+// quotient.
+__host__ __device__ inline unsigned recip32(int d) { return d == 1 ? 0xffffffffu : (unsigned)(((1ull << 32) + d - 1) / d); }
+__device__ __forceinline__ int divBy(int t, int d, unsigned r)
+{
+	int q = (int)__umulhi((unsigned)t, r);
+	if (q * d > t) q--;
+	return d == 1 ? t : q;
+}
+
 // One workgroup (number blk within its launch) of k_post.  Pieces start on workgroup
 // boundaries, so the piece and its operations are the same for the whole workgroup; the
 // launch's table holds each workgroup's piece, so a workgroup reaches its cell through three
 // dependent loads (piece, operation, cell) where a search of the pieces added about seven
 // (measured with 256-thread workgroups: 64 k-point worlds' H program 95 -> 84 us; 256^3
-// nanoblock H program 17.5 -> 16.1 us).
+// nanoblock H program 17.5 -> 16.1 us).  That chain is what bounds it: piece and operation come
+// through the scalar cache, and a thread takes POST_U cells, whose loads are in flight together
+// (256^3 H program with its current update 23 -> 18 us, 64 spheres 42 -> 36, 6 worlds 32 -> 27).
 // (tid: the thread's place in the workgroup.)
-template<class T>
-__device__ __forceinline__ void postCells(const PostArgs<T> &a, const PostOp<T> *ops, const PostPiece *pieces, int blk, int tid)
+template<class T, class A>
+__device__ __forceinline__ void postCells(const A &a, const PostOp<T> *allOps, const PostPiece *pieces, int blk, int tid)
 {
-	const PostPiece &P = pieces[blk];
-	const int ni = P.b.i1 - P.b.i0 + 1, nj = P.b.j1 - P.b.j0 + 1, nk = P.b.k1 - P.b.k0 + 1;
-	const int t = blk * POST_WG + tid - (int)P.off;
-	if (t >= ni * nj * nk) return;
-	const int dk = t % nk, r = t / nk, dj = r % nj, di = r / nj;
-	const int i = P.b.i0 + di, j = P.b.j0 + dj, k = P.b.k0 + dk;
-	const PostOp<T> &o = ops[P.list[0]];
-	const long d = o.LF.at(i, j, k);
+	const auto &P = uniform(pieces)[blk];
+	const auto *const ops = uniform(allOps);
+	const int nk = P.b.k1 - P.b.k0 + 1, nj = P.b.j1 - P.b.j0 + 1, count = (P.b.i1 - P.b.i0 + 1) * nj * nk;
+	const int t0 = blk * POST_BLK + tid - (int)P.off;
+	const auto &o = ops[P.list[0]];
+	T *const F = o.F, *const G = o.G;
+	int i[POST_U], j[POST_U], k[POST_U];
+	long d[POST_U];
+	T f[POST_U], g[POST_U];
+#pragma unroll
+	for (int u = 0; u < POST_U; u++) {
+		// cells beyond the piece repeat its last one's loads and store nothing
+		const int t = min(t0 + u * POST_WG, count - 1), r = divBy(t, nk, P.rk), di = divBy(r, nj, P.rj);
+		i[u] = P.b.i0 + di, j[u] = P.b.j0 + r - di * nj, k[u] = P.b.k0 + t - r * nk;
+		d[u] = layAt(o.LF, i[u], j[u], k[u]);
+	}
 	if (P.kind == OP_COPY) {
-		const long s = o.LF.at(i + P.si, j + P.sj, k + P.sk);
-		T f = o.F[s], g = o.G ? o.G[s] : T(0);
-		for (int u = P.n - 1; u >= 0; u--) {
-			const PostOp<T> &r = ops[P.list[u]];
-			if (o.G) {
-				const T fs = f, gs = g;
-				f = r.c * fs + r.s * gs;
-				g = r.c * gs - r.s * fs;
+		const long off = layAt(o.LF, P.si, P.sj, P.sk) - layAt(o.LF, 0, 0, 0);
+#pragma unroll
+		for (int u = 0; u < POST_U; u++) f[u] = glb(F)[d[u] + off], g[u] = G ? glb(G)[d[u] + off] : T(0);
+		for (int x = P.n - 1; x >= 0; x--) {
+			const auto &r = ops[P.list[x]];
+			const T c = r.c, s = r.s;
+#pragma unroll
+			for (int u = 0; u < POST_U; u++) {
+				const T fs = f[u], gs = g[u];
+				f[u] = G ? c * fs + s * gs : c * fs;
+				g[u] = c * gs - s * fs;
 			}
-			else f = r.c * f;
 		}
-		o.F[d] = f;
-		if (o.G) o.G[d] = g;
+#pragma unroll
+		for (int u = 0; u < POST_U; u++)
+			if (t0 + u * POST_WG < count) {
+				glb(F)[d[u]] = f[u];
+				if (G) glb(G)[d[u]] = g[u];
+			}
 		return;
 	}
 	bool on = false;
-	T f = T(0);
-	for (int u = 0; u < P.n; u++) {
-		const PostOp<T> &r = ops[P.list[u]];
+	for (int x = 0; x < P.n; x++) {
+		const auto &r = ops[P.list[x]];
 		if (!opOn(a, r)) continue;
-		if (!on) f = o.F[d], on = true;
-		f = addTo(r, f, i, j, k, r.kind == OP_SOURCE ? a.wave[r.slot] : T(0));
+		if (!on)
+#pragma unroll
+			for (int u = 0; u < POST_U; u++) f[u] = glb(F)[d[u]];
+		on = true;
+		const T wave = r.kind == OP_SOURCE ? a.wave[r.slot] : T(0);
+#pragma unroll
+		for (int u = 0; u < POST_U; u++) f[u] = addTo<T>(r, f[u], i[u], j[u], k[u], wave);
 	}
-	if (on) o.F[d] = f;
+	if (!on) return;
+#pragma unroll
+	for (int u = 0; u < POST_U; u++)
+		if (t0 + u * POST_WG < count) glb(F)[d[u]] = f[u];
 }
 
-template<class T>
-__device__ __forceinline__ void postBlock(const PostArgs<T> &a, int blk)
+template<class T, class A>
+__device__ __forceinline__ void postBlock(const A &a, int blk)
 {
-	if (blk < a.post) postCells(a, a.ops, a.pieces, blk, (int)threadIdx.x);
-	else if (a.ade.blocks) adeBlock(a.ade, blk - a.post);
+	if (blk < a.post) postCells<T>(a, a.ops, a.pieces, blk, (int)threadIdx.x);
+	else if (a.ade.blocks) adeBlock<T>(a.ade, blk - a.post);
 }
 
 template<class T>
 __global__ __launch_bounds__(POST_WG) void k_post(PostArgs<T> a)
 {
-	postBlock(a, (int)blockIdx.x);
+	postBlock<T>(a, (int)blockIdx.x);
 }
 
 // Several worlds' programs in one launch: entry e owns workgroups [start[e], start[e+1]).
@@ -294,7 +333,7 @@ __global__ __launch_bounds__(POST_WG) void k_post_batch(const PostArgs<T> *__res
 {
 	const int b = (int)blockIdx.x;
 	const int e = batchEntry(start, n, b);
-	postBlock(args[e], b - start[e]);
+	postBlock<T>(uniform(args)[e], b - uniform(start)[e]);
 }
 
 #include "step_kernel.inc"
@@ -901,10 +940,13 @@ struct DevSrc {
 
 struct PostSeg {
 	void *ops = nullptr;        // PostOp<T>[] in device memory
-	void *pieces = nullptr;     // PostPiece[total / POST_WG] in device memory: each workgroup's
+	void *pieces = nullptr;     // PostPiece[total / POST_BLK] in device memory: each workgroup's
 	                            //  piece
-	long total = 0;             // threads (a multiple of POST_WG)
+	long total = 0;             // cells (a multiple of POST_BLK)
+	long rest = 0;              // those of them before the copies that the curl can make (see rowCopyOf)
 };
+
+struct alis_dev_batch;
 
 struct DevTfsf {
 	alis_dev_tfsf S{};
@@ -998,7 +1040,13 @@ struct alis_dev_world {
 	// A small auxiliary world's half step in the main world's launches (k_curl_aux): main world:
 	// 1 + h while its core of half step h waits for its ghosts; auxiliary world: its core and its
 	// ghosts of half step h wait for them too.
+	// (A world without one also waits: the curl then makes some of the ghost copies.)
 	int pendMain = 0, pendCore = 0, pendGhosts = 0;
+	bool pendFold = false;      // main world waiting: with its auxiliary world
+	alis_dev_batch *pendBatch = nullptr;  // the batch whose core of a half step waits
+	struct RowCopyBox { Box b; double c, s; };
+	RowCopyBox rowCopy[2][2] = {};        // [h][end] (RowCopy)
+	int rowEnds[2] = {0, 0};
 	int foldState = 0;          // main world: 0 not decided yet, 1 its auxiliary world can, -1 cannot
 	int pendH = 0;              // auxiliary world: its H core (1) and ghosts (2) wait for the
 	                            //  main world's deferred step, which reads the old H
@@ -1329,7 +1377,8 @@ void buildPieces(const std::vector<PostOp<T>> &v, int nadd, std::vector<PostPiec
 					for (int u = 0; u < P.n; u++) P.list[u] = (unsigned char)K[4 + u];
 					P.b = Box{b.i0 + di, b.i0 + di1, b.j0 + dj, b.j0 + dj1, b.k0 + dk, b.k0 + dk1};
 					P.off = total;
-					total += (P.b.count() + POST_WG - 1) / POST_WG * POST_WG;
+					P.rk = recip32(P.b.k1 - P.b.k0 + 1), P.rj = recip32(P.b.j1 - P.b.j0 + 1);
+					total += (P.b.count() + POST_BLK - 1) / POST_BLK * POST_BLK;
 					out.push_back(P);
 				}
 	}
@@ -1613,6 +1662,14 @@ HalfArgs<T> halfArgs(alis_dev_world *D, int h, int m)
 	a.pq = (int)(D->L.sj / N);
 	a.tiles = (a.nj * a.pq + CURL_WG - 1) / CURL_WG;
 	a.inv = a.pq == 1 ? 0xffffffffu : (unsigned)(((1ull << 32) + a.pq - 1) / a.pq);
+	if (D->postBuilt) {
+		a.ends = D->rowEnds[h];
+		for (int end = 0; end < 2; end++) {
+			const alis_dev_world::RowCopyBox &x = D->rowCopy[h][end];
+			a.copy[end] = RowCopy<T>{x.b.i0, x.b.i1, x.b.j0, x.b.j1, (T)x.c, (T)x.s};
+		}
+		for (int slot = 0; m == 1 && slot < 2; slot++) a.P[slot] = (T *)D->F[h][0][(h ? 0 : 2) + (h ? slot : 0)];
+	}
 	for (int ax = 0; ax < 3; ax++) {
 		SlabPair<T> &P = a.slab[ax];
 		for (int side = 0; side < 2; side++) {
@@ -1739,9 +1796,10 @@ int zSamples(alis_dev_world *D, PhsZ<T> *zs, std::vector<DevPhaser *> &owners, b
 	return n;
 }
 
+// copies: the launch makes the ghost copies along z that it can; the program without them follows.
 // x: an auxiliary world's share of the launch, or null.
 template<class T>
-int coreHalf(alis_dev_world *D, int h, const AuxCurl<T> *x = nullptr)
+int coreHalf(alis_dev_world *D, int h, bool copies = false, const AuxCurl<T> *x = nullptr)
 {
 	dropPresamples(D);
 	hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1753,6 +1811,7 @@ int coreHalf(alis_dev_world *D, int h, const AuxCurl<T> *x = nullptr)
 	std::vector<DevPhaser *> sampled;
 	for (int m = 0; m <= D->cplx; m++) {
 		HalfArgs<T> a = halfArgs<T>(D, h, m);
+		if (!copies || m < D->cplx) a.ends = 0;
 		ZFaces<T> z{};
 		const bool aux = x && m == 0;
 		const dim3 grid(a.tiles, a.ni + (aux ? 1 : 0)), block(CURL_WG);
@@ -1897,17 +1956,74 @@ std::vector<Box> outsideParts(Box b, const Box &r)
 	return out;
 }
 
+// Whether the curl can make a copy piece as it stores the source's quad, and the end and component it
+// belongs to (see rowCopyOf).
+typedef std::function<bool(const PostPiece &, int &end, int &slot)> RowCopyWish;
+
 // Upload one launch's program (nadd additive operations, then copies) compiled into pieces.
 template<class T>
-int postSegment(alis_dev_world *D, const std::vector<PostOp<T>> &v, int nadd, std::vector<PostPiece> &pieces, PostSeg &seg)
+int postSegment(alis_dev_world *D, const std::vector<PostOp<T>> &v, int nadd, std::vector<PostPiece> &pieces, PostSeg &seg,
+                int h = 0, const RowCopyWish &wish = nullptr)
 {
 	pieces.clear();
 	buildPieces(v, nadd, pieces, seg.total);
 	if (pieces.empty()) return 0;
+	seg.rest = seg.total;
+	if (wish) {
+		// The copies that the curl can make come last: an end's over the rows that all its
+		// components' pieces have in common, within those that the curl updates.
+		auto part = [](PostPiece P, const Box &b) {
+			P.b = b, P.rk = recip32(b.k1 - b.k0 + 1), P.rj = recip32(b.j1 - b.j0 + 1);
+			return P;
+		};
+		auto common = [](Box b, const Box &x) {
+			b.i0 = std::max(b.i0, x.i0), b.i1 = std::min(b.i1, x.i1), b.j0 = std::max(b.j0, x.j0), b.j1 = std::min(b.j1, x.j1);
+			return b;
+		};
+		const Box rows{D->iMIN, D->iMAX, D->jMIN, D->jMAX, 0, 0};
+		int of[2][2] = {{-1, -1}, {-1, -1}};             // [end][slot]: the largest piece
+		for (int n = 0; n < (int)pieces.size(); n++) {
+			const Box b = common(pieces[n].b, rows);
+			int end, slot;
+			if (!b.count() || !wish(part(pieces[n], b), end, slot)) continue;
+			if (of[end][slot] < 0 || pieces[of[end][slot]].b.count() < pieces[n].b.count()) of[end][slot] = n;
+		}
+		std::vector<int> taken(pieces.size(), -1);       // the end whose rows it gives away
+		for (int end = 0; end < 2; end++) {
+			if (of[end][0] < 0 || (h == 1 && of[end][1] < 0)) continue;
+			Box b = common(pieces[of[end][0]].b, rows);
+			if (h == 1) b = common(b, pieces[of[end][1]].b);
+			const PostOp<T> &o = v[pieces[of[end][0]].list[0]], &o1 = v[pieces[of[end][h == 1 ? 1 : 0]].list[0]];
+			if (!b.count() || o.c != o1.c || o.s != o1.s) continue;
+			D->rowCopy[h][end] = {b, (double)o.c, (double)o.s};
+			D->rowEnds[h] |= 1 << end;
+			for (int slot = 0; slot < (h == 1 ? 2 : 1); slot++) taken[of[end][slot]] = end;
+		}
+		std::vector<PostPiece> front, back;
+		for (size_t n = 0; n < pieces.size(); n++) {
+			const PostPiece &P = pieces[n];
+			if (taken[n] < 0) {
+				front.push_back(P);
+				continue;
+			}
+			Box b = D->rowCopy[h][taken[n]].b;
+			b.k0 = P.b.k0, b.k1 = P.b.k1;
+			back.push_back(part(P, b));
+			for (const Box &x : outsideParts(P.b, b)) front.push_back(part(P, x));
+		}
+		long off = 0;
+		auto place = [&](PostPiece &P) { P.off = off, off += (P.b.count() + POST_BLK - 1) / POST_BLK * POST_BLK; };
+		for (PostPiece &P : front) place(P);
+		seg.rest = off;
+		for (PostPiece &P : back) place(P);
+		seg.total = off;
+		pieces = front;
+		pieces.insert(pieces.end(), back.begin(), back.end());
+	}
 	if (seg.total >= (1L << 31)) return fail("end-of-half-step launch over 2^31 threads");
-	std::vector<PostPiece> perBlock(seg.total / POST_WG);
+	std::vector<PostPiece> perBlock(seg.total / POST_BLK);
 	for (const PostPiece &P : pieces)
-		for (long b = P.off / POST_WG; b < (P.off + P.b.count() + POST_WG - 1) / POST_WG; b++) perBlock[b] = P;
+		for (long b = P.off / POST_BLK; b < (P.off + P.b.count() + POST_BLK - 1) / POST_BLK; b++) perBlock[b] = P;
 	if (devAlloc(D, &seg.ops, v.size() * sizeof(PostOp<T>))) return -1;
 	if (devAlloc(D, &seg.pieces, perBlock.size() * sizeof(PostPiece))) return -1;
 	HIPCHECK(hipMemcpyAsync(seg.ops, v.data(), v.size() * sizeof(PostOp<T>), hipMemcpyHostToDevice, D->st));
@@ -1960,6 +2076,36 @@ std::vector<PostOp<T>> copyOps(const alis_dev_world *D, int h)
 	}
 	dropEmpty(copies);
 	return copies;
+}
+
+struct BasePiece { const void *F; PostPiece P; };
+
+// Whether the curl can make copy piece P of program v as it stores the source's quad (RowCopy): one
+// copy between neighbours along z at a row's end (a world that is not periodic along z), over rows
+// in which nothing else touches its two cells: no strip or source, no other copy, no copy of an
+// earlier launch that reads the target before.  end and slot: where it belongs in HalfArgs.
+template<class T>
+bool rowCopyOf(alis_dev_world *D, int h, const std::vector<PostOp<T>> &v, const PostPiece &P, const std::vector<PostOp<T>> &adds,
+               const std::vector<PostOp<T>> &copies, const std::vector<BasePiece> &earlier, int &end, int &slot)
+{
+	if (P.kind != OP_COPY || P.n != 1 || P.si || P.sj || P.b.k0 != P.b.k1 || D->kNUM < 3) return false;
+	const int to = P.b.k0, from = to + P.sk;
+	end = to == D->kMAX + 1 && from == D->kMAX ? 1 : h == 1 && to == D->kMIN && from == to + 1 ? 0 : -1;
+	if (end < 0 || P.b.i0 < D->iMIN || P.b.i1 > D->iMAX || P.b.j0 < D->jMIN || P.b.j1 > D->jMAX) return false;
+	const PostOp<T> &o = v[P.list[0]];
+	slot = -1;
+	for (int a = 0; a < 2; a++) if (o.F == (T *)D->F[h][0][h ? a : 2] && (h || a == 0)) slot = a;
+	if (slot < 0 || ((D->rowEnds[h] >> end) & 1)) return false;
+	Box cells = P.b;
+	cells.k0 = std::min(to, from), cells.k1 = std::max(to, from);
+	for (const PostOp<T> &x : adds) if ((x.F == o.F || x.F == o.G) && boxesMeet(x.b, cells)) return false;
+	for (const PostOp<T> &x : copies)
+		if (x.F == o.F && boxesMeet(x.b, cells) && !(x.di == o.di && x.dj == o.dj && x.dk == o.dk && !memcmp(&x.b, &o.b, sizeof(Box)))) return false;
+	for (const BasePiece &x : earlier) {
+		const Box base{x.P.b.i0 + x.P.si, x.P.b.i1 + x.P.si, x.P.b.j0 + x.P.sj, x.P.b.j1 + x.P.sj, x.P.b.k0 + x.P.sk, x.P.b.k1 + x.P.sk};
+		if (x.F == o.F && boxesMeet(base, P.b)) return false;
+	}
+	return true;
 }
 
 // Build the end-of-half-step programs of D: strips of every TF/SF box, sources of the
@@ -2049,12 +2195,17 @@ int buildPost(alis_dev_world *D)
 		}
 		D->post[h].clear();
 		D->carry[h].clear();
+		D->rowEnds[h] = 0;
+		std::vector<BasePiece> earlier;   // copies of the launches before
 		for (size_t g = 0; g < segOps.size(); g++) {
 			const std::vector<PostOp<T>> &v = segOps[g];
 			std::vector<PostPiece> pieces;
 			PostSeg seg;
-			if (postSegment(D, v, segAdd[g], pieces, seg)) return -1;
+			const RowCopyWish wish = [&](const PostPiece &P, int &end, int &slot) { return rowCopyOf(D, h, v, P, adds, copies, earlier, end, slot); };
+			if (postSegment<T>(D, v, segAdd[g], pieces, seg, h, wish)) return -1;
 			if (pieces.empty()) continue;
+			for (const PostPiece &P : pieces)
+				if (P.kind == OP_COPY) earlier.push_back({v[P.list[0]].F, P});
 			// A copy chain starts from a cell no earlier copy of its launch writes.  Where that
 			// cell lies outside the update range and a copy of the program writes it (later:
 			// the program reads the value the previous step left there), a fused step's new
@@ -2111,6 +2262,7 @@ int waitForAux(alis_dev_world *D, unsigned strips)
 	for (size_t s = 0; s < D->tf.size(); s++) {
 		alis_dev_world *X = D->tf[s].aux;
 		if (!((strips >> s) & 1u)) continue;
+		if (X->pendMain && flushE(X)) return -1;
 		if (X->st == D->st) continue;
 		if (!X->halfDone) {
 			HIPCHECK(hipEventCreateWithFlags(&X->halfDone, hipEventDisableTiming));
@@ -2127,7 +2279,7 @@ int flushAde(alis_dev_world *D)
 {
 	if (!D->pendAde) return 0;
 	D->pendAde = false;
-	k_ade<T><<<objBlocks(D), POST_WG, 0, D->st>>>(objArgs<T>(D));
+	k_ade<T><<<objBlocks(D), OBJ_WG, 0, D->st>>>(objArgs<T>(D));
 	HIPCHECK(hipGetLastError());
 	return 0;
 }
@@ -2161,7 +2313,7 @@ int foldsAux(alis_dev_world *D, bool &on)
 		for (int h = 0; h < 2; h++) {
 			if (A->post[h].empty() || A->post[h].size() > (size_t)AUX_SEGS + 1) return 0;
 			for (size_t g = 0; g + 1 < A->post[h].size(); g++)
-				if (A->post[h][g].total > AUX_UNITS * (long)POST_WG) return 0;
+				if (A->post[h][g].total > AUX_CELLS) return 0;
 		}
 		if (joinStream(A, D)) return -1;
 		D->foldState = 1;
@@ -2171,7 +2323,7 @@ int foldsAux(alis_dev_world *D, bool &on)
 }
 
 template<class T>
-int postHalf(alis_dev_world *D, int h, const PostArgs<T> *x = nullptr);
+int postHalf(alis_dev_world *D, int h, bool copied = false, const PostArgs<T> *x = nullptr);
 
 // A half step of D and of its auxiliary world, both waiting: two launches (three with objects, or a
 // main program of several).
@@ -2180,30 +2332,36 @@ int foldedHalf(alis_dev_world *D, int h)
 {
 	alis_dev_world *A = D->tf[0].aux;
 	D->pendMain = A->pendCore = A->pendGhosts = 0;
+	D->pendFold = false;
 	dropPresamples(A);
 	if (!A->postBuilt && buildPost<T>(A)) return -1;
 	AuxCurl<T> x{};
 	static_assert(sizeof(HalfArgs<T>) + sizeof x + sizeof(ZFaces<T>) <= 4096 && 2 * sizeof(PostArgs<T>) <= 4096, "kernel arguments");
 	x.parts = 1 + A->cplx;
-	for (int m = 0; m <= A->cplx; m++) x.part[m] = halfArgs<T>(A, h, m);
+	for (int m = 0; m <= A->cplx; m++) {
+		x.part[m] = halfArgs<T>(A, h, m);
+		if (m < A->cplx) x.part[m].ends = 0;
+	}
 	x.post = postArgs<T>(A, h);
 	for (size_t g = 0; g + 1 < A->post[h].size(); g++) {
 		const PostSeg &G = A->post[h][g];
 		x.seg[x.segs].ops = (const PostOp<T> *)G.ops, x.seg[x.segs].pieces = (const PostPiece *)G.pieces;
-		x.seg[x.segs++].n = (int)blocksFor(G.total, POST_WG);
+		x.seg[x.segs].n = (int)(G.rest / POST_BLK);
+		if (x.seg[x.segs].n) x.segs++;
 	}
-	if (coreHalf<T>(D, h, &x)) return -1;
+	if (!D->postBuilt && buildPost<T>(D)) return -1;
+	if (coreHalf<T>(D, h, true, &x)) return -1;
 	PostArgs<T> last = x.post;
 	const PostSeg &G = A->post[h].back();
 	last.ops = (const PostOp<T> *)G.ops, last.pieces = (const PostPiece *)G.pieces;
-	last.total = G.total, last.post = (int)blocksFor(G.total, POST_WG);
-	return postHalf<T>(D, h, &last);
+	last.post = (int)(G.rest / POST_BLK);
+	return postHalf<T>(D, h, true, last.post ? &last : nullptr);
 }
 
 // Run the end of half step h: the recorded strips and sources, then the ghost copies.
-// x: an auxiliary world's launch to take along, or null.
+// copied: the curl has made the copies it can.  x: an auxiliary world's launch to take along, or null.
 template<class T>
-int postHalf(alis_dev_world *D, int h, const PostArgs<T> *x)
+int postHalf(alis_dev_world *D, int h, bool copied, const PostArgs<T> *x)
 {
 	if (!D->postBuilt && buildPost<T>(D)) return -1;
 	PostArgs<T> a = postArgs<T>(D, h);
@@ -2219,13 +2377,14 @@ int postHalf(alis_dev_world *D, int h, const PostArgs<T> *x)
 	for (size_t s = 0; s < D->tf.size(); s++) bind = bind || sideStream(s);
 	if (bind && !D->halfDone) HIPCHECK(hipEventCreateWithFlags(&D->halfDone, hipEventDisableTiming));
 	int last = -1;
-	for (int g = 0; g < (int)D->post[h].size(); g++) if (D->post[h][g].total) last = g;
+	auto cells = [&](const PostSeg &G) { return copied ? G.rest : G.total; };
+	for (int g = 0; g < (int)D->post[h].size(); g++) if (cells(D->post[h][g])) last = g;
 	for (int g = 0; g <= last; g++) {
 		const PostSeg &G = D->post[h][g];
-		if (!G.total) continue;
+		if (!cells(G)) continue;
 		a.ops = (const PostOp<T> *)G.ops;
 		a.pieces = (const PostPiece *)G.pieces;
-		a.total = G.total, a.post = (int)blocksFor(G.total, POST_WG);
+		a.post = (int)(cells(G) / POST_BLK);
 		unsigned blocks = a.post;
 		if (g == last && h == 1 && D->pendAde) a.ade = objArgs<T>(D), blocks += objBlocks(D), D->pendAde = false;
 		if (g == last && x) launchEv(k_post_aux<T>, dim3(blocks + x->post), dim3(POST_WG), 0, D->st, nullptr, bind ? D->halfDone : nullptr, a, *x, (int)blocks);
@@ -2489,7 +2648,7 @@ int fusedStep(alis_dev_world *D)
 	for (const PostSeg &G : D->copies) {
 		a.ops = (const PostOp<T> *)G.ops;
 		a.pieces = (const PostPiece *)G.pieces;
-		a.total = G.total, a.post = (int)blocksFor(G.total, POST_WG);
+		a.post = (int)(G.total / POST_BLK);
 		unsigned blocks = a.post;
 		a.ade = ObjArgs<T>{};
 		if (D->pendAde) a.ade = objArgs<T>(D), blocks += objBlocks(D), D->pendAde = false;
@@ -2520,20 +2679,23 @@ int auxHalves(alis_dev_world *D)
 	return 0;
 }
 
+int batchFlush(alis_dev_batch *B);
+
 // Complete a deferred step the separate way (a call that reads or changes the world between
 // its E and H halves, or that reads an auxiliary world whose H half waits).
 template<class T>
 int flushStep(alis_dev_world *D)
 {
+	if (D->pendBatch) return batchFlush(D->pendBatch);
 	if (D->pendH && D->mainOf) return flushStep<T>(D->mainOf);
 	if (D->pendCore && D->mainOf) return flushStep<T>(D->mainOf);
 	if (D->pendMain) {
 		const int h = D->pendMain - 1;
-		alis_dev_world *A = D->tf[0].aux;
+		alis_dev_world *A = D->pendFold ? D->tf[0].aux : nullptr;
 		const bool core = A && A->pendCore, ghosts = A && A->pendGhosts;
-		D->pendMain = 0;
+		D->pendMain = 0, D->pendFold = false;
 		if (A) A->pendCore = A->pendGhosts = 0;
-		if (coreHalf<T>(D, h)) return -1;
+		if (coreHalf<T>(D, h) || flushAde<T>(D)) return -1;
 		if (core && coreHalf<T>(A, h)) return -1;
 		return ghosts ? postHalf<T>(A, h) : 0;
 	}
@@ -2562,7 +2724,7 @@ int coreEntry(alis_dev_world *D, int h)
 		D->pendH = 1;
 		return 0;
 	}
-	if (D->mainOf && D->mainOf->pendMain == 1 + h && !D->pendCore && !D->pendGhosts) {
+	if (D->mainOf && D->mainOf->pendFold && D->mainOf->pendMain == 1 + h && !D->pendCore && !D->pendGhosts) {
 		D->pendCore = 1 + h;
 		return 0;
 	}
@@ -2575,13 +2737,10 @@ int coreEntry(alis_dev_world *D, int h)
 			return 0;
 		}
 	}
-	bool fold;
-	if (foldsAux<T>(D, fold)) return -1;
-	if (fold) {                         // with the auxiliary world's half step at alis_dev_ghosts
-		D->pendMain = 1 + h;
-		return 0;
-	}
-	return coreHalf<T>(D, h);
+	// at alis_dev_ghosts, with the auxiliary world's half step where it can come along
+	if (foldsAux<T>(D, D->pendFold)) return -1;
+	D->pendMain = 1 + h;
+	return 0;
 }
 
 template<class T>
@@ -2596,7 +2755,12 @@ int ghostsEntry(alis_dev_world *D, int h)
 		D->pendGhosts = 1 + h;
 		return 0;
 	}
-	if (D->pendMain == 1 + h && D->tf[0].aux && D->tf[0].aux->pendGhosts == 1 + h) return foldedHalf<T>(D, h);
+	if (D->pendMain == 1 + h && D->pendFold && D->tf[0].aux && D->tf[0].aux->pendGhosts == 1 + h) return foldedHalf<T>(D, h);
+	if (D->pendMain == 1 + h && !D->pendFold) {
+		D->pendMain = 0;
+		if (!D->postBuilt && buildPost<T>(D)) return -1;
+		return coreHalf<T>(D, h, true) ? -1 : postHalf<T>(D, h, true);
+	}
 	if (h == 1 && D->pendH == 1) {
 		D->pendH = 2;
 		return 0;
@@ -2877,7 +3041,8 @@ struct alis_dev_batch {
 	std::vector<CurlClass> curlClass[2];
 	void *objArgs = nullptr, *objStart = nullptr;   // ObjArgs<T>[] of the worlds with objects
 	int objEntries = 0, objBlocks = 0;
-	bool postReady = false;
+	int pend = 0;               // 1 + h: the core of half step h waits for its post
+	bool postReady[2] = {false, false};
 	struct Round {
 		std::vector<int> world;     // index into W
 		std::vector<int> seg;       // segment of that world
@@ -2886,11 +3051,12 @@ struct alis_dev_batch {
 		void *start = nullptr;      // int[] workgroup starts (device)
 		long blocks = 0;
 	};
-	std::vector<Round> rounds[2];
+	// per half step; [1]: after curls that made the copies they can
+	std::vector<Round> rounds[2][2];
 	// every round's arguments of a half step: staged together, fetched in one copy
-	void *postArgs[2] = {}, *postPinned[2] = {};
-	size_t postBytes[2] = {};
-	hipEvent_t postDone[2] = {};    // the last copy from postPinned has been made
+	void *postArgs[2][2] = {}, *postPinned[2][2] = {};
+	size_t postBytes[2][2] = {};
+	hipEvent_t postDone[2][2] = {};    // the last copy from postPinned has been made
 	std::vector<void *> allocs;
 	bool held = false;              // counted in its worlds' inBatch
 };
@@ -2901,6 +3067,14 @@ int batchAlloc(alis_dev_batch *B, void **p, size_t bytes)
 {
 	HIPCHECK(hipMalloc(p, bytes ? bytes : 16));
 	B->allocs.push_back(*p);
+	return 0;
+}
+
+template<class T>
+int batchPrograms(alis_dev_batch *B)
+{
+	for (alis_dev_world *D : B->W)
+		if (!D->postBuilt && buildPost<T>(D)) return -1;
 	return 0;
 }
 
@@ -2916,7 +3090,8 @@ int batchBuildCurl(alis_dev_batch *B)
 		for (alis_dev_world *D : B->W) {
 			const bool pair = pairs && D->cplx;
 			for (int m = 0; m <= D->cplx; m++) {
-				const HalfArgs<T> a = halfArgs<T>(D, h, m);
+				HalfArgs<T> a = halfArgs<T>(D, h, m);
+				if (!pair && m < D->cplx) a.ends = 0;        // the imaginary part's entry makes both parts' copies
 				// 1/eps: 2 per-segment table (and arrays where a segment is mixed), 1 arrays, 0 none
 				const int cm = a.seg ? 2 : a.C[0] ? 1 : 0;
 				if (pair && m == 1) all.back().a[1] = a;
@@ -2969,53 +3144,55 @@ int batchBuildObjects(alis_dev_batch *B)
 }
 
 template<class T>
-int batchBuildPost(alis_dev_batch *B)
+int batchBuildPost(alis_dev_batch *B, bool copied)
 {
-	for (alis_dev_world *D : B->W)
-		if (!D->postBuilt && buildPost<T>(D)) return -1;
 	for (int h = 0; h < 2; h++) {
 		size_t rounds = 0;
 		for (alis_dev_world *D : B->W) rounds = std::max(rounds, D->post[h].size());
-		B->rounds[h].assign(rounds, alis_dev_batch::Round{});
+		B->rounds[copied][h].assign(rounds, alis_dev_batch::Round{});
 		for (size_t r = 0; r < rounds; r++) {
-			alis_dev_batch::Round &R = B->rounds[h][r];
+			alis_dev_batch::Round &R = B->rounds[copied][h][r];
 			std::vector<int> start;
 			for (int w = 0; w < (int)B->W.size(); w++) {
 				alis_dev_world *D = B->W[w];
-				if (r >= D->post[h].size() || !D->post[h][r].total) continue;
+				if (r >= D->post[h].size()) continue;
+				long blocks = (copied ? D->post[h][r].rest : D->post[h][r].total) / POST_BLK;
+				// the current update runs with a world's last H launch
+				if (h == 1 && r + 1 == D->post[h].size()) blocks += objBlocks(D);
+				if (!blocks) continue;
 				R.world.push_back(w), R.seg.push_back((int)r);
 				start.push_back((int)R.blocks);
-				R.blocks += D->post[h][r].total / POST_WG;
-				// the current update runs with a world's last H launch
-				if (h == 1 && r + 1 == D->post[h].size()) R.blocks += objBlocks(D);
+				R.blocks += blocks;
 			}
 			if (R.world.empty()) continue;
 			if (batchAlloc(B, &R.start, start.size() * sizeof(int))) return -1;
 			HIPCHECK(hipMemcpyAsync(R.start, start.data(), start.size() * sizeof(int), hipMemcpyHostToDevice, B->st));
 		}
 		size_t bytes = 0;
-		for (const alis_dev_batch::Round &R : B->rounds[h]) bytes += (R.world.size() * sizeof(PostArgs<T>) + 255) / 256 * 256;
+		for (const alis_dev_batch::Round &R : B->rounds[copied][h]) bytes += (R.world.size() * sizeof(PostArgs<T>) + 255) / 256 * 256;
 		if (!bytes) continue;
-		if (batchAlloc(B, &B->postArgs[h], bytes)) return -1;
-		HIPCHECK(hipHostMalloc(&B->postPinned[h], bytes, hipHostMallocDefault));
-		HIPCHECK(hipEventCreateWithFlags(&B->postDone[h], hipEventDisableTiming));
-		HIPCHECK(hipEventRecord(B->postDone[h], B->st));
-		B->postBytes[h] = bytes;
+		if (batchAlloc(B, &B->postArgs[copied][h], bytes)) return -1;
+		HIPCHECK(hipHostMalloc(&B->postPinned[copied][h], bytes, hipHostMallocDefault));
+		HIPCHECK(hipEventCreateWithFlags(&B->postDone[copied][h], hipEventDisableTiming));
+		HIPCHECK(hipEventRecord(B->postDone[copied][h], B->st));
+		B->postBytes[copied][h] = bytes;
 		size_t off = 0;
-		for (alis_dev_batch::Round &R : B->rounds[h]) {
+		for (alis_dev_batch::Round &R : B->rounds[copied][h]) {
 			if (R.world.empty()) continue;
-			R.args = (char *)B->postArgs[h] + off, R.pinned = (char *)B->postPinned[h] + off;
+			R.args = (char *)B->postArgs[copied][h] + off, R.pinned = (char *)B->postPinned[copied][h] + off;
 			off += (R.world.size() * sizeof(PostArgs<T>) + 255) / 256 * 256;
 		}
 	}
 	HIPCHECK(hipStreamSynchronize(B->st));
-	B->postReady = true;
+	B->postReady[copied] = true;
 	return 0;
 }
 
+// copies: the launch makes the ghost copies along z that it can (see coreHalf).
 template<class T>
-int batchCore(alis_dev_batch *B, int h)
+int batchCore(alis_dev_batch *B, int h, bool copies)
 {
+	if (batchPrograms<T>(B) || (!B->curl[0] && batchBuildCurl<T>(B))) return -1;
 	alis_dev_world *D0 = B->W[0];
 	for (alis_dev_world *W : B->W) {
 		dropPresamples(W);
@@ -3037,7 +3214,7 @@ int batchCore(alis_dev_batch *B, int h)
 		const int *start = (const int *)B->curlStart[h] + c.first;
 		const dim3 grid(c.blocks), block(CURL_WG);
 		hipEvent_t s0 = q == 0 ? e0 : nullptr, s1 = q + 1 == cls.size() ? e1 : nullptr;
-#define CURL_BATCH(H, C) (c.pair ? launchEv(k_curl_batch<T, H, C, true>, grid, block, 0, B->st, s0, s1, args, start, c.n) : launchEv(k_curl_batch<T, H, C, false>, grid, block, 0, B->st, s0, s1, args, start, c.n))
+#define CURL_BATCH(H, C) (c.pair ? launchEv(k_curl_batch<T, H, C, true>, grid, block, 0, B->st, s0, s1, args, start, c.n, (int)copies) : launchEv(k_curl_batch<T, H, C, false>, grid, block, 0, B->st, s0, s1, args, start, c.n, (int)copies))
 		if (h == 1) CURL_BATCH(1, 0);
 		else if (c.cm == 2) CURL_BATCH(0, 2);
 		else if (c.cm == 1) CURL_BATCH(0, 1);
@@ -3053,12 +3230,12 @@ int batchCore(alis_dev_batch *B, int h)
 }
 
 template<class T>
-int batchPost(alis_dev_batch *B, int h)
+int batchPost(alis_dev_batch *B, int h, bool copied)
 {
-	if (!B->postReady && batchBuildPost<T>(B)) return -1;
-	if (!B->postBytes[h]) return 0;
-	HIPCHECK(hipEventSynchronize(B->postDone[h]));
-	for (alis_dev_batch::Round &R : B->rounds[h]) {
+	if (batchPrograms<T>(B) || (!B->postReady[copied] && batchBuildPost<T>(B, copied))) return -1;
+	if (!B->postBytes[copied][h]) return 0;
+	HIPCHECK(hipEventSynchronize(B->postDone[copied][h]));
+	for (alis_dev_batch::Round &R : B->rounds[copied][h]) {
 		if (R.world.empty()) continue;
 		PostArgs<T> *a = (PostArgs<T> *)R.pinned;
 		for (size_t e = 0; e < R.world.size(); e++) {
@@ -3067,15 +3244,15 @@ int batchPost(alis_dev_batch *B, int h)
 			memset(&a[e], 0, sizeof(PostArgs<T>));
 			a[e].ops = (const PostOp<T> *)g.ops;
 			a[e].pieces = (const PostPiece *)g.pieces;
-			a[e].total = g.total, a[e].post = (int)(g.total / POST_WG);
+			a[e].post = (int)((copied ? g.rest : g.total) / POST_BLK);
 			if (h == 1 && R.seg[e] + 1 == (int)D->post[h].size() && D->pendAde) a[e].ade = objArgs<T>(D), D->pendAde = false;
 			a[e].strips = D->pendStrips[h];
 			for (size_t w = 0; w < D->pendSrc[h].size(); w++) a[e].src[w] = D->pendSrc[h][w];
 			for (size_t q = 0; q < D->pendWave[h].size(); q++) a[e].wave[q] = (T)D->pendWave[h][q];
 		}
 	}
-	fetchArgs(B->postArgs[h], B->postPinned[h], B->postBytes[h], B->st, B->postDone[h]);
-	for (alis_dev_batch::Round &R : B->rounds[h]) {
+	fetchArgs(B->postArgs[copied][h], B->postPinned[copied][h], B->postBytes[copied][h], B->st, B->postDone[copied][h]);
+	for (alis_dev_batch::Round &R : B->rounds[copied][h]) {
 		if (R.world.empty()) continue;
 		k_post_batch<T><<<R.blocks, POST_WG, 0, B->st>>>((const PostArgs<T> *)R.args, (const int *)R.start, (int)R.world.size());
 		HIPCHECK(hipGetLastError());
@@ -3085,6 +3262,17 @@ int batchPost(alis_dev_batch *B, int h)
 		D->pendStrips[h] = 0;
 		std::fill(D->pendSrc[h].begin(), D->pendSrc[h].end(), 0u);
 	}
+	return 0;
+}
+
+// The waiting core of B, apart from its post.
+int batchFlush(alis_dev_batch *B)
+{
+	const int h = B->pend - 1;
+	B->pend = 0;
+	for (alis_dev_world *W : B->W) W->pendBatch = nullptr;
+	if (B->fp64 ? batchCore<double>(B, h, false) : batchCore<float>(B, h, false)) return -1;
+	for (alis_dev_world *W : B->W) if (B->fp64 ? flushAde<double>(W) : flushAde<float>(W)) return -1;
 	return 0;
 }
 
@@ -3161,7 +3349,7 @@ int alis_dev_link_tfsf(alis_dev_world *D, int s, alis_dev_world *aux)
 void alis_dev_release(alis_dev_world *D)
 {
 	if (!D) return;
-	if (D->pendMain || D->pendCore) (void)flushE(D);     // an auxiliary world's half step outlives its main world
+	if (D->pendMain || D->pendCore || D->pendBatch) (void)flushE(D);     // an auxiliary world's half step outlives its main world
 	if (D->st) hipStreamSynchronize(D->st);
 	for (DevTfsf &t : D->tf) if (t.aux && t.aux->mainOf == D) t.aux->mainOf = nullptr;
 	if (D->mainOf)
@@ -4023,8 +4211,7 @@ int alis_dev_batch_create(alis_dev_world *const *D, int n, alis_dev_batch **out)
 		if (joinStream(D[w], D[0])) { delete B; return -1; }
 	}
 	B->st = D[0]->st;
-	int rc = B->fp64 ? batchBuildCurl<double>(B) || batchBuildObjects<double>(B) : batchBuildCurl<float>(B) || batchBuildObjects<float>(B);
-	if (rc) rc = -1;
+	const int rc = B->fp64 ? batchBuildObjects<double>(B) : batchBuildObjects<float>(B);
 	if (rc) { alis_dev_batch_release(B); return rc; }
 	for (alis_dev_world *W : B->W) W->inBatch++;   // their arrays stay where the arguments name them
 	B->held = true;
@@ -4043,30 +4230,43 @@ static int batchStream(alis_dev_batch *B)
 	return 0;
 }
 
+// The core waits for the batch's post, like alis_dev_core (see coreEntry).
 int alis_dev_batch_core(alis_dev_batch *B, int h)
 {
 	if (h < 0 || h > 1) return fail("no such half step");
 	if (batchStream(B)) return -1;
-	return B->fp64 ? batchCore<double>(B, h) : batchCore<float>(B, h);
+	for (alis_dev_world *W : B->W) if (flushE(W)) return -1;
+	B->pend = 1 + h;
+	for (alis_dev_world *W : B->W) W->pendBatch = B;
+	return 0;
 }
 
 int alis_dev_batch_post(alis_dev_batch *B, int h)
 {
 	if (h < 0 || h > 1) return fail("no such half step");
 	if (batchStream(B)) return -1;
-	return B->fp64 ? batchPost<double>(B, h) : batchPost<float>(B, h);
+	const bool whole = B->pend == 1 + h;
+	if (whole) {
+		B->pend = 0;
+		for (alis_dev_world *W : B->W) W->pendBatch = nullptr;
+		if (B->fp64 ? batchCore<double>(B, h, true) : batchCore<float>(B, h, true)) return -1;
+	}
+	else for (alis_dev_world *W : B->W) if (W->pendBatch && flushE(W)) return -1;
+	return B->fp64 ? batchPost<double>(B, h, whole) : batchPost<float>(B, h, whole);
 }
 
 void alis_dev_batch_release(alis_dev_batch *B)
 {
 	if (!B) return;
+	if (B->pend) (void)batchFlush(B);
 	for (alis_dev_world *W : B->W) hipStreamSynchronize(W->st);   // the batch's launches ran on one of these
 	if (B->held) for (alis_dev_world *W : B->W) W->inBatch--;
 	for (void *p : B->allocs) hipFree(p);
-	for (int h = 0; h < 2; h++) {
-		if (B->postPinned[h]) hipHostFree(B->postPinned[h]);
-		if (B->postDone[h]) hipEventDestroy(B->postDone[h]);
-	}
+	for (int z = 0; z < 2; z++)
+		for (int h = 0; h < 2; h++) {
+			if (B->postPinned[z][h]) hipHostFree(B->postPinned[z][h]);
+			if (B->postDone[z][h]) hipEventDestroy(B->postDone[z][h]);
+		}
 	delete B;
 }
 

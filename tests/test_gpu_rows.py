@@ -73,3 +73,49 @@ def test_scatterer_rows(cells, bits):
 @pytest.mark.parametrize("bits", [32, 64])
 def test_half_step_in_parts(bits):
     _agree("nanoblock", 109, bits, 8, parted=True)
+
+
+@pytest.mark.parametrize("worlds", [2])
+def test_batch_half_step_in_parts(worlds):
+    """A read between the core and the post of a batch (complex worlds, Bloch boundaries)."""
+    out = {}
+    for kind in LIBS:
+        w, e = ctypes.CDLL(str(LIBS[kind])), ctypes.CDLL(str(ENGINES[kind]))
+        w.wl_create.restype = w.wl_device_of.restype = ctypes.c_void_p
+        w.wl_create.argtypes = [ctypes.c_char_p] + [ctypes.c_int] * 3
+        w.wl_step.argtypes = w.wl_device_of.argtypes = [ctypes.c_void_p, ctypes.c_int]
+        w.wl_free.argtypes = [ctypes.c_void_p]
+        w.wl_field.restype = ctypes.c_long
+        w.wl_field.argtypes = [ctypes.c_void_p] + [ctypes.c_int] * 4 + [ctypes.POINTER(ctypes.c_double), ctypes.c_long]
+        e.alis_dev_batch_create.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_int, ctypes.POINTER(ctypes.c_void_p)]
+        for f in (e.alis_dev_batch_core, e.alis_dev_batch_post):
+            f.argtypes = [ctypes.c_void_p, ctypes.c_int]
+        e.alis_dev_batch_release.argtypes = [ctypes.c_void_p]
+        e.alis_dev_batch_release.restype = None
+        c = w.wl_create(b"kpoints", worlds, 32, 64)
+        w.wl_step(c, 3)
+        dev = (ctypes.c_void_p * worlds)(*[w.wl_device_of(c, q) for q in range(worlds)])
+        B = ctypes.c_void_p()
+        assert e.alis_dev_batch_create(dev, worlds, ctypes.byref(B)) == 0
+        buf = (ctypes.c_double * 2000000)()
+        got = []
+
+        def read():
+            for q in range(worlds):
+                for h in range(2):
+                    for m in range(2):
+                        for a in range(3):
+                            n = w.wl_field(c, q, h, m, a, buf, len(buf))
+                            assert n > 0
+                            got.append(np.frombuffer(buf, dtype=np.float64, count=n).copy())
+        for h in range(2):
+            assert e.alis_dev_batch_core(B, h) == 0
+            read()
+            assert e.alis_dev_batch_post(B, h) == 0
+        for h in range(2):
+            assert e.alis_dev_batch_core(B, h) == 0 and e.alis_dev_batch_post(B, h) == 0
+        read()
+        e.alis_dev_batch_release(B)
+        w.wl_free(c)
+        out[kind] = np.concatenate(got)
+    assert np.abs(out["oracle"]).max() > 0 and np.array_equal(out["hip"], out["oracle"])
