@@ -119,3 +119,26 @@ def test_batch_half_step_in_parts(worlds):
         w.wl_free(c)
         out[kind] = np.concatenate(got)
     assert np.abs(out["oracle"]).max() > 0 and np.array_equal(out["hip"], out["oracle"])
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+def test_whole_sync_over_many_chunks(bits):
+    """The host fields of a world whose arrays take several chunks of the copy to the host (110^3: 10 of
+    4 MiB, over all its threads): the sum of their squares is the oracle's (FP64: as rounded to float)."""
+    sums = {}
+    for kind in LIBS:
+        w = ctypes.CDLL(str(LIBS[kind]))
+        w.wl_create.restype = ctypes.c_void_p
+        w.wl_create.argtypes = [ctypes.c_char_p] + [ctypes.c_int] * 3
+        w.wl_step.argtypes = [ctypes.c_void_p, ctypes.c_int]
+        w.wl_checksum.restype = ctypes.c_double
+        w.wl_checksum.argtypes = w.wl_free.argtypes = [ctypes.c_void_p]
+        c = w.wl_create(b"nanoblock", 110, bits, 64)
+        sums[kind] = []
+        for _ in range(2):
+            w.wl_step(c, 15)                             # (the first steps are all zeros)
+            sums[kind].append(w.wl_checksum(c))
+        w.wl_free(c)
+    assert sums["oracle"][0] > 0
+    for got, ref in zip(sums["hip"], sums["oracle"]):
+        assert got == ref if bits == 32 else abs(got - ref) <= 1e-7 * ref
