@@ -122,6 +122,22 @@ template<class T> __device__ inline __attribute__((address_space(1))) T *glb(T *
 // scalar cache.
 template<class P> __device__ __forceinline__ const __attribute__((address_space(4))) P *uniform(const P *p) { return (const __attribute__((address_space(4))) P *)p; }
 
+// The operations of the end of a half step (see k_post).
+enum { OP_COPY = 0, OP_STRIP = 1, OP_SOURCE = 2 };
+
+template<class T> struct PostOp {
+	int kind, slot;             // slot: TF/SF box (STRIP) or source index (SOURCE)
+	T *F, *G;                   // target; COPY: imaginary partner or null
+	const T *A;                 // STRIP: auxiliary field
+	const T *C;                 // STRIP: 1/eps or null; SOURCE: amplitude array or null
+	const T *W;                 // SOURCE: per-cell waves or null
+	Lay LF, LA, LC;
+	Box b;
+	int di, dj, dk;
+	T c, s;                     // COPY: cos, sin; STRIP: dt/ds; SOURCE: scalar amplitude
+	int exX, exY, auxIMAX, auxJMAX, altX, altY;
+};
+
 #include "curl_quads.inc"
 #include "objects.inc"
 
@@ -175,22 +191,11 @@ __global__ __launch_bounds__(256) void k_carry(CarryArgs<T> a)
 // Cells that a later copy overwrites belong to no earlier piece.  The host splits a
 // program into several launches where a chain's base cell is written by the same launch
 // (see buildPost), so every launch only reads cells it does not write.
-enum { OP_COPY = 0, OP_STRIP = 1, OP_SOURCE = 2 };
-
-template<class T> struct PostOp {
-	int kind, slot;             // slot: TF/SF box (STRIP) or source index (SOURCE)
-	T *F, *G;                   // target; COPY: imaginary partner or null
-	const T *A;                 // STRIP: auxiliary field
-	const T *C;                 // STRIP: 1/eps or null; SOURCE: amplitude array or null
-	const T *W;                 // SOURCE: per-cell waves or null
-	Lay LF, LA, LC;
-	Box b;
-	int di, dj, dk;
-	T c, s;                     // COPY: cos, sin; STRIP: dt/ds; SOURCE: scalar amplitude
-	int exX, exY, auxIMAX, auxJMAX, altX, altY;
-};
-
 constexpr int MAXSRC = 128;     // sources per chain (E or H) of one world
+// A curl launch applies the additive operations where its workgroups meet ADDS_FEW of them in all, or
+// where it has at most ADDS_TILES workgroups and they meet ADDS_MET each (see buildPost).
+constexpr int ADDS_FEW = 64, ADDS_TILES = 4096;
+constexpr double ADDS_MET = 0.75;
 constexpr int MAXCHAIN = 24;    // copies per launch
 constexpr int MAXPOST = 48;     // operations per launch
 constexpr int POST_WG = 64;     // threads per workgroup of k_post: one wavefront (64 k-point worlds:
@@ -258,8 +263,8 @@ __device__ __forceinline__ int divBy(int t, int d, unsigned r)
 // nanoblock H program 17.5 -> 16.1 us).  That chain is what bounds it: piece and operation come
 // through the scalar cache, and a thread takes POST_U cells, whose loads are in flight together
 // (256^3 H program with its current update 23 -> 18 us, 64 spheres 42 -> 36, 6 worlds 32 -> 27).
-// (tid: the thread's place in the workgroup.)
-template<class T, class A>
+// tid: the thread's place in the workgroup; ADDS: pieces may be additive.
+template<class T, bool ADDS = true, class A>
 __device__ __forceinline__ void postCells(const A &a, const PostOp<T> *allOps, const PostPiece *pieces, int blk, int tid)
 {
 	const auto &P = uniform(pieces)[blk];
@@ -300,22 +305,24 @@ __device__ __forceinline__ void postCells(const A &a, const PostOp<T> *allOps, c
 			}
 		return;
 	}
-	bool on = false;
-	for (int x = 0; x < P.n; x++) {
-		const auto &r = ops[P.list[x]];
-		if (!opOn(a, r)) continue;
-		if (!on)
+	if constexpr (ADDS) {
+		bool on = false;
+		for (int x = 0; x < P.n; x++) {
+			const auto &r = ops[P.list[x]];
+			if (!opOn(a, r)) continue;
+			if (!on)
 #pragma unroll
-			for (int u = 0; u < POST_U; u++) f[u] = glb(F)[d[u]];
-		on = true;
-		const T wave = r.kind == OP_SOURCE ? a.wave[r.slot] : T(0);
+				for (int u = 0; u < POST_U; u++) f[u] = glb(F)[d[u]];
+			on = true;
+			const T wave = r.kind == OP_SOURCE ? a.wave[r.slot] : T(0);
 #pragma unroll
-		for (int u = 0; u < POST_U; u++) f[u] = addTo<T>(r, f[u], i[u], j[u], k[u], wave);
+			for (int u = 0; u < POST_U; u++) f[u] = addTo<T>(r, f[u], i[u], j[u], k[u], wave);
+		}
+		if (!on) return;
+#pragma unroll
+		for (int u = 0; u < POST_U; u++)
+			if (t0 + u * POST_WG < count) glb(F)[d[u]] = f[u];
 	}
-	if (!on) return;
-#pragma unroll
-	for (int u = 0; u < POST_U; u++)
-		if (t0 + u * POST_WG < count) glb(F)[d[u]] = f[u];
 }
 
 template<class T, class A>
@@ -949,7 +956,9 @@ struct PostSeg {
 	void *pieces = nullptr;     // PostPiece[total / POST_BLK] in device memory: each workgroup's
 	                            //  piece
 	long total = 0;             // cells (a multiple of POST_BLK)
-	long rest = 0;              // those of them before the copies that the curl can make (see rowCopyOf)
+	// the cells stand in this order: copies, strips and sources (up to `rest`), and the copies that the
+	// curl can make (see rowCopyOf); bare: the first alone
+	long rest = 0, bare = 0;
 };
 
 struct alis_dev_batch;
@@ -1050,6 +1059,7 @@ struct alis_dev_world {
 	// (A world without one also waits: the curl then makes some of the ghost copies.)
 	int pendMain = 0, pendCore = 0, pendGhosts = 0;
 	bool pendFold = false;      // main world waiting: with its auxiliary world
+	bool pendPost = false;      // E's ghost copies wait for H's (which no H curl reads): one launch
 	alis_dev_batch *pendBatch = nullptr;  // the batch whose core of a half step waits
 	struct RowCopyBox { Box b; double c, s; };
 	RowCopyBox rowCopy[2][2] = {};        // [h][end] (RowCopy)
@@ -1069,8 +1079,10 @@ struct alis_dev_world {
 	int objWgs = 0;             // workgroups of one component of one part
 	bool pendAde = false;       // the current update of the last H core is still to run
 	struct AddRef { int kind, slot; };
-	std::vector<AddRef> adds[2][2];   // [part][half]: the additive operations of k_step's lists
-	void *addTab[2][2] = {}, *addAt[2][2] = {};   // their tables on the device (StepAdd<T>, bits per plane)
+	std::vector<AddRef> adds[2][2];   // [part][half]: the additive operations of the curl's lists
+	// their tables on the device (StepAdd<T>; bits per plane, and per workgroup of a curl launch)
+	void *addTab[2][2] = {}, *addAt[2][2] = {}, *addTile[2][2] = {};
+	bool addsInCurl[2] = {false, false};   // per half: they lie in the update range and fit AddArgs
 	struct Carry { int axis; Box b; };
 	std::vector<Carry> carry[2];  // cells a fused step's ghost copies take from the other set
 	std::vector<Box> hWrites;   // the boxes the end-of-H-half program writes
@@ -1803,10 +1815,31 @@ int zSamples(alis_dev_world *D, PhsZ<T> *zs, std::vector<DevPhaser *> &owners, b
 	return n;
 }
 
-// copies: the launch makes the ghost copies along z that it can; the program without them follows.
+// What the curl of half step h makes of its end: 1 the copies along z that it can, 2 and the strips
+// and sources.
+int curlMakes(const alis_dev_world *D, int h) { return D->addsInCurl[h] ? 2 : 1; }
+
+// The additive operations of part m that this half step's curl applies.
+template<class T>
+AddArgs<T> addArgs(const alis_dev_world *D, int h, int m, bool whole)
+{
+	AddArgs<T> a{};
+	if (!whole || !D->addsInCurl[h]) return a;
+	a.add = (const StepAdd<T> *)D->addTab[m][h], a.at = (const unsigned long long *)D->addTile[m][h];
+	for (size_t u = 0; u < D->adds[m][h].size(); u++) {
+		const alis_dev_world::AddRef &r = D->adds[m][h][u];
+		const bool on = r.kind == OP_STRIP ? (D->pendStrips[h] >> r.slot) & 1u : (D->pendSrc[h][r.slot >> 5] >> (r.slot & 31)) & 1u;
+		if (on) a.on |= 1ull << u;
+		if (on && r.kind == OP_SOURCE) a.wave[u] = (T)D->pendWave[h][r.slot];
+	}
+	return a;
+}
+
+// whole: the launch also does what it can of the end of the half step (curlMakes), and the rest of
+// that program follows.
 // x: an auxiliary world's share of the launch, or null.
 template<class T>
-int coreHalf(alis_dev_world *D, int h, bool copies = false, const AuxCurl<T> *x = nullptr)
+int coreHalf(alis_dev_world *D, int h, bool whole = false, const AuxCurl<T> *x = nullptr)
 {
 	dropPresamples(D);
 	hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1818,20 +1851,22 @@ int coreHalf(alis_dev_world *D, int h, bool copies = false, const AuxCurl<T> *x 
 	std::vector<DevPhaser *> sampled;
 	for (int m = 0; m <= D->cplx; m++) {
 		HalfArgs<T> a = halfArgs<T>(D, h, m);
-		if (!copies || m < D->cplx) a.ends = 0;
+		if (!whole || m < D->cplx) a.ends = 0;
+		const AddArgs<T> adds = addArgs<T>(D, h, m, whole);
 		ZFaces<T> z{};
 		const bool aux = x && m == 0;
 		const dim3 grid(a.tiles, a.ni + (aux ? 1 : 0)), block(CURL_WG);
 		if (h == 0 && m == 0 && D->objWgs) k_currents<T><<<objBlocks(D), OBJ_WG, 0, D->st>>>(objArgs<T>(D));
 		if (h == 1 && m == 0) z.n = zSamples<T>(D, z.z, sampled, false);   // phasers sample part 0
 		hipEvent_t s0 = m == 0 ? e0 : nullptr, s1 = m == D->cplx ? e1 : nullptr;
-#define CURL(H, C) (aux ? launchEv(k_curl_aux<T, H, C, false>, grid, block, 0, D->st, s0, s1, a, *x, z) : launchEv(k_curl<T, H, C>, grid, block, 0, D->st, s0, s1, a))
-		if (h == 0 && D->seg) CURL(0, 2);
-		else if (h == 0 && D->C[0]) CURL(0, 1);
-		else if (h == 0) CURL(0, 0);
-		else if (z.n && aux) launchEv(k_curl_aux<T, 1, 0, true>, grid, block, 0, D->st, s0, s1, a, *x, z);
-		else if (z.n) launchEv(k_curl_zs<T>, grid, block, 0, D->st, s0, s1, a, z);
-		else CURL(1, 0);
+#define CURL(H, C, Z) (aux && adds.on ? launchEv(k_curl_aux<T, H, C, Z, true>, grid, block, 0, D->st, s0, s1, a, *x, adds, z) : \
+                       aux ? launchEv(k_curl_aux<T, H, C, Z, false>, grid, block, 0, D->st, s0, s1, a, *x, adds, z) : \
+                       adds.on || Z ? launchEv(k_curl_adds<T, H, C, Z>, grid, block, 0, D->st, s0, s1, a, adds, z) : launchEv(k_curl<T, H, C>, grid, block, 0, D->st, s0, s1, a))
+		if (h == 0 && D->seg) CURL(0, 2, false);
+		else if (h == 0 && D->C[0]) CURL(0, 1, false);
+		else if (h == 0) CURL(0, 0, false);
+		else if (z.n) CURL(1, 0, true);
+		else CURL(1, 0, false);
 #undef CURL
 	}
 	if (h == 1 && D->objWgs) D->pendAde = true;   // with the end of the half step (or flushStep)
@@ -1975,7 +2010,7 @@ int postSegment(alis_dev_world *D, const std::vector<PostOp<T>> &v, int nadd, st
 	pieces.clear();
 	buildPieces(v, nadd, pieces, seg.total);
 	if (pieces.empty()) return 0;
-	seg.rest = seg.total;
+	seg.rest = seg.bare = seg.total;
 	if (wish) {
 		// The copies that the curl can make come last: an end's over the rows that all its
 		// components' pieces have in common, within those that the curl updates.
@@ -2006,11 +2041,11 @@ int postSegment(alis_dev_world *D, const std::vector<PostOp<T>> &v, int nadd, st
 			D->rowEnds[h] |= 1 << end;
 			for (int slot = 0; slot < (h == 1 ? 2 : 1); slot++) taken[of[end][slot]] = end;
 		}
-		std::vector<PostPiece> front, back;
+		std::vector<PostPiece> front, middle, back;
 		for (size_t n = 0; n < pieces.size(); n++) {
 			const PostPiece &P = pieces[n];
 			if (taken[n] < 0) {
-				front.push_back(P);
+				(P.kind == OP_COPY ? front : middle).push_back(P);
 				continue;
 			}
 			Box b = D->rowCopy[h][taken[n]].b;
@@ -2021,10 +2056,13 @@ int postSegment(alis_dev_world *D, const std::vector<PostOp<T>> &v, int nadd, st
 		long off = 0;
 		auto place = [&](PostPiece &P) { P.off = off, off += (P.b.count() + POST_BLK - 1) / POST_BLK * POST_BLK; };
 		for (PostPiece &P : front) place(P);
+		seg.bare = off;
+		for (PostPiece &P : middle) place(P);
 		seg.rest = off;
 		for (PostPiece &P : back) place(P);
 		seg.total = off;
 		pieces = front;
+		pieces.insert(pieces.end(), middle.begin(), middle.end());
 		pieces.insert(pieces.end(), back.begin(), back.end());
 	}
 	if (seg.total >= (1L << 31)) return fail("end-of-half-step launch over 2^31 threads");
@@ -2125,6 +2163,7 @@ int buildPost(alis_dev_world *D)
 	if ((int)D->tf.size() > 32) return fail("more than 32 TF/SF boxes in one world");
 	const Box range{D->iMIN, D->iMAX, D->jMIN, D->jMAX, D->kMIN, D->kMAX};
 	D->addsInside = true;
+	const int rowTiles = (int)(((long)D->jNUM * (D->L.sj / Quads<T>::N) + CURL_WG - 1) / CURL_WG);
 	D->copiesBuilt = false;
 	for (int h = 0; h < 2; h++) {
 		if ((int)D->src[h].size() > MAXSRC) return fail("more than 128 sources in one chain");
@@ -2147,7 +2186,8 @@ int buildPost(alis_dev_world *D)
 		}
 		copies = copyOps<T>(D, h);
 		dropEmpty(adds);
-		// k_step applies additive operations to the cells it updates
+		// the curl applies additive operations to the cells it updates
+		bool inside = true;
 		std::vector<StepAdd<T>> list[2];
 		for (PostOp<T> o : adds) {
 			// what an operation adds to cells beyond is lost where a ghost copy overwrites them
@@ -2155,7 +2195,7 @@ int buildPost(alis_dev_world *D)
 				bool lost = false;
 				for (const PostOp<T> &t : copies)
 					lost = lost || ((t.F == o.F || t.G == o.F) && x.i0 >= t.b.i0 && x.i1 <= t.b.i1 && x.j0 >= t.b.j0 && x.j1 <= t.b.j1 && x.k0 >= t.b.k0 && x.k1 <= t.b.k1);
-				if (!lost) D->addsInside = false;
+				if (!lost) inside = false;
 			}
 			o.b = Box{std::max(o.b.i0, range.i0), std::min(o.b.i1, range.i1), std::max(o.b.j0, range.j0), std::min(o.b.j1, range.j1),
 			          std::max(o.b.k0, range.k0), std::min(o.b.k1, range.k1)};
@@ -2164,23 +2204,43 @@ int buildPost(alis_dev_world *D)
 				for (int a = 0; a < 3; a++)
 					if (o.F == (T *)D->F[h][m][a]) list[m].push_back(StepAdd<T>{o, a});
 		}
+		for (int m = 0; m <= D->cplx; m++) inside = inside && list[m].size() <= (size_t)MAXADD;
+		D->addsInCurl[h] = inside;
+		long met = 0;                                    // operations that workgroups meet
+		D->addsInside = D->addsInside && inside;
 		for (int m = 0; m <= D->cplx; m++) {
 			D->adds[m][h].clear();
-			D->addTab[m][h] = D->addAt[m][h] = nullptr;
-			if (list[m].size() > (size_t)MAXADD) D->addsInside = false;
-			if (!D->addsInside || list[m].empty()) continue;
-			std::vector<unsigned long long> at(D->iNUM, 0ull);
+			D->addTab[m][h] = D->addAt[m][h] = D->addTile[m][h] = nullptr;
+			if (!inside || list[m].empty()) continue;
+			std::vector<unsigned long long> at(D->iNUM, 0ull), tile((size_t)D->iNUM * rowTiles, 0ull);
 			for (size_t u = 0; u < list[m].size(); u++) {
 				const PostOp<T> &o = list[m][u].o;
 				D->adds[m][h].push_back({o.kind, o.slot});
-				for (int i = o.b.i0; i <= o.b.i1; i++) at[i - D->iMIN] |= 1ull << u;
+				// the workgroups of a plane that hold its rows' quads k0 .. k1
+				const long pq = D->L.sj / Quads<T>::N, q0 = (o.b.k0 - D->kMIN) / Quads<T>::N, q1 = (o.b.k1 - D->kMIN) / Quads<T>::N;
+				std::vector<char> in(rowTiles, 0);
+				for (int j = o.b.j0; j <= o.b.j1; j++)
+					for (long t = ((j - D->jMIN) * pq + q0) / CURL_WG; t <= ((j - D->jMIN) * pq + q1) / CURL_WG; t++) in[t] = 1;
+				for (int i = o.b.i0; i <= o.b.i1; i++) {
+					at[i - D->iMIN] |= 1ull << u;
+					for (int t = 0; t < rowTiles; t++) if (in[t]) tile[(size_t)(i - D->iMIN) * rowTiles + t] |= 1ull << u, met++;
+				}
 			}
 			if (devAlloc(D, &D->addTab[m][h], list[m].size() * sizeof(StepAdd<T>))) return -1;
 			if (devAlloc(D, &D->addAt[m][h], at.size() * sizeof(at[0]))) return -1;
+			if (devAlloc(D, &D->addTile[m][h], tile.size() * sizeof(at[0]))) return -1;
 			HIPCHECK(hipMemcpyAsync(D->addTab[m][h], list[m].data(), list[m].size() * sizeof(StepAdd<T>), hipMemcpyHostToDevice, D->st));
 			HIPCHECK(hipMemcpyAsync(D->addAt[m][h], at.data(), at.size() * sizeof(at[0]), hipMemcpyHostToDevice, D->st));
+			HIPCHECK(hipMemcpyAsync(D->addTile[m][h], tile.data(), tile.size() * sizeof(at[0]), hipMemcpyHostToDevice, D->st));
 			HIPCHECK(hipStreamSynchronize(D->st));
 		}
+		// An operation that a workgroup meets is a chain of loads at the end of its wavefronts.  It pays
+		// where it saves the program's launch and little more than that launch's latency is at stake: a
+		// few workgroups meet any (sources; 40^3 dipole 1.25x, 64^3 1.14x), or the curl itself is a few
+		// rounds of the chip (strips of a 128^3 scatterer 1.02x; 256^3 0.98x).  Strips across a whole world,
+		// four for every workgroup, cost E 266 -> 400 us at 400x400x200 against 46 in k_post.
+		const double workgroups = (double)D->iNUM * rowTiles * (1 + D->cplx);
+		if (met > ADDS_FEW && (workgroups > ADDS_TILES || met > ADDS_MET * workgroups)) D->addsInCurl[h] = false;
 		if (h == 1) {
 			D->hWrites.clear(), D->hCopies.clear();
 			for (const PostOp<T> &o : adds) D->hWrites.push_back(o.b);
@@ -2269,7 +2329,7 @@ int waitForAux(alis_dev_world *D, unsigned strips)
 	for (size_t s = 0; s < D->tf.size(); s++) {
 		alis_dev_world *X = D->tf[s].aux;
 		if (!((strips >> s) & 1u)) continue;
-		if (X->pendMain && flushE(X)) return -1;
+		if ((X->pendMain || X->pendPost) && flushE(X)) return -1;
 		if (X->st == D->st) continue;
 		if (!X->halfDone) {
 			HIPCHECK(hipEventCreateWithFlags(&X->halfDone, hipEventDisableTiming));
@@ -2318,9 +2378,10 @@ int foldsAux(alis_dev_world *D, bool &on)
 		const long tiles = ((long)A->jNUM * (A->L.sj / Quads<T>::N) + CURL_WG - 1) / CURL_WG * A->iNUM * (1 + A->cplx);
 		if (tiles > AUX_TILES) return 0;
 		for (int h = 0; h < 2; h++) {
-			if (A->post[h].empty() || A->post[h].size() > (size_t)AUX_SEGS + 1) return 0;
+			if (!A->addsInCurl[h]) return 0;
+			if (A->post[h].size() > (size_t)AUX_SEGS) return 0;
 			for (size_t g = 0; g + 1 < A->post[h].size(); g++)
-				if (A->post[h][g].total > AUX_CELLS) return 0;
+				if (A->post[h][g].bare > AUX_CELLS) return 0;
 		}
 		if (joinStream(A, D)) return -1;
 		D->foldState = 1;
@@ -2330,7 +2391,46 @@ int foldsAux(alis_dev_world *D, bool &on)
 }
 
 template<class T>
-int postHalf(alis_dev_world *D, int h, bool copied = false, const PostArgs<T> *x = nullptr);
+int postHalf(alis_dev_world *D, int h, int made = 0, const PostArgs<T> *x = nullptr);
+
+// E's ghost copies, where they wait.
+template<class T>
+int postWaiting(alis_dev_world *D)
+{
+	if (!D->pendPost) return 0;
+	D->pendPost = false;
+	// (operations recorded since belong to the next E half step)
+	const unsigned strips = D->pendStrips[0];
+	const std::vector<unsigned> src = D->pendSrc[0];
+	const int rc = postHalf<T>(D, 0, 2);
+	D->pendStrips[0] = strips, D->pendSrc[0] = src;
+	return rc;
+}
+
+// The end of half step h after a whole curl.  E's ghost copies wait for H's where they are all that is
+// left of E's program: 40^3 dipole, 4 launches a step -> 3.
+template<class T>
+int endHalf(alis_dev_world *D, int h, const PostArgs<T> *x)
+{
+	const int made = curlMakes(D, h);
+	if (h == 0 && made == 2 && !x && !D->isAux && (D->tf.empty() || D->tf[0].aux->st == D->st) && D->tf.size() < 2) {
+		size_t programs = 0;
+		for (const PostSeg &G : D->post[0]) programs += G.bare > 0;
+		if (programs <= 1) {
+			(void)postArgs<T>(D, 0);             // the curl has applied the recorded operations
+			D->pendPost = programs > 0;
+			return 0;
+		}
+	}
+	if (h == 1 && D->pendPost && !x) {
+		PostArgs<T> e{};
+		for (const PostSeg &G : D->post[0])
+			if (G.bare) e.ops = (const PostOp<T> *)G.ops, e.pieces = (const PostPiece *)G.pieces, e.post = (int)(G.bare / POST_BLK);
+		D->pendPost = false;
+		return postHalf<T>(D, 1, made, &e);
+	}
+	return postHalf<T>(D, h, made, x);
+}
 
 // A half step of D and of its auxiliary world, both waiting: two launches (three with objects, or a
 // main program of several).
@@ -2343,32 +2443,36 @@ int foldedHalf(alis_dev_world *D, int h)
 	dropPresamples(A);
 	if (!A->postBuilt && buildPost<T>(A)) return -1;
 	AuxCurl<T> x{};
-	static_assert(sizeof(HalfArgs<T>) + sizeof x + sizeof(ZFaces<T>) <= 4096 && 2 * sizeof(PostArgs<T>) <= 4096, "kernel arguments");
+	static_assert(sizeof(HalfArgs<T>) + sizeof x + sizeof(AddArgs<T>) + sizeof(ZFaces<T>) <= 4096 && 2 * sizeof(PostArgs<T>) <= 4096, "kernel arguments");
 	x.parts = 1 + A->cplx;
 	for (int m = 0; m <= A->cplx; m++) {
 		x.part[m] = halfArgs<T>(A, h, m);
 		if (m < A->cplx) x.part[m].ends = 0;
 	}
-	x.post = postArgs<T>(A, h);
-	for (size_t g = 0; g + 1 < A->post[h].size(); g++) {
+	for (int m = 0; m <= A->cplx; m++) x.adds[m] = addArgs<T>(A, h, m, true);
+	PostArgs<T> last = postArgs<T>(A, h);               // (its sources are in x.adds)
+	// its copies: in the curl launch too, but for a last program of many cells
+	PostArgs<T> *rest = nullptr;
+	for (size_t g = 0; g < A->post[h].size(); g++) {
 		const PostSeg &G = A->post[h][g];
+		if (!G.bare) continue;
+		if (g + 1 == A->post[h].size() && G.bare > AUX_CELLS) {
+			last.ops = (const PostOp<T> *)G.ops, last.pieces = (const PostPiece *)G.pieces;
+			last.post = (int)(G.bare / POST_BLK), rest = &last;
+			break;
+		}
 		x.seg[x.segs].ops = (const PostOp<T> *)G.ops, x.seg[x.segs].pieces = (const PostPiece *)G.pieces;
-		x.seg[x.segs].n = (int)(G.rest / POST_BLK);
-		if (x.seg[x.segs].n) x.segs++;
+		x.seg[x.segs++].n = (int)(G.bare / POST_BLK);
 	}
 	if (!D->postBuilt && buildPost<T>(D)) return -1;
+	if (rest && postWaiting<T>(D)) return -1;
 	if (coreHalf<T>(D, h, true, &x)) return -1;
-	PostArgs<T> last = x.post;
-	const PostSeg &G = A->post[h].back();
-	last.ops = (const PostOp<T> *)G.ops, last.pieces = (const PostPiece *)G.pieces;
-	last.post = (int)(G.rest / POST_BLK);
-	return postHalf<T>(D, h, true, last.post ? &last : nullptr);
+	return endHalf<T>(D, h, rest);
 }
 
-// Run the end of half step h: the recorded strips and sources, then the ghost copies.
-// copied: the curl has made the copies it can.  x: an auxiliary world's launch to take along, or null.
+// made: what the curl has done of it (curlMakes), or 0.  x: an auxiliary world's launch to take along, or null.
 template<class T>
-int postHalf(alis_dev_world *D, int h, bool copied, const PostArgs<T> *x)
+int postHalf(alis_dev_world *D, int h, int made, const PostArgs<T> *x)
 {
 	if (!D->postBuilt && buildPost<T>(D)) return -1;
 	PostArgs<T> a = postArgs<T>(D, h);
@@ -2384,7 +2488,7 @@ int postHalf(alis_dev_world *D, int h, bool copied, const PostArgs<T> *x)
 	for (size_t s = 0; s < D->tf.size(); s++) bind = bind || sideStream(s);
 	if (bind && !D->halfDone) HIPCHECK(hipEventCreateWithFlags(&D->halfDone, hipEventDisableTiming));
 	int last = -1;
-	auto cells = [&](const PostSeg &G) { return copied ? G.rest : G.total; };
+	auto cells = [&](const PostSeg &G) { return made == 2 ? G.bare : made ? G.rest : G.total; };
 	for (int g = 0; g < (int)D->post[h].size(); g++) if (cells(D->post[h][g])) last = g;
 	for (int g = 0; g <= last; g++) {
 		const PostSeg &G = D->post[h][g];
@@ -2694,6 +2798,7 @@ template<class T>
 int flushStep(alis_dev_world *D)
 {
 	if (D->pendBatch) return batchFlush(D->pendBatch);
+	if (postWaiting<T>(D)) return -1;
 	if (D->pendH && D->mainOf) return flushStep<T>(D->mainOf);
 	if (D->pendCore && D->mainOf) return flushStep<T>(D->mainOf);
 	if (D->pendMain) {
@@ -2735,7 +2840,7 @@ int coreEntry(alis_dev_world *D, int h)
 		D->pendCore = 1 + h;
 		return 0;
 	}
-	if (flushStep<T>(D)) return -1;
+	if (!(h == 1 && D->pendPost) && flushStep<T>(D)) return -1;
 	if (h == 0) {
 		bool on;
 		if (fusedSteps<T>(D, on)) return -1;
@@ -2766,13 +2871,15 @@ int ghostsEntry(alis_dev_world *D, int h)
 	if (D->pendMain == 1 + h && !D->pendFold) {
 		D->pendMain = 0;
 		if (!D->postBuilt && buildPost<T>(D)) return -1;
-		return coreHalf<T>(D, h, true) ? -1 : postHalf<T>(D, h, true);
+		// the strips read the auxiliary worlds' fields in the curl
+		if (waitForAux(D, D->pendStrips[h]) || coreHalf<T>(D, h, true)) return -1;
+		return endHalf<T>(D, h, nullptr);
 	}
 	if (h == 1 && D->pendH == 1) {
 		D->pendH = 2;
 		return 0;
 	}
-	if ((h == 0 || D->pendE || D->pendH || D->pendCore || D->pendMain) && flushStep<T>(D)) return -1;   // (an H program takes its current update along)
+	if ((h == 0 || D->pendE || D->pendH || D->pendCore || D->pendMain || D->pendPost) && flushStep<T>(D)) return -1;   // (an H program takes its current update along)
 	return postHalf<T>(D, h);
 }
 

@@ -17,7 +17,7 @@ LIBS = {"hip": ROOT / "alis_amd" / "libalis_workloads.so", "oracle": ROOT / "ora
 ENGINES = {"hip": ROOT / "alis_amd" / "libalis.so", "oracle": ROOT / "oracle" / "liboracle.so"}
 
 
-def _fields(kind, name, cells, bits, steps, parted=False):
+def _fields(kind, name, cells, bits, steps, parted=None):
     w, e = ctypes.CDLL(str(LIBS[kind])), ctypes.CDLL(str(ENGINES[kind]))
     w.wl_create.restype = w.wl_device.restype = ctypes.c_void_p
     w.wl_create.argtypes = [ctypes.c_char_p] + [ctypes.c_int] * 3
@@ -42,15 +42,18 @@ def _fields(kind, name, cells, bits, steps, parted=False):
         dev = w.wl_device(c)
         for h in range(2):
             assert e.alis_dev_core(dev, h) == 0
-            read(h)
+            if parted == "core":
+                read(h)
             assert e.alis_dev_ghosts(dev, h) == 0
+            if parted == "ghosts":
+                read(0)
         w.wl_step(c, 2)
     read(0), read(1)
     w.wl_free(c)
     return np.concatenate(out)
 
 
-def _agree(name, cells, bits, steps, parted=False):
+def _agree(name, cells, bits, steps, parted=None):
     print(f"[gpu] {name} {cells}^3 fp{bits}", flush=True)
     got, ref = _fields("hip", name, cells, bits, steps, parted), _fields("oracle", name, cells, bits, steps, parted)
     assert got.shape == ref.shape and np.abs(ref).max() > 0
@@ -70,9 +73,10 @@ def test_scatterer_rows(cells, bits):
     _agree("nanoblock", cells, bits, 12)
 
 
-@pytest.mark.parametrize("bits", [32, 64])
-def test_half_step_in_parts(bits):
-    _agree("nanoblock", 109, bits, 8, parted=True)
+@pytest.mark.parametrize("name,cells,bits,parted", [("nanoblock", 109, 32, "core"), ("nanoblock", 109, 64, "core"), ("dipole", 59, 32, "core"),
+                                                    ("dipole", 59, 32, "ghosts"), ("dipole", 60, 64, "ghosts")])
+def test_half_step_in_parts(name, cells, bits, parted):
+    _agree(name, cells, bits, 15, parted)
 
 
 @pytest.mark.parametrize("worlds", [2])
