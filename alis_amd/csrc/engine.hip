@@ -4221,6 +4221,9 @@ __global__ void k_ff_finish(double2 *S, const double2 *part, FFReduce r)
 // (blockIdx.z); each wavefront a 32 x 32 quarter as 2 x 2 tiles of 16 x 16, real and
 // imaginary parts in their own accumulators: Cr += Ar Br - Ai Bi, Ci += Ar Bi + Ai Br.  The
 // k loop stages 16 values of p of A and B in LDS per round (zero beyond the matrix edges).
+// What bounds it: the matrix units, and products with the padding beyond the matrix: 16-row tiles
+// and groups of 4 p that hold nothing of it are left out (321 x 321 x 8192, four matrices: 608 ->
+// 552 us, 49 TFLOP/s of the 65 that a large double-precision product reaches here).
 typedef double v4d __attribute__((ext_vector_type(4)));
 constexpr int FFG_T = 64, FFG_K = 16;
 
@@ -4239,6 +4242,8 @@ __global__ __launch_bounds__(256) void k_ff_gemm(FFGemm g)
 	const int v0 = (int)blockIdx.y * FFG_T, c0 = (int)blockIdx.x * FFG_T;
 	const double2 *A = g.A[m];
 	const int wv = (wave >> 1) * 32, wc = (wave & 1) * 32;
+	// 16-row tiles of the wavefront's quarter that hold rows of the matrix
+	const int na = __builtin_amdgcn_readfirstlane(min(max(g.nv - v0 - wv + 15, 0) / 16, 2));
 	v4d cr[2][2], ci[2][2];
 #pragma unroll
 	for (int a = 0; a < 2; a++)
@@ -4274,8 +4279,10 @@ __global__ __launch_bounds__(256) void k_ff_gemm(FFGemm g)
 		}
 		__syncthreads();
 		if (p0 + FFG_K < g.np) fetch(p0 + FFG_K);
+		const int kn = na ? min(FFG_K, g.np - p0) : 0;       // (past the matrix there are only zeros)
 #pragma unroll
 		for (int ks = 0; ks < FFG_K; ks += 4) {
+			if (ks >= kn) break;
 			const int k = ks + (lane >> 4);
 			double ar[2], ai[2], br[2], bi[2];
 #pragma unroll
@@ -4284,7 +4291,8 @@ __global__ __launch_bounds__(256) void k_ff_gemm(FFGemm g)
 				br[a] = Br[k][wc + 16 * a + (lane & 15)], bi[a] = Bi[k][wc + 16 * a + (lane & 15)];
 			}
 #pragma unroll
-			for (int a = 0; a < 2; a++)
+			for (int a = 0; a < 2; a++) {
+				if (a >= na) break;
 #pragma unroll
 				for (int b = 0; b < 2; b++) {
 					cr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[a], br[b], cr[a][b], 0, 0, 0);
@@ -4292,6 +4300,7 @@ __global__ __launch_bounds__(256) void k_ff_gemm(FFGemm g)
 					ci[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[a], bi[b], ci[a][b], 0, 0, 0);
 					ci[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[a], br[b], ci[a][b], 0, 0, 0);
 				}
+			}
 		}
 		__syncthreads();
 	}
