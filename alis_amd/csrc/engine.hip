@@ -3448,7 +3448,7 @@ int batchBuildPost(alis_dev_batch *B, bool copied)
 
 // copies: the launch makes the ghost copies along z that it can (see coreHalf).
 template<class T>
-int batchCore(alis_dev_batch *B, int h, bool copies)
+int batchCore(alis_dev_batch *B, int h, bool copies, const FetchArgs &next = FetchArgs{}, hipEvent_t fetched = nullptr)
 {
 	if (batchPrograms<T>(B) || (!B->curl[0] && batchBuildCurl<T>(B))) return -1;
 	alis_dev_world *D0 = B->W[0];
@@ -3470,15 +3470,19 @@ int batchCore(alis_dev_batch *B, int h, bool copies)
 		const alis_dev_batch::CurlClass &c = cls[q];
 		const HalfArgs<T> *args = (const HalfArgs<T> *)B->curl[h] + c.arg;
 		const int *start = (const int *)B->curlStart[h] + c.first;
-		const dim3 grid(c.blocks), block(CURL_WG);
+		const FetchArgs fetch = q == 0 ? next : FetchArgs{};
+		const dim3 grid(c.blocks + fetch.blocks), block(CURL_WG);
 		hipEvent_t s0 = q == 0 ? e0 : nullptr, s1 = q + 1 == cls.size() ? e1 : nullptr;
-#define CURL_BATCH(H, C) (c.pair ? launchEv(k_curl_batch<T, H, C, true>, grid, block, 0, B->st, s0, s1, args, start, c.n, (int)copies) : launchEv(k_curl_batch<T, H, C, false>, grid, block, 0, B->st, s0, s1, args, start, c.n, (int)copies))
+		const bool bind = q == 0 && !s1;                 // `fetched`: the end of this launch
+		if (bind) s1 = fetched;
+#define CURL_BATCH(H, C) (c.pair ? launchEv(k_curl_batch<T, H, C, true>, grid, block, 0, B->st, s0, s1, args, start, c.n, (int)copies, fetch) : launchEv(k_curl_batch<T, H, C, false>, grid, block, 0, B->st, s0, s1, args, start, c.n, (int)copies, fetch))
 		if (h == 1) CURL_BATCH(1, 0);
 		else if (c.cm == 2) CURL_BATCH(0, 2);
 		else if (c.cm == 1) CURL_BATCH(0, 1);
 		else CURL_BATCH(0, 0);
 #undef CURL_BATCH
 		HIPCHECK(hipGetLastError());
+		if (q == 0 && fetched && !bind) HIPCHECK(hipEventRecord(fetched, B->st));
 	}
 	if (e1) {
 		D0->evPairs[h].push_back(e0);
@@ -3487,13 +3491,15 @@ int batchCore(alis_dev_batch *B, int h, bool copies)
 	return 0;
 }
 
+// The arguments of the end of half step h into pinned memory; whole: the current update of H is one of
+// them although its core is still to come.
 template<class T>
-int batchPost(alis_dev_batch *B, int h, bool copied)
+int batchPostArgs(alis_dev_batch *B, int h, bool whole)
 {
-	if (batchPrograms<T>(B) || (!B->postReady[copied] && batchBuildPost<T>(B, copied))) return -1;
-	if (!B->postBytes[copied][h]) return 0;
-	HIPCHECK(hipEventSynchronize(B->postDone[copied][h]));
-	for (alis_dev_batch::Round &R : B->rounds[copied][h]) {
+	if (batchPrograms<T>(B) || (!B->postReady[whole] && batchBuildPost<T>(B, whole))) return -1;
+	if (!B->postBytes[whole][h]) return 0;
+	HIPCHECK(hipEventSynchronize(B->postDone[whole][h]));
+	for (alis_dev_batch::Round &R : B->rounds[whole][h]) {
 		if (R.world.empty()) continue;
 		PostArgs<T> *a = (PostArgs<T> *)R.pinned;
 		for (size_t e = 0; e < R.world.size(); e++) {
@@ -3502,18 +3508,34 @@ int batchPost(alis_dev_batch *B, int h, bool copied)
 			memset(&a[e], 0, sizeof(PostArgs<T>));
 			a[e].ops = (const PostOp<T> *)g.ops;
 			a[e].pieces = (const PostPiece *)g.pieces;
-			a[e].post = (int)((copied ? g.rest : g.total) / POST_BLK);
-			if (h == 1 && R.seg[e] + 1 == (int)D->post[h].size() && D->pendAde) a[e].ade = objArgs<T>(D), D->pendAde = false;
+			a[e].post = (int)((whole ? g.rest : g.total) / POST_BLK);
+			if (h == 1 && R.seg[e] + 1 == (int)D->post[h].size() && (whole ? D->objWgs > 0 : D->pendAde)) a[e].ade = objArgs<T>(D);
 			a[e].strips = D->pendStrips[h];
 			for (size_t w = 0; w < D->pendSrc[h].size(); w++) a[e].src[w] = D->pendSrc[h][w];
 			for (size_t q = 0; q < D->pendWave[h].size(); q++) a[e].wave[q] = (T)D->pendWave[h][q];
 		}
 	}
-	fetchArgs(B->postArgs[copied][h], B->postPinned[copied][h], B->postBytes[copied][h], B->st, B->postDone[copied][h]);
-	for (alis_dev_batch::Round &R : B->rounds[copied][h]) {
+	return 0;
+}
+
+// The end of half step h; whole: with its core, in whose launch the arguments of the end are fetched.
+template<class T>
+int batchPost(alis_dev_batch *B, int h, bool whole)
+{
+	if (batchPostArgs<T>(B, h, whole)) return -1;
+	const size_t bytes = B->postBytes[whole][h];
+	if (whole) {
+		FetchArgs next{};
+		if (bytes) next = FetchArgs{(unsigned *)B->postArgs[whole][h], (const unsigned *)B->postPinned[whole][h], (int)(bytes / 4), std::max(1, std::min(64, (int)(bytes / 4096)))};
+		if (batchCore<T>(B, h, true, next, bytes ? B->postDone[whole][h] : nullptr)) return -1;
+	}
+	else if (bytes) fetchArgs(B->postArgs[whole][h], B->postPinned[whole][h], bytes, B->st, B->postDone[whole][h]);
+	for (alis_dev_batch::Round &R : B->rounds[whole][h]) {
 		if (R.world.empty()) continue;
 		k_post_batch<T><<<R.blocks, POST_WG, 0, B->st>>>((const PostArgs<T> *)R.args, (const int *)R.start, (int)R.world.size());
 		HIPCHECK(hipGetLastError());
+		for (size_t e = 0; e < R.world.size(); e++)
+			if (h == 1 && ((const PostArgs<T> *)R.pinned)[e].ade.blocks) B->W[R.world[e]]->pendAde = false;
 	}
 	for (alis_dev_world *D : B->W) {
 		if (h == 1 && flushAde<T>(D)) return -1;     // a world without an H program
@@ -4518,7 +4540,6 @@ int alis_dev_batch_post(alis_dev_batch *B, int h)
 	if (whole) {
 		B->pend = 0;
 		for (alis_dev_world *W : B->W) W->pendBatch = nullptr;
-		if (B->fp64 ? batchCore<double>(B, h, true) : batchCore<float>(B, h, true)) return -1;
 	}
 	else for (alis_dev_world *W : B->W) if (W->pendBatch && flushE(W)) return -1;
 	return B->fp64 ? batchPost<double>(B, h, whole) : batchPost<float>(B, h, whole);
