@@ -382,35 +382,44 @@ template<class T> struct PhsArgs {
 	int q0, nq;                 // the launch's frequencies (of the accumulators)
 };
 
-// The sampled fields of face cell t of a phaser: the two tangential E components and the two
-// sums of the tangential H components across the face (src/phaser.c:83-110).
-template<class T>
-__device__ __forceinline__ void phaserFields(const PhsArgs<T> &a, long t, T &e1, T &e2, T &h1, T &h2)
+constexpr int PHS_WG = 64;      // face cells (threads) per workgroup of a sampling launch
+
+// Workgroups of a sampling launch: faces start on workgroup boundaries.
+template<class A>
+__host__ __device__ inline long faceCells(const A &a, int f) { return (f + 1 < a.nface ? a.face[f + 1].off : a.ncell) - a.face[f].off; }
+template<class A>
+__host__ inline int sampleBlocks(const A &a)
+{
+	long n = 0;
+	for (int f = 0; f < a.nface; f++) n += (faceCells(a, f) + PHS_WG - 1) / PHS_WG;
+	return (int)n;
+}
+
+// Workgroup blk of such a launch: of each of its face cells the two tangential E components and the
+// two sums of the tangential H components across the face (src/phaser.c:83-110) into slot
+// [4][cell], but of cells the H curl has sampled.  What bounds it: the latency of one chain
+// (face, cell's place, fields), so a workgroup lies in one face, whose description is scalar, and divides
+// in 32 bits (14 600 face cells 6.4 -> 4.7 us, 104 000 in a batch 8.0 -> 6.9).
+template<class T, class A>
+__device__ __forceinline__ void sampleBlock(const A &a, int blk, T *slot)
 {
 	int f = 0;
-	while (f + 1 < a.nface && t >= a.face[f + 1].off) f++;
-	const PhsFaceGeom &g = a.face[f];
-	long local = t - g.off;
-	int u = (int)(local / g.n2), v = (int)(local % g.n2);
-	int i, j, k;
-	if (g.kind < 2) {
-		i = g.fixed, j = a.jMin + u, k = a.kMin + v;
-		long id = a.L.at(i, j, k), s = a.L.si;
-		e1 = a.E[1][id], e2 = a.E[2][id];
-		h1 = a.H[1][id] + a.H[1][id + s], h2 = a.H[2][id] + a.H[2][id + s];
+	for (; f + 1 < a.nface; f++) {
+		const int blocks = (int)((faceCells(a, f) + PHS_WG - 1) / PHS_WG);
+		if (blk < blocks) break;
+		blk -= blocks;
 	}
-	else if (g.kind < 4) {
-		i = a.iMin + u, j = g.fixed, k = a.kMin + v;
-		long id = a.L.at(i, j, k), s = a.L.sj;
-		e1 = a.E[2][id], e2 = a.E[0][id];
-		h1 = a.H[2][id] + a.H[2][id + s], h2 = a.H[0][id] + a.H[0][id + s];
-	}
-	else {
-		i = a.iMin + u, j = a.jMin + v, k = g.fixed;
-		long id = a.L.at(i, j, k);
-		e1 = a.E[0][id], e2 = a.E[1][id];
-		h1 = a.H[0][id] + a.H[0][id + 1], h2 = a.H[1][id] + a.H[1][id + 1];
-	}
+	const auto &g = a.face[f];
+	const unsigned local = (unsigned)blk * PHS_WG + threadIdx.x;
+	if (local >= faceCells(a, f)) return;
+	const int u = (int)(local / (unsigned)g.n2), v = (int)(local % (unsigned)g.n2), axis = g.kind / 2;
+	const int i = axis == 0 ? g.fixed : a.iMin + u, j = axis == 1 ? g.fixed : a.jMin + (axis == 0 ? u : v), k = axis == 2 ? g.fixed : a.kMin + v;
+	if (axis == 2 && i >= g.si0 && i <= g.si1 && j >= g.sj0 && j <= g.sj1) return;
+	const long id = layAt(a.L, i, j, k), s = axis == 0 ? a.L.si : axis == 1 ? a.L.sj : 1, t = g.off + local;
+	const int c1 = axis == 2 ? 0 : axis + 1, c2 = axis == 0 ? 2 : axis == 1 ? 0 : 1;
+	const T e1 = glb(a.E[c1])[id], e2 = glb(a.E[c2])[id];
+	const T p1 = glb(a.H[c1])[id], q1 = glb(a.H[c1])[id + s], p2 = glb(a.H[c2])[id], q2 = glb(a.H[c2])[id + s];
+	glb(slot)[t] = e1, glb(slot)[a.ncell + t] = e2, glb(slot)[2 * a.ncell + t] = p1 + q1, glb(slot)[3 * a.ncell + t] = p2 + q2;
 }
 
 // Workgroup w of a one-dimensional phaser grid of ny frequency blocks per cell block: the
@@ -427,23 +436,9 @@ __device__ inline void phaserBlock(int w, int ny, int &xb, int &yb)
 // a flush adds the pending samples to the accumulators in sample order, the same additions as
 // one immediate update per sample, reading and writing the accumulators once for all of them.
 template<class T>
-__global__ __launch_bounds__(256) void k_phs_sample(PhsArgs<T> a, T *__restrict__ slot, long n)
+__global__ __launch_bounds__(PHS_WG) void k_phs_sample(PhsArgs<T> a, T *__restrict__ slot)
 {
-	const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (t >= n) return;
-	{
-		int f = 0;
-		while (f + 1 < a.nface && t >= a.face[f + 1].off) f++;
-		const PhsFaceGeom &g = a.face[f];
-		if (g.kind >= 4 && g.si0 <= g.si1) {        // cells the H curl sampled
-			const long local = t - g.off;
-			const int i = a.iMin + (int)(local / g.n2), j = a.jMin + (int)(local % g.n2);
-			if (i >= g.si0 && i <= g.si1 && j >= g.sj0 && j <= g.sj1) return;
-		}
-	}
-	T e1, e2, h1, h2;
-	phaserFields(a, t, e1, e2, h1, h2);
-	slot[t] = e1, slot[a.ncell + t] = e2, slot[2 * a.ncell + t] = h1, slot[3 * a.ncell + t] = h2;
+	sampleBlock<T>(a, (int)blockIdx.x, slot);
 }
 
 // s += y with Neumaier's compensation (Neumaier 1974, the improved Kahan-Babuska sum): c
@@ -533,17 +528,11 @@ __global__ __launch_bounds__(256) void k_phs_flush(PhsArgs<T> a, const T *__rest
 // The same for several phasers (of several worlds) in one launch each: the samples of every
 // entry (acc: its ring slot), and the flushes of the entries whose ring is full.
 template<class T>
-__global__ __launch_bounds__(256) void k_phs_sample_batch(const PhsArgs<T> *__restrict__ args, const int *__restrict__ start, int n)
+__global__ __launch_bounds__(PHS_WG) void k_phs_sample_batch(const PhsArgs<T> *__restrict__ args, const int *__restrict__ start, int n)
 {
-	const int b = (int)blockIdx.x;
-	const int e = batchEntry(start, n, b);
-	const PhsArgs<T> &a = args[e];
-	const long t = (long)(b - start[e]) * 256 + threadIdx.x;
-	if (t >= a.ncell) return;
-	T e1, e2, h1, h2;
-	phaserFields(a, t, e1, e2, h1, h2);
-	T *slot = (T *)a.acc;
-	slot[t] = e1, slot[a.ncell + t] = e2, slot[2 * a.ncell + t] = h1, slot[3 * a.ncell + t] = h2;
+	const int b = (int)blockIdx.x, e = batchEntry(start, n, b);
+	const auto &a = uniform(args)[e];
+	sampleBlock<T>(a, b - uniform(start)[e], (T *)a.acc);
 }
 
 template<class T> struct PhsFlush {
@@ -3149,7 +3138,7 @@ int phaserUpdate(alis_dev_world *D, DevPhaser &P, int qa, int qn, const double *
 	const bool pre = P.pre && P.preSlot == P.pend;   // the H curl stored the z faces' inner cells
 	P.pre = false;
 	for (int f = 0; !pre && f < a.nface; f++) a.face[f].si0 = 1, a.face[f].si1 = 0;
-	k_phs_sample<T><<<blocksFor(P.ncell), 256, 0, D->st>>>(a, (T *)P.ring + (size_t)P.pend * 4 * P.ncell, P.ncell);
+	k_phs_sample<T><<<sampleBlocks(a), PHS_WG, 0, D->st>>>(a, (T *)P.ring + (size_t)P.pend * 4 * P.ncell);
 	HIPCHECK(hipGetLastError());
 	double *x = P.exPinned + (size_t)P.pend * 4 * qn;
 	for (int q = 0; q < qn; q++)
@@ -3207,9 +3196,10 @@ int phaserBatchUpdate(alis_dev_world *L, alis_dev_world *const *D, const int *id
 		P.pre = false;              // this path samples every face itself
 		PhsArgs<T> a = phaserArgs<T>(D[e], P, q0[e], nq[e]);
 		a.acc = (T *)P.ring + (size_t)P.pend * 4 * P.ncell;
+		for (int f = 0; f < a.nface; f++) a.face[f].si0 = 1, a.face[f].si1 = 0;
 		sa.push_back(a);
 		sstart.push_back(sblocks);
-		sblocks += (int)blocksFor(P.ncell);
+		sblocks += sampleBlocks(a);
 		double *x = P.exPinned + (size_t)P.pend * 4 * P.pnq;
 		for (int q = 0; q < nq[e]; q++)
 			x[4 * q] = expE[e][2 * q], x[4 * q + 1] = expE[e][2 * q + 1], x[4 * q + 2] = expH[e][2 * q], x[4 * q + 3] = expH[e][2 * q + 1];
@@ -3222,7 +3212,7 @@ int phaserBatchUpdate(alis_dev_world *L, alis_dev_world *const *D, const int *id
 		memcpy(L->phsStage.pinned, sa.data(), sa.size() * sizeof(PhsArgs<T>));
 		memcpy((char *)L->phsStage.pinned + ab, sstart.data(), sstart.size() * sizeof(int));
 		fetchArgs(L->phsStage.dev, L->phsStage.pinned, bytes, L->st, L->phsStage.done);
-		k_phs_sample_batch<T><<<sblocks, 256, 0, L->st>>>((const PhsArgs<T> *)L->phsStage.dev, (const int *)((char *)L->phsStage.dev + ab), (int)sa.size());
+		k_phs_sample_batch<T><<<sblocks, PHS_WG, 0, L->st>>>((const PhsArgs<T> *)L->phsStage.dev, (const int *)((char *)L->phsStage.dev + ab), (int)sa.size());
 		HIPCHECK(hipGetLastError());
 	}
 	if (full.empty()) return 0;
