@@ -94,7 +94,7 @@ template<class T> struct ObjDev {
 	T *J[2][3][MAXPOLE], *K[2][3][MAXPOLE];
 };
 
-// A z face of a phaser whose samples the H curl stores (k_curl, ROWS): of the face (i0..i1,
+// A z face of a phaser whose samples the H curl stores (ZS): of the face (i0..i1,
 // j0..j1) at k, the cells (si0..si1, sj0..sj1), at their places from `base` in the ring slot
 // [4][cells] (E x, E y, H x(k) + H x(k+1), H y(k) + H y(k+1)), as k_phs_sample stores them.
 template<class T> struct PhsZ {
@@ -362,6 +362,7 @@ struct PhsFaceGeom {
 	long off;                   // first cell of this face in the concatenated cell list
 	int si0, si1, sj0, sj1;     // z faces: cells (i, j) the H curl sampled (k_phs_sample skips
 	                            // them), none when si0 > si1
+	int pq = 0, q0 = 0;         // but not those with (j pq + q0) % 64 = 63, where pq is not 0
 };
 
 constexpr int PHS_QPT = 4;      // frequencies per thread (measured: 1 < 2 < 4)
@@ -414,7 +415,7 @@ __device__ __forceinline__ void sampleBlock(const A &a, int blk, T *slot)
 	if (local >= faceCells(a, f)) return;
 	const int u = (int)(local / (unsigned)g.n2), v = (int)(local % (unsigned)g.n2), axis = g.kind / 2;
 	const int i = axis == 0 ? g.fixed : a.iMin + u, j = axis == 1 ? g.fixed : a.jMin + (axis == 0 ? u : v), k = axis == 2 ? g.fixed : a.kMin + v;
-	if (axis == 2 && i >= g.si0 && i <= g.si1 && j >= g.sj0 && j <= g.sj1) return;
+	if (axis == 2 && i >= g.si0 && i <= g.si1 && j >= g.sj0 && j <= g.sj1 && !(g.pq && (j * g.pq + g.q0) % 64 == 63)) return;
 	const long id = layAt(a.L, i, j, k), s = axis == 0 ? a.L.si : axis == 1 ? a.L.sj : 1, t = g.off + local;
 	const int c1 = axis == 2 ? 0 : axis + 1, c2 = axis == 0 ? 2 : axis == 1 ? 0 : 1;
 	const T e1 = glb(a.E[c1])[id], e2 = glb(a.E[c2])[id];
@@ -1741,12 +1742,12 @@ void dropPresamples(alis_dev_world *D)
 	for (DevPhaser &P : D->phs) P.pre = false;
 }
 
-// The z faces of D's phasers that the H curl can sample (PhsZ): a face whose k + 1 lies in
-// the same quad as k, over the rectangle of
-// its cells that the end-of-H-half program leaves alone at k and k + 1 (shrunk from the edges
+// The z faces of D's phasers that the H curl can sample (PhsZ): over the rectangle of the face's cells that the end-of-H-half program leaves alone at k and k + 1 (shrunk from the edges
 // its boxes reach: the ghost planes of periodic boundaries), so the values the curl has are
-// the ones the phaser update would read; k_phs_sample samples the other cells.
-// fused: by k_step, which applies the strips and sources itself, so only the ghost copies count.
+// the ones the phaser update would read; k_phs_sample samples the other cells (and, where k + 1 lies
+// in the next quad, those of a wavefront's last lane).
+// fused: by k_step, which applies the strips and sources itself, so only the ghost copies count; a
+// face whose k + 1 lies in the next quad is left out.
 template<class T>
 int zSamples(alis_dev_world *D, PhsZ<T> *zs, std::vector<DevPhaser *> &owners, bool fused)
 {
@@ -1761,7 +1762,7 @@ int zSamples(alis_dev_world *D, PhsZ<T> *zs, std::vector<DevPhaser *> &owners, b
 			const PhsFaceGeom &g = P.face[f];
 			if (g.kind < 4) continue;
 			const int k = g.fixed;
-			if ((k - D->kMIN) % reach == reach - 1 || k + 1 > D->kMAX || n == MAXZS) { ok = false; break; }
+			if ((fused && (k - D->kMIN) % reach == reach - 1) || k + 1 > D->kMAX || n == MAXZS) { ok = false; break; }
 			int i0 = P.iMin, i1 = P.iMax, j0 = P.jMin, j1 = P.jMax;
 			for (const Box &b : fused ? D->hCopies : D->hWrites) {
 				if (b.k1 < k || b.k0 > k + 1 || b.i1 < i0 || b.i0 > i1 || b.j1 < j0 || b.j0 > j1) continue;
@@ -1784,6 +1785,9 @@ int zSamples(alis_dev_world *D, PhsZ<T> *zs, std::vector<DevPhaser *> &owners, b
 			PhsFaceGeom &g = P.face[f];
 			if (g.kind < 4) continue;
 			g.si0 = zs[z].si0, g.si1 = zs[z].si1, g.sj0 = zs[z].sj0, g.sj1 = zs[z].sj1;
+			g.pq = 0;
+			if ((g.fixed - D->kMIN) % reach == reach - 1)
+				g.pq = (int)(D->L.sj / reach), g.q0 = (g.fixed - D->kMIN) / reach - D->jMIN * g.pq;
 			z++;
 		}
 		owners.push_back(&P);

@@ -146,3 +146,30 @@ def test_whole_sync_over_many_chunks(bits):
     assert sums["oracle"][0] > 0
     for got, ref in zip(sums["hip"], sums["oracle"]):
         assert got == ref if bits == 32 else abs(got - ref) <= 1e-7 * ref
+
+
+@pytest.mark.parametrize("cells,bits", [(108, 32), (109, 32), (110, 32), (111, 32), (109, 64), (110, 64)])
+def test_face_samples_of_the_curl(cells, bits, monkeypatch):
+    """A phaser's z faces at every place of a quad, sampled by the H curl (the pair across the face in one
+    quad, in the next lane's, or in the next wavefront's) and by k_phs_sample: the same accumulators."""
+    w, e = ctypes.CDLL(str(LIBS["hip"])), ctypes.CDLL(str(ENGINES["hip"]))
+    w.wl_create.restype = w.wl_device.restype = ctypes.c_void_p
+    w.wl_create.argtypes = [ctypes.c_char_p] + [ctypes.c_int] * 3
+    w.wl_step.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    w.wl_device.argtypes = w.wl_free.argtypes = [ctypes.c_void_p]
+    e.alis_dev_phaser_size.restype = ctypes.c_long
+    e.alis_dev_phaser_size.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    e.alis_dev_phaser_read.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.POINTER(ctypes.c_double), ctypes.c_long]
+    got = []
+    for mode in ("force", "0"):
+        monkeypatch.setenv("ALIS_PRESAMPLE", mode)
+        c = w.wl_create(b"nanoblock", cells, bits, 64)
+        w.wl_step(c, 40)
+        dev = w.wl_device(c)
+        n = e.alis_dev_phaser_size(dev, 0)
+        assert n > 0
+        out = np.zeros(n)
+        assert e.alis_dev_phaser_read(dev, 0, out.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), n) == 0
+        w.wl_free(c)
+        got.append(out)
+    assert np.abs(got[0]).max() > 0 and np.array_equal(got[0], got[1])
