@@ -2876,27 +2876,30 @@ int ghostsEntry(alis_dev_world *D, int h)
 	return postHalf<T>(D, h);
 }
 
-// Pinned chunks and their events for mirrorAll, two per thread: 32 MiB, shared by all worlds, one
-// call at a time, given back with the last world.
+// Pinned chunks and their events for mirrorAll, two per thread, made as calls need them: 32 MiB at most,
+// shared by all worlds, one call at a time, given back with the last world.
 struct MirrorStage {
 	std::mutex lock;
-	float *pinned = nullptr;
+	float *pinned[2 * MIRROR_THREADS] = {};
 	hipEvent_t done[2 * MIRROR_THREADS] = {};
 	int worlds = 0;
 
-	bool ready()
+	// The first of each thread's chunks, and the second where there are more chunks than threads.
+	bool ready(int threads, long chunks)
 	{
-		if (pinned) return true;
-		bool ok = hipHostMalloc((void **)&pinned, 2 * MIRROR_THREADS * MIRROR_CHUNK * sizeof(float), hipHostMallocDefault) == hipSuccess;
-		for (hipEvent_t &e : done) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+		bool ok = true;
+		for (int x = 0; x < 2 * threads && ok; x++) {
+			if (x % 2 && chunks <= threads) continue;
+			ok = (pinned[x] || hipHostMalloc((void **)&pinned[x], MIRROR_CHUNK * sizeof(float), hipHostMallocDefault) == hipSuccess)
+			     && (done[x] || hipEventCreateWithFlags(&done[x], hipEventDisableTiming) == hipSuccess);
+		}
 		if (!ok) clear(), (void)hipGetLastError();
 		return ok;
 	}
 	void clear()
 	{
-		if (pinned) (void)hipHostFree(pinned);
+		for (float *&p : pinned) if (p) (void)hipHostFree(p), p = nullptr;
 		for (hipEvent_t &e : done) if (e) (void)hipEventDestroy(e), e = nullptr;
-		pinned = nullptr;
 	}
 	void hold(int n)
 	{
@@ -2918,7 +2921,7 @@ hipError_t mirrorChunks(int device, hipStream_t st, const MirrorSeg<T> *seg, con
 	auto length = [&](long c) { return std::min(MIRROR_CHUNK, total - c * MIRROR_CHUNK); };
 	auto launch = [&](long c, int x) {
 		if (c >= chunks || e != hipSuccess) return;
-		float *const dst = g_mirror.pinned + (2 * t + x) * MIRROR_CHUNK;
+		float *const dst = g_mirror.pinned[2 * t + x];
 		k_mirror<T><<<blocksFor(length(c), 1024), 256, 0, st>>>(seg, (int)out.size(), c * MIRROR_CHUNK, length(c), dst);
 		e = hipGetLastError();
 		if (e == hipSuccess) e = hipEventRecord(g_mirror.done[2 * t + x], st);
@@ -2929,7 +2932,7 @@ hipError_t mirrorChunks(int device, hipStream_t st, const MirrorSeg<T> *seg, con
 		launch(c + threads, x ^ 1);
 		if (e == hipSuccess) e = hipEventSynchronize(g_mirror.done[2 * t + x]);
 		if (e != hipSuccess) break;
-		const float *v = g_mirror.pinned + (2 * t + x) * MIRROR_CHUNK;
+		const float *v = g_mirror.pinned[2 * t + x];
 		const long a = c * MIRROR_CHUNK, b = a + length(c);
 		size_t s = std::upper_bound(out.begin(), out.end(), a, [](long p, const MirrorHost &h) { return p < h.off; }) - out.begin() - 1;
 		for (; s < out.size() && out[s].off < b; s++) {
@@ -2946,7 +2949,6 @@ int mirrorAll(alis_dev_world *D, bool &done)
 {
 	done = false;
 	std::lock_guard<std::mutex> guard(g_mirror.lock);
-	if (!g_mirror.ready()) return 0;
 	const alis_dev_world_desc *W = &D->W;
 	std::vector<MirrorSeg<T>> seg;
 	std::vector<MirrorHost> out;
@@ -2978,13 +2980,14 @@ int mirrorAll(alis_dev_world *D, bool &done)
 			for (int m = 0; m <= D->cplx; m++)
 				for (int q = 0; q < 2; q++) take(S.p[m][q], S.L, S.b, hostBlock(W->slab[h][m][f][q], S.b));
 		}
+	const long chunks = (total + MIRROR_CHUNK - 1) / MIRROR_CHUNK;
+	const int threads = (int)std::min<long>(std::min<long>(MIRROR_THREADS, std::max(1u, std::thread::hardware_concurrency())), chunks);
+	if (!g_mirror.ready(threads, chunks)) return 0;
 	const size_t table = seg.size() * sizeof(MirrorSeg<T>);
 	if (ensureScratch(D, (long)((table + sizeof(double) - 1) / sizeof(double)))) return -1;
 	HIPCHECK(hipMemcpyAsync(D->scratch, seg.data(), table, hipMemcpyHostToDevice, D->st));
 	int device = 0;
 	HIPCHECK(hipGetDevice(&device));
-	const long chunks = (total + MIRROR_CHUNK - 1) / MIRROR_CHUNK;
-	const int threads = (int)std::min<long>(std::min<long>(MIRROR_THREADS, std::max(1u, std::thread::hardware_concurrency())), chunks);
 #ifdef MADV_POPULATE_WRITE
 	// Fresh host arrays: their pages in one call, where the copying threads would fault them in one by
 	// one and wait for each other (400x400x200, first sync with its world's first pass: 980 ms by
