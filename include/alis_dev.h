@@ -103,9 +103,9 @@ void alis_dev_release(alis_dev_world *D);
  * batch): the E half step and the H core are deferred, and the H half's alis_dev_ghosts runs
  * both halves in one pass over the grid (k_step, strips and sources included) followed by the
  * ghost copies; the results are those of the separate half steps, bit for bit.
- * A world with one TF/SF box whose auxiliary world is small defers the core of a half step, and
- * the auxiliary world its whole half step, to its own alis_dev_ghosts, which runs both in the
- * same launches.
+ * Otherwise the core waits for the alis_dev_ghosts of its half step, whose work its launch shares
+ * (ghost copies, sources, the half step of a small TF/SF auxiliary world), and E's last ghost
+ * copies may wait for H's.  Errors of what waits come from the call that runs it.
  * Any other call on the world (or on a world that reads it) first completes what is deferred
  * the separate way. */
 int alis_dev_core(alis_dev_world *D, int h);
