@@ -3297,6 +3297,9 @@ struct alis_dev_batch {
 	void *objArgs = nullptr, *objStart = nullptr;   // ObjArgs<T>[] of the worlds with objects
 	int objEntries = 0, objBlocks = 0;
 	int pend = 0;               // 1 + h: the core of half step h waits for its post
+	// ALIS_BATCH_PAIRS=0 with Bloch worlds: their parts are entries of one launch, side by side, and a
+	// ghost copy between the parts reads and writes both, so the curls make none
+	bool apart = false;
 	bool postReady[2] = {false, false};
 	struct Round {
 		std::vector<int> world;     // index into W
@@ -3341,14 +3344,11 @@ int batchBuildCurl(alis_dev_batch *B)
 	for (int h = 0; h < 2; h++) {
 		// an entry: one part of a world, or both parts of a Bloch world (pair)
 		struct Entry { HalfArgs<T> a[2]; int cls; };
-		const char *pe = getenv("ALIS_BATCH_PAIRS");
-		const bool pairs = !(pe && !strcmp(pe, "0"));
 		std::vector<Entry> all;
 		for (alis_dev_world *D : B->W) {
-			const bool pair = pairs && D->cplx;
+			const bool pair = D->cplx && !B->apart;
 			for (int m = 0; m <= D->cplx; m++) {
 				HalfArgs<T> a = halfArgs<T>(D, h, m);
-				if (!pair && m < D->cplx) a.ends = 0;        // the imaginary part's entry makes both parts' copies
 				// 1/eps: 2 per-segment table (and arrays where a segment is mixed), 1 arrays, 0 none
 				const int cm = a.seg ? 2 : a.C[0] ? 1 : 0;
 				if (pair && m == 1) all.back().a[1] = a;
@@ -3505,14 +3505,14 @@ int batchCore(alis_dev_batch *B, int h, bool copies, const FetchArgs &next = Fet
 }
 
 // The arguments of the end of half step h into pinned memory; whole: the current update of H is one of
-// them although its core is still to come.
+// them although its core is still to come; copied: the curl makes the copies that it can.
 template<class T>
-int batchPostArgs(alis_dev_batch *B, int h, bool whole)
+int batchPostArgs(alis_dev_batch *B, int h, bool whole, bool copied)
 {
-	if (batchPrograms<T>(B) || (!B->postReady[whole] && batchBuildPost<T>(B, whole))) return -1;
-	if (!B->postBytes[whole][h]) return 0;
-	HIPCHECK(hipEventSynchronize(B->postDone[whole][h]));
-	for (alis_dev_batch::Round &R : B->rounds[whole][h]) {
+	if (batchPrograms<T>(B) || (!B->postReady[copied] && batchBuildPost<T>(B, copied))) return -1;
+	if (!B->postBytes[copied][h]) return 0;
+	HIPCHECK(hipEventSynchronize(B->postDone[copied][h]));
+	for (alis_dev_batch::Round &R : B->rounds[copied][h]) {
 		if (R.world.empty()) continue;
 		PostArgs<T> *a = (PostArgs<T> *)R.pinned;
 		for (size_t e = 0; e < R.world.size(); e++) {
@@ -3521,7 +3521,7 @@ int batchPostArgs(alis_dev_batch *B, int h, bool whole)
 			memset(&a[e], 0, sizeof(PostArgs<T>));
 			a[e].ops = (const PostOp<T> *)g.ops;
 			a[e].pieces = (const PostPiece *)g.pieces;
-			a[e].post = (int)((whole ? g.rest : g.total) / POST_BLK);
+			a[e].post = (int)((copied ? g.rest : g.total) / POST_BLK);
 			if (h == 1 && R.seg[e] + 1 == (int)D->post[h].size() && (whole ? D->objWgs > 0 : D->pendAde)) a[e].ade = objArgs<T>(D);
 			a[e].strips = D->pendStrips[h];
 			for (size_t w = 0; w < D->pendSrc[h].size(); w++) a[e].src[w] = D->pendSrc[h][w];
@@ -3535,15 +3535,16 @@ int batchPostArgs(alis_dev_batch *B, int h, bool whole)
 template<class T>
 int batchPost(alis_dev_batch *B, int h, bool whole)
 {
-	if (batchPostArgs<T>(B, h, whole)) return -1;
-	const size_t bytes = B->postBytes[whole][h];
+	const bool copied = whole && !B->apart;
+	if (batchPostArgs<T>(B, h, whole, copied)) return -1;
+	const size_t bytes = B->postBytes[copied][h];
 	if (whole) {
 		FetchArgs next{};
-		if (bytes) next = FetchArgs{(unsigned *)B->postArgs[whole][h], (const unsigned *)B->postPinned[whole][h], (int)(bytes / 4), std::max(1, std::min(64, (int)(bytes / 4096)))};
-		if (batchCore<T>(B, h, true, next, bytes ? B->postDone[whole][h] : nullptr)) return -1;
+		if (bytes) next = FetchArgs{(unsigned *)B->postArgs[copied][h], (const unsigned *)B->postPinned[copied][h], (int)(bytes / 4), std::max(1, std::min(64, (int)(bytes / 4096)))};
+		if (batchCore<T>(B, h, copied, next, bytes ? B->postDone[copied][h] : nullptr)) return -1;
 	}
-	else if (bytes) fetchArgs(B->postArgs[whole][h], B->postPinned[whole][h], bytes, B->st, B->postDone[whole][h]);
-	for (alis_dev_batch::Round &R : B->rounds[whole][h]) {
+	else if (bytes) fetchArgs(B->postArgs[copied][h], B->postPinned[copied][h], bytes, B->st, B->postDone[copied][h]);
+	for (alis_dev_batch::Round &R : B->rounds[copied][h]) {
 		if (R.world.empty()) continue;
 		k_post_batch<T><<<R.blocks, POST_WG, 0, B->st>>>((const PostArgs<T> *)R.args, (const int *)R.start, (int)R.world.size());
 		HIPCHECK(hipGetLastError());
@@ -4509,7 +4510,9 @@ int alis_dev_batch_create(alis_dev_world *const *D, int n, alis_dev_batch **out)
 	alis_dev_batch *B = new alis_dev_batch;
 	B->W.assign(D, D + n);
 	B->fp64 = D[0]->fp64;
+	const char *pairs = getenv("ALIS_BATCH_PAIRS");
 	for (int w = 0; w < n; w++) {
+		if (D[w]->cplx && pairs && !strcmp(pairs, "0")) B->apart = true;
 		if (D[w]->fp64 != B->fp64) { delete B; return fail("worlds of one batch must share their precision"); }
 		for (int v = 0; v < w; v++) if (D[v] == D[w]) { delete B; return fail("a world appears twice in a batch"); }
 		if (joinStream(D[w], D[0])) { delete B; return -1; }

@@ -1,0 +1,64 @@
+/*
+ * Worlds for the tests that call the engine ABI directly (test_engine_calls.py), made through alis.h:
+ * cubes with 8-cell CPML, TF/SF boxes side by side along x or a point dipole, a gold sphere.
+ */
+#include "alis.h"
+#include "../alis_amd/host/internal.h"
+
+world ec_world(int cells, int boxes, int sphere)
+{
+	const float dx = 10, e = dx * (cells - 18) / 2;
+	dom D = {{-e, e}, {-e, e}, {-e, e}};
+	res R = {5, {dx}, {1240}};
+	sur S = {{PML}, {PML}, {PML}, {8}};
+	world W = createWorld(D, R, S, "");
+	matter Gold = {{1.5}, {{9, 0.07}, {2.6, 0.3, 0.5}, {3.5, 0.6, 0.8}}};
+	object Sphere = {Ball, {{-4 * dx, 4 * dx}, {-4 * dx, 4 * dx}, {-4 * dx, 4 * dx}}};
+	if (sphere) putObjects(W, Gold, Sphere, Air);
+	for (int b = 0; b < boxes; b++) {
+		const float x = -0.8f * e + 1.6f * e * b / boxes;
+		dom T = {{x, x + 1.2f * e / boxes}, {-0.6f * e, 0.6f * e}, {-0.6f * e, 0.6f * e}};
+		planewave(W, T, Ppol, 0, 0, Pulse, 600, 400);
+	}
+	if (!boxes) pointDipole(W, Ez, 0, 0, 0, Pulse, 600, 240);
+	return W;
+}
+
+void ec_step(world W, int n) { for (int s = 0; s < n; s++) updateE(W), updateH(W); }
+void ec_free(world W) { deleteWorld(W); }
+alis_dev_world *ec_device(world W) { return W->dev; }
+alis_dev_world *ec_aux(world W, int n)
+{
+	tfsf S = W->S;
+	while (n--) S = S->S;
+	return S->W->dev;
+}
+
+/* W's device worlds belong to the caller from here on. */
+void ec_disown(world W)
+{
+	W->dev = 0;
+	for (tfsf S = W->S; S; S = S->S) S->W->dev = 0;
+}
+
+/* Commit W with the box of its dispersive object reaching `below` cells under the grid. */
+int ec_commit_below(world W, int below)
+{
+	alis_dev_world_desc d;
+	alis_dev_world *D;
+	describeWorld(W, &d);
+	alis_dev_ade *o = (alis_dev_ade *)d.obj;
+	o->k0 = d.kMIN - below;
+	for (int c = 0; c < 3; c++) {
+		o->fill[c] = makeField(o->i0, o->i1, o->j0, o->j1, o->k0, o->k1);
+		for (int p = 0; p < o->nk; p++)
+			for (int m = 0; m <= d.complexField; m++) {
+				o->J[m][c][p] = makeField(o->i0, o->i1, o->j0, o->j1, o->k0, o->k1);
+				o->K[m][c][p] = makeField(o->i0, o->i1, o->j0, o->j1, o->k0, o->k1);
+			}
+	}
+	const int rc = alis_dev_commit(&d, 0, 1, &D);
+	freeWorldDesc(&d);
+	if (!rc) alis_dev_release(D);
+	return rc;
+}

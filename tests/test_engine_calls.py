@@ -1,0 +1,97 @@
+"""Calls of the engine ABI whose work waits for a later one, checked on the CPU: the order in which
+the engine launches, waits and copies, recorded by a HIP runtime that runs no kernel
+(hip_recorder.c), and the memory it allocates.  Each case is a process of its own."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from scenarios import ROOT
+
+HEAD = r'''
+import ctypes, re, sys, threading
+GLOBAL, V, I = ctypes.RTLD_GLOBAL, ctypes.c_void_p, ctypes.c_int
+rec = ctypes.CDLL(sys.argv[1] + "/hip_recorder.so", mode=GLOBAL)
+lib = ctypes.CDLL(sys.argv[2] + "/alis_amd/libalis.so", mode=GLOBAL)
+ec = ctypes.CDLL(sys.argv[1] + "/engine_client.so")
+rec.hipRecLog.restype = lib.alis_dev_error.restype = ctypes.c_char_p
+rec.hipRecOutside.restype = ctypes.c_long
+rec.hipRecStreamOf.argtypes = [V]
+ec.ec_world.restype = ec.ec_device.restype = ec.ec_aux.restype = V
+ec.ec_step.argtypes = ec.ec_aux.argtypes = ec.ec_commit_below.argtypes = [V, I]
+ec.ec_device.argtypes = ec.ec_free.argtypes = ec.ec_disown.argtypes = [V]
+lib.alis_dev_core.argtypes = lib.alis_dev_ghosts.argtypes = [V, I]
+lib.alis_dev_batch_core.argtypes = lib.alis_dev_batch_post.argtypes = [V, I]
+lib.alis_dev_strips.argtypes = [V, I, I]
+lib.alis_dev_sync.argtypes = [V] + 6 * [I]
+lib.alis_dev_synchronize.argtypes = lib.alis_dev_batch_release.argtypes = lib.alis_dev_release.argtypes = [V]
+lib.alis_dev_batch_create.argtypes = [ctypes.POINTER(V), I, ctypes.POINTER(V)]
+lib.alis_dev_batch_release.restype = lib.alis_dev_release.restype = None
+
+def ok(rc):
+    assert rc == 0, lib.alis_dev_error().decode()
+
+def calls(f, *args):
+    """(launch, kernel, half step of a curl, workgroups, stream) and (wait, stream, other) of f."""
+    rec.hipRecClear()
+    f(*args)
+    out = []
+    for line in rec.hipRecLog().decode().splitlines():
+        what, name, n, s = line.split()
+        if what == "wait":
+            out.append((what, int(n), int(s)))
+        else:
+            half = re.search(r"k_curl\w*?I[fd]Li(\d)", name)
+            out.append((what, re.search(r"k_[a-z_]+", name).group(), int(half.group(1)) if half else -1, int(n), int(s)))
+    return out
+
+def kernels(log):
+    return [c[1] for c in log if c[0] == "launch"]
+
+def batch(devices):
+    B = V()
+    ok(lib.alis_dev_batch_create((V * len(devices))(*devices), len(devices), ctypes.byref(B)))
+    return B
+'''
+
+
+@pytest.fixture(scope="module")
+def libs(tmp_path_factory):
+    out = tmp_path_factory.mktemp("recorder")
+    for name in ("hip_recorder", "engine_client"):
+        subprocess.run(["gcc", "-O1", "-std=gnu99", "-shared", "-fPIC", f"-I{ROOT / 'include'}", "-o", str(out / f"{name}.so"),
+                        str(ROOT / "tests" / f"{name}.c"), "-lpthread"], check=True)
+    return out
+
+
+def run(libs, code, **env):
+    r = subprocess.run([sys.executable, "-c", HEAD + code, str(libs), str(ROOT)], capture_output=True, text=True, timeout=120,
+                       cwd=libs, env={**os.environ, **env})
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("worlds", [2, 3])
+def test_parts_of_a_world_as_entries_of_their_own(libs, worlds):
+    """ALIS_BATCH_PAIRS=0: the parts of a Bloch world run side by side in one launch, so neither may make
+    the ghost copies along z, which need the other's values and write both: all copies are left to
+    the end of the half step, as they are where the core runs by itself."""
+    run(libs, f"""
+wl = ctypes.CDLL(sys.argv[2] + "/alis_amd/libalis_workloads.so")
+wl.wl_create.restype = wl.wl_device_of.restype = V
+wl.wl_step.argtypes = wl.wl_device_of.argtypes = [V, I]
+c = wl.wl_create(b"kpoints", {worlds}, 32, 64)
+wl.wl_step(c, 1)
+B = batch([wl.wl_device_of(c, q) for q in range({worlds})])
+
+def half(h, apart):
+    ok(lib.alis_dev_batch_core(B, h))
+    if apart:
+        ok(lib.alis_dev_synchronize(wl.wl_device_of(c, 0)))
+    ok(lib.alis_dev_batch_post(B, h))
+
+for h in range(2):
+    posts = [[k[3] for k in calls(half, h, apart) if k[1] == "k_post_batch"] for apart in (True, False)]
+    assert posts[0] and posts[0] == posts[1], posts
+lib.alis_dev_batch_release(B)
+""", ALIS_BATCH_PAIRS="0")

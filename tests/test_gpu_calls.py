@@ -1,0 +1,56 @@
+"""Batches of Bloch worlds (complex fields, CPML along z) in other ways than updateWorldsE/H: FP32 fields
+bit for bit the CPU oracle's, after enough steps that the fields reach the ends of z."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from scenarios import ROOT
+
+pytestmark = pytest.mark.gpu
+
+LIBS = {"hip": (ROOT / "alis_amd" / "libalis_workloads.so", ROOT / "alis_amd" / "libalis.so"),
+        "oracle": (ROOT / "oracle" / "libwl_oracle.so", ROOT / "oracle" / "liboracle.so")}
+WORLDS, STEPS = 2, 90
+
+
+def _fields(kind, program=None):
+    """The fields of WORLDS k-point worlds after STEPS steps and then program(engine, batch, devices)."""
+    w, e = (ctypes.CDLL(str(p)) for p in LIBS[kind])
+    V, I = ctypes.c_void_p, ctypes.c_int
+    w.wl_create.restype = w.wl_device_of.restype = V
+    w.wl_create.argtypes = [ctypes.c_char_p] + [I] * 3
+    w.wl_step.argtypes = w.wl_device_of.argtypes = [V, I]
+    w.wl_free.argtypes = [V]
+    w.wl_field.restype = ctypes.c_long
+    w.wl_field.argtypes = [V] + [I] * 4 + [ctypes.POINTER(ctypes.c_double), ctypes.c_long]
+    e.alis_dev_batch_create.argtypes = [ctypes.POINTER(V), I, ctypes.POINTER(V)]
+    for f in (e.alis_dev_core, e.alis_dev_ghosts, e.alis_dev_batch_core, e.alis_dev_batch_post):
+        f.argtypes = [V, I]
+    e.alis_dev_batch_release.argtypes, e.alis_dev_batch_release.restype = [V], None
+    c = w.wl_create(b"kpoints", WORLDS, 32, 64)
+    w.wl_step(c, STEPS)
+    if program:
+        dev = (V * WORLDS)(*[w.wl_device_of(c, q) for q in range(WORLDS)])
+        B = V()
+        assert e.alis_dev_batch_create(dev, WORLDS, ctypes.byref(B)) == 0
+        program(e, B, dev)
+        e.alis_dev_batch_release(B)
+        w.wl_step(c, 2)
+    buf = (ctypes.c_double * 400000)()
+    out = []
+    for q in range(WORLDS):
+        for h in range(2):
+            for m in range(2):
+                for a in range(3):
+                    n = w.wl_field(c, q, h, m, a, buf, len(buf))
+                    assert n > 0
+                    out.append(np.frombuffer(buf, dtype=np.float64, count=n).copy())
+    w.wl_free(c)
+    return np.concatenate(out)
+
+
+def test_parts_in_entries_of_their_own(monkeypatch):
+    monkeypatch.setenv("ALIS_BATCH_PAIRS", "0")
+    got, ref = _fields("hip"), _fields("oracle")
+    assert np.abs(ref).max() > 0 and np.array_equal(got, ref)
