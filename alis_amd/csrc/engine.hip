@@ -2785,6 +2785,13 @@ int auxHalves(alis_dev_world *D)
 
 int batchFlush(alis_dev_batch *B);
 
+// Whether a part of D's half step waits for a later call (other than the objects' current update, which an
+// H program takes along).
+bool halfWaits(const alis_dev_world *D)
+{
+	return D->pendE || D->pendH || D->pendCore || D->pendMain || D->pendPost || D->pendBatch;
+}
+
 // Complete a deferred step the separate way (a call that reads or changes the world between
 // its E and H halves, or that reads an auxiliary world whose H half waits).
 template<class T>
@@ -4557,7 +4564,8 @@ int alis_dev_batch_post(alis_dev_batch *B, int h)
 		B->pend = 0;
 		for (alis_dev_world *W : B->W) W->pendBatch = nullptr;
 	}
-	else for (alis_dev_world *W : B->W) if (W->pendBatch && flushE(W)) return -1;
+	else
+		for (alis_dev_world *W : B->W) if (halfWaits(W) && flushE(W)) return -1;
 	return B->fp64 ? batchPost<double>(B, h, whole) : batchPost<float>(B, h, whole);
 }
 

@@ -95,3 +95,28 @@ for h in range(2):
     assert posts[0] and posts[0] == posts[1], posts
 lib.alis_dev_batch_release(B)
 """, ALIS_BATCH_PAIRS="0")
+
+
+@pytest.mark.parametrize("boxes", [0, 1])
+def test_cores_of_their_own_before_a_batch_post(libs, boxes):
+    """alis_dev_core of every world, then the post of their batch: the curls come before the end of the half
+    step that they belong to."""
+    run(libs, f"""
+W = [V(ec.ec_world(40, {boxes}, 1)) for _ in range(2)]
+for w in W:
+    ec.ec_step(w, 1)
+dev = [ec.ec_device(w) for w in W] + [ec.ec_aux(w, 0) for w in W if {boxes}]
+B = batch(dev)
+
+def half(h):
+    for d in dev:
+        ok(lib.alis_dev_core(d, h))
+    ok(lib.alis_dev_batch_post(B, h))
+
+for h in (0, 1, 0, 1):
+    log = calls(half, h)
+    curls = [n for n, c in enumerate(log) if c[2] == h and c[1].startswith("k_curl")]
+    posts = [n for n, c in enumerate(log) if c[1] == "k_post_batch"]
+    assert len(curls) == len(dev) and posts and curls[-1] < posts[0], log
+lib.alis_dev_batch_release(B)
+""")

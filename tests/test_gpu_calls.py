@@ -54,3 +54,16 @@ def test_parts_in_entries_of_their_own(monkeypatch):
     monkeypatch.setenv("ALIS_BATCH_PAIRS", "0")
     got, ref = _fields("hip"), _fields("oracle")
     assert np.abs(ref).max() > 0 and np.array_equal(got, ref)
+
+
+def _cores_apart(e, B, dev):
+    for h in range(2):
+        for d in dev:
+            assert e.alis_dev_core(d, h) == 0
+        assert e.alis_dev_batch_post(B, h) == 0
+
+
+@pytest.mark.parametrize("program", [_cores_apart])
+def test_half_steps_of_single_and_shared_calls(program):
+    got, ref = _fields("hip", program), _fields("oracle", program)
+    assert np.abs(ref).max() > 0 and np.array_equal(got, ref)
