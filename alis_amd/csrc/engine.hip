@@ -2879,7 +2879,7 @@ int ghostsEntry(alis_dev_world *D, int h)
 		D->pendH = 2;
 		return 0;
 	}
-	if ((h == 0 || D->pendE || D->pendH || D->pendCore || D->pendMain || D->pendPost) && flushStep<T>(D)) return -1;   // (an H program takes its current update along)
+	if ((h == 0 || halfWaits(D)) && flushStep<T>(D)) return -1;   // (an H program takes its current update along)
 	return postHalf<T>(D, h);
 }
 

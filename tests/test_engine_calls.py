@@ -120,3 +120,25 @@ for h in (0, 1, 0, 1):
     assert len(curls) == len(dev) and posts and curls[-1] < posts[0], log
 lib.alis_dev_batch_release(B)
 """)
+
+
+def test_ends_of_their_own_after_a_batch_core(libs):
+    """The core of a batch, then alis_dev_ghosts of each world: the curl comes before the end of either half
+    step."""
+    run(libs, """
+W = [V(ec.ec_world(40, 0, 0)) for _ in range(2)]
+for w in W:
+    ec.ec_step(w, 1)
+dev = [ec.ec_device(w) for w in W]
+B = batch(dev)
+
+def half(h):
+    ok(lib.alis_dev_batch_core(B, h))
+    for d in dev:
+        ok(lib.alis_dev_ghosts(d, h))
+
+for h in (0, 1, 0, 1):
+    k = kernels(calls(half, h))
+    assert k[0] == "k_curl_batch" and k.count("k_curl_batch") == 1 and "k_post" in k, k
+lib.alis_dev_batch_release(B)
+""")

@@ -63,7 +63,14 @@ def _cores_apart(e, B, dev):
         assert e.alis_dev_batch_post(B, h) == 0
 
 
-@pytest.mark.parametrize("program", [_cores_apart])
+def _ends_apart(e, B, dev):
+    for h in range(2):
+        assert e.alis_dev_batch_core(B, h) == 0
+        for d in dev:
+            assert e.alis_dev_ghosts(d, h) == 0
+
+
+@pytest.mark.parametrize("program", [_cores_apart, _ends_apart])
 def test_half_steps_of_single_and_shared_calls(program):
     got, ref = _fields("hip", program), _fields("oracle", program)
     assert np.abs(ref).max() > 0 and np.array_equal(got, ref)
