@@ -1182,7 +1182,7 @@ Lay fieldLayout(const alis_dev_world *D)
 // quad of the grid is one quad here.
 Lay quadLayout(const alis_dev_world *D, const Box &b)
 {
-	const int quad = 16 / (int)D->esz, k0 = D->kMIN + (b.k0 - D->kMIN) / quad * quad;
+	const int quad = 16 / (int)D->esz, rest = ((b.k0 - D->kMIN) % quad + quad) % quad, k0 = b.k0 - rest;   // (boxes may start below the grid)
 	Lay L;
 	L.i0 = b.i0, L.j0 = b.j0, L.k0 = k0, L.koff = 0;
 	L.sj = (b.k1 - k0 + quad) / quad * quad;

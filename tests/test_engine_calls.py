@@ -142,3 +142,14 @@ for h in (0, 1, 0, 1):
     assert k[0] == "k_curl_batch" and k.count("k_curl_batch") == 1 and "k_post" in k, k
 lib.alis_dev_batch_release(B)
 """)
+
+
+@pytest.mark.parametrize("below", [0, 1, 3, 4, 5, 8, 11])
+def test_object_box_below_the_grid(libs, below):
+    """A dispersive object whose box starts under kMIN: its arrays, laid out along the grid's quads, hold
+    every cell of the box."""
+    run(libs, f"""
+W = ec.ec_world(40, 0, 1)
+ok(ec.ec_commit_below(W, {below}))
+assert rec.hipRecOutside() == 0
+""")
