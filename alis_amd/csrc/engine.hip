@@ -2406,7 +2406,8 @@ template<class T>
 int endHalf(alis_dev_world *D, int h, const PostArgs<T> *x)
 {
 	const int made = curlMakes(D, h);
-	if (h == 0 && made == 2 && !x && !D->isAux && (D->tf.empty() || D->tf[0].aux->st == D->st) && D->tf.size() < 2) {
+	const bool alone = D->tf.empty() || (D->tf.size() == 1 && (!D->tf[0].aux || D->tf[0].aux->st == D->st));   // (released: null)
+	if (h == 0 && made == 2 && !x && !D->isAux && alone) {
 		size_t programs = 0;
 		for (const PostSeg &G : D->post[0]) programs += G.bare > 0;
 		if (programs <= 1) {

@@ -5,8 +5,10 @@
 #include "alis.h"
 #include "../alis_amd/host/internal.h"
 
-world ec_world(int cells, int boxes, int sphere)
+/* percent: the boxes' edges, of the domain's. */
+world ec_boxes(int cells, int boxes, int sphere, int percent)
 {
+	const float half = 0.01f * percent;
 	const float dx = 10, e = dx * (cells - 18) / 2;
 	dom D = {{-e, e}, {-e, e}, {-e, e}};
 	res R = {5, {dx}, {1240}};
@@ -17,13 +19,14 @@ world ec_world(int cells, int boxes, int sphere)
 	if (sphere) putObjects(W, Gold, Sphere, Air);
 	for (int b = 0; b < boxes; b++) {
 		const float x = -0.8f * e + 1.6f * e * b / boxes;
-		dom T = {{x, x + 1.2f * e / boxes}, {-0.6f * e, 0.6f * e}, {-0.6f * e, 0.6f * e}};
+		dom T = {{x, x + 2 * half * e / boxes}, {-half * e, half * e}, {-half * e, half * e}};
 		planewave(W, T, Ppol, 0, 0, Pulse, 600, 400);
 	}
 	if (!boxes) pointDipole(W, Ez, 0, 0, 0, Pulse, 600, 240);
 	return W;
 }
 
+world ec_world(int cells, int boxes, int sphere) { return ec_boxes(cells, boxes, sphere, 60); }
 void ec_step(world W, int n) { for (int s = 0; s < n; s++) updateE(W), updateH(W); }
 void ec_free(world W) { deleteWorld(W); }
 alis_dev_world *ec_device(world W) { return W->dev; }

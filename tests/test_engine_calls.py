@@ -18,7 +18,7 @@ ec = ctypes.CDLL(sys.argv[1] + "/engine_client.so")
 rec.hipRecLog.restype = lib.alis_dev_error.restype = ctypes.c_char_p
 rec.hipRecOutside.restype = ctypes.c_long
 rec.hipRecStreamOf.argtypes = [V]
-ec.ec_world.restype = ec.ec_device.restype = ec.ec_aux.restype = V
+ec.ec_world.restype = ec.ec_boxes.restype = ec.ec_device.restype = ec.ec_aux.restype = V
 ec.ec_step.argtypes = ec.ec_aux.argtypes = ec.ec_commit_below.argtypes = [V, I]
 ec.ec_device.argtypes = ec.ec_free.argtypes = ec.ec_disown.argtypes = [V]
 lib.alis_dev_core.argtypes = lib.alis_dev_ghosts.argtypes = [V, I]
@@ -152,4 +152,24 @@ def test_object_box_below_the_grid(libs, below):
 W = ec.ec_world(40, 0, 1)
 ok(ec.ec_commit_below(W, {below}))
 assert rec.hipRecOutside() == 0
+""")
+
+
+def test_main_world_without_its_auxiliary_world(libs):
+    """The auxiliary world of a TF/SF box released before its main world, which steps on without strips."""
+    run(libs, """
+W = ec.ec_boxes(64, 1, 0, 25)
+ec.ec_step(W, 2)
+D, A = ec.ec_device(W), ec.ec_aux(W, 0)
+ec.ec_disown(W)
+lib.alis_dev_release(A)
+
+def step():
+    for h in range(2):
+        ok(lib.alis_dev_core(D, h))
+        ok(lib.alis_dev_ghosts(D, h))
+
+for _ in range(2):
+    assert [c[2] for c in calls(step) if c[1].startswith("k_curl")] == [0, 1]
+lib.alis_dev_release(D)
 """)
