@@ -3652,7 +3652,7 @@ int alis_dev_link_tfsf(alis_dev_world *D, int s, alis_dev_world *aux)
 void alis_dev_release(alis_dev_world *D)
 {
 	if (!D) return;
-	if (D->pendMain || D->pendCore || D->pendBatch) (void)flushE(D);     // an auxiliary world's half step outlives its main world
+	if (halfWaits(D)) (void)flushE(D);     // an auxiliary world's half step outlives its main world
 	if (D->st) hipStreamSynchronize(D->st);
 	for (DevTfsf &t : D->tf) if (t.aux && t.aux->mainOf == D) t.aux->mainOf = nullptr;
 	if (D->mainOf)

@@ -173,3 +173,38 @@ for _ in range(2):
     assert [c[2] for c in calls(step) if c[1].startswith("k_curl")] == [0, 1]
 lib.alis_dev_release(D)
 """)
+
+
+@pytest.mark.parametrize("calls_made", [1, 2])
+def test_auxiliary_world_outlives_a_deferred_step(libs, calls_made):
+    """ALIS_FUSE=force: an auxiliary world's H half step waits for its main world's fused step; where that
+    world is released first, the half step is made all the same."""
+    run(libs, f"""
+W = ec.ec_world(40, 1, 0)
+ec.ec_step(W, 2)
+D, A = ec.ec_device(W), ec.ec_aux(W, 0)
+ec.ec_disown(W)
+
+def part():
+    ok(lib.alis_dev_core(D, 0))
+    ok(lib.alis_dev_core(A, 0)), ok(lib.alis_dev_ghosts(A, 0))
+    ok(lib.alis_dev_ghosts(D, 0))
+    ok(lib.alis_dev_core(D, 1))
+    ok(lib.alis_dev_core(A, 1))
+    if {calls_made} == 2:
+        ok(lib.alis_dev_ghosts(A, 1))
+    lib.alis_dev_release(D)
+    if {calls_made} == 1:
+        ok(lib.alis_dev_ghosts(A, 1))
+    ok(lib.alis_dev_synchronize(A))
+
+k = [c[2] for c in calls(part) if c[1].startswith("k_curl") and c[3] <= 4]     # (the small world's)
+assert k == [0, 1], k
+
+def step():
+    for h in range(2):
+        ok(lib.alis_dev_core(A, h)), ok(lib.alis_dev_ghosts(A, h))
+
+assert [c[2] for c in calls(step) if c[1].startswith("k_curl")] == [0, 1]
+lib.alis_dev_release(A)
+""", ALIS_FUSE="force")
