@@ -4835,6 +4835,7 @@ int alis_dev_timing(alis_dev_world *D, int enable)
 int alis_dev_timing_read(alis_dev_world *D, int h, double *ms, long *launches)
 {
 	if (h < 0 || h > 2) return fail("no such timed launch");
+	if (flushE(D)) return -1;
 	HIPCHECK(hipStreamSynchronize(D->st));
 	auto &v = D->evPairs[h];
 	for (size_t a = 0; a + 1 < v.size(); a += 2) {

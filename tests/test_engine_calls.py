@@ -208,3 +208,21 @@ def step():
 assert [c[2] for c in calls(step) if c[1].startswith("k_curl")] == [0, 1]
 lib.alis_dev_release(A)
 """, ALIS_FUSE="force")
+
+
+def test_timing_counts_a_waiting_core(libs):
+    """alis_dev_timing_read after alis_dev_core: the launch that the call asked for is counted."""
+    run(libs, """
+W = ec.ec_world(40, 0, 0)
+ec.ec_step(W, 1)
+D = ec.ec_device(W)
+lib.alis_dev_timing.argtypes = [V, I]
+lib.alis_dev_timing_read.argtypes = [V, I, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_long)]
+ok(lib.alis_dev_timing(D, 1))
+for h in range(2):
+    ok(lib.alis_dev_core(D, h))
+    ms, n = ctypes.c_double(), ctypes.c_long()
+    ok(lib.alis_dev_timing_read(D, h, ctypes.byref(ms), ctypes.byref(n)))
+    assert n.value == 1 and ms.value > 0
+    ok(lib.alis_dev_ghosts(D, h))
+""")
