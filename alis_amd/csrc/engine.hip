@@ -23,6 +23,7 @@
 #include <cmath>
 #include <algorithm>
 #include <functional>
+#include <list>
 #include <map>
 #include <mutex>
 #include <system_error>
@@ -2884,13 +2885,13 @@ int ghostsEntry(alis_dev_world *D, int h)
 	return postHalf<T>(D, h);
 }
 
-// Pinned chunks and their events for mirrorAll, two per thread, made as calls need them: 32 MiB at most,
-// shared by all worlds, one call at a time, given back with the last world.
+// Pinned chunks and their events for mirrorAll, two per thread, made as calls need them: 32 MiB at most.
+// An event belongs to the device that was current when it was made, and may be recorded on that
+// device's streams only.
 struct MirrorStage {
-	std::mutex lock;
+	int device = 0;
 	float *pinned[2 * MIRROR_THREADS] = {};
 	hipEvent_t done[2 * MIRROR_THREADS] = {};
-	int worlds = 0;
 
 	// The first of each thread's chunks, and the second where there are more chunks than threads.
 	bool ready(int threads, long chunks)
@@ -2909,38 +2910,67 @@ struct MirrorStage {
 		for (float *&p : pinned) if (p) (void)hipHostFree(p), p = nullptr;
 		for (hipEvent_t &e : done) if (e) (void)hipEventDestroy(e), e = nullptr;
 	}
+};
+
+// One per device, shared by its worlds; one call at a time; given back with the last world.
+struct MirrorStages {
+	std::mutex lock;
+	std::list<MirrorStage> all;
+	int worlds = 0;
+
+	MirrorStage &of(int device)
+	{
+		for (MirrorStage &s : all) if (s.device == device) return s;
+		all.emplace_back();
+		all.back().device = device;
+		return all.back();
+	}
 	void hold(int n)
 	{
 		std::lock_guard<std::mutex> g(lock);
 		worlds += n;
-		if (!worlds) clear();
+		if (worlds) return;
+		for (MirrorStage &s : all) s.clear();
+		all.clear();
 	}
 };
-MirrorStage g_mirror;
+MirrorStages g_mirror;
+
+// The calling thread's current device while this lives.
+struct OnDevice {
+	int was = 0;
+	hipError_t err;
+	explicit OnDevice(int device)
+	{
+		err = hipGetDevice(&was);
+		if (err == hipSuccess) err = hipSetDevice(device);
+	}
+	~OnDevice() { (void)hipSetDevice(was); }
+};
 
 struct MirrorHost { float *host; long off, n; };
 
 // Thread `t` of `threads`: chunks t, t + threads, ... of the run.
 template<class T>
-hipError_t mirrorChunks(int device, hipStream_t st, const MirrorSeg<T> *seg, const std::vector<MirrorHost> &out, long total, int t, int threads)
+hipError_t mirrorChunks(const MirrorStage &stage, hipStream_t st, const MirrorSeg<T> *seg, const std::vector<MirrorHost> &out, long total, int t, int threads)
 {
-	hipError_t e = hipSetDevice(device);
+	hipError_t e = hipSetDevice(stage.device);
 	const long chunks = (total + MIRROR_CHUNK - 1) / MIRROR_CHUNK;
 	auto length = [&](long c) { return std::min(MIRROR_CHUNK, total - c * MIRROR_CHUNK); };
 	auto launch = [&](long c, int x) {
 		if (c >= chunks || e != hipSuccess) return;
-		float *const dst = g_mirror.pinned[2 * t + x];
+		float *const dst = stage.pinned[2 * t + x];
 		k_mirror<T><<<blocksFor(length(c), 1024), 256, 0, st>>>(seg, (int)out.size(), c * MIRROR_CHUNK, length(c), dst);
 		e = hipGetLastError();
-		if (e == hipSuccess) e = hipEventRecord(g_mirror.done[2 * t + x], st);
+		if (e == hipSuccess) e = hipEventRecord(stage.done[2 * t + x], st);
 	};
 	launch(t, 0);
 	int x = 0;
 	for (long c = t; c < chunks && e == hipSuccess; c += threads, x ^= 1) {
 		launch(c + threads, x ^ 1);
-		if (e == hipSuccess) e = hipEventSynchronize(g_mirror.done[2 * t + x]);
+		if (e == hipSuccess) e = hipEventSynchronize(stage.done[2 * t + x]);
 		if (e != hipSuccess) break;
-		const float *v = g_mirror.pinned[2 * t + x];
+		const float *v = stage.pinned[2 * t + x];
 		const long a = c * MIRROR_CHUNK, b = a + length(c);
 		size_t s = std::upper_bound(out.begin(), out.end(), a, [](long p, const MirrorHost &h) { return p < h.off; }) - out.begin() - 1;
 		for (; s < out.size() && out[s].off < b; s++) {
@@ -2990,12 +3020,13 @@ int mirrorAll(alis_dev_world *D, bool &done)
 		}
 	const long chunks = (total + MIRROR_CHUNK - 1) / MIRROR_CHUNK;
 	const int threads = (int)std::min<long>(std::min<long>(MIRROR_THREADS, std::max(1u, std::thread::hardware_concurrency())), chunks);
-	if (!g_mirror.ready(threads, chunks)) return 0;
+	const OnDevice here(D->device);
+	HIPCHECK(here.err);
+	MirrorStage &stage = g_mirror.of(D->device);
+	if (!stage.ready(threads, chunks)) return 0;
 	const size_t table = seg.size() * sizeof(MirrorSeg<T>);
 	if (ensureScratch(D, (long)((table + sizeof(double) - 1) / sizeof(double)))) return -1;
 	HIPCHECK(hipMemcpyAsync(D->scratch, seg.data(), table, hipMemcpyHostToDevice, D->st));
-	int device = 0;
-	HIPCHECK(hipGetDevice(&device));
 #ifdef MADV_POPULATE_WRITE
 	// Fresh host arrays: their pages in one call, where the copying threads would fault them in one by
 	// one and wait for each other (400x400x200, first sync with its world's first pass: 980 ms by
@@ -3010,7 +3041,7 @@ int mirrorAll(alis_dev_world *D, bool &done)
 	D->mirrored = true;
 #endif
 	hipError_t err[MIRROR_THREADS] = {};
-	auto work = [&](int t, int of) { err[t] = mirrorChunks<T>(device, D->st, (const MirrorSeg<T> *)D->scratch, out, total, t, of); };
+	auto work = [&](int t, int of) { err[t] = mirrorChunks<T>(stage, D->st, (const MirrorSeg<T> *)D->scratch, out, total, t, of); };
 	std::vector<std::thread> pool;
 	pool.reserve(MIRROR_THREADS);
 	int alone = 0;                         // threads that could not be started: their share runs here

@@ -8,7 +8,8 @@
  *
  * Loaded (RTLD_GLOBAL) before the library, whose references then bind here.  There are two devices;
  * an event may be recorded only on a stream of its own device.  A box that k_unpack would write
- * outside its allocation is counted (hipRecOutside).
+ * outside its allocation is counted (hipRecOutside), and so is a launch of k_mirror from a thread
+ * whose current device is not the stream's (hipRecForeign).
  */
 #define _GNU_SOURCE
 #include <pthread.h>
@@ -30,7 +31,7 @@ static pthread_cond_t changed = PTHREAD_COND_INITIALIZER;
 static char *text;
 static size_t used, room;
 static int nstreams, waiting, nevents, npinned;
-static long outside;
+static long outside, foreign;
 
 static void say(const char *what, const char *name, long n, int s)
 {
@@ -46,6 +47,7 @@ static void say(const char *what, const char *name, long n, int s)
 const char *hipRecLog(void) { return text ? text : ""; }
 void hipRecClear(void) { if (text) text[used = 0] = 0; }
 long hipRecOutside(void) { return outside; }
+long hipRecForeign(void) { return foreign; }
 int hipRecStreamOf(void *s) { return ((stream *)s)->id; }
 int hipRecPinned(void) { return npinned; }
 
@@ -195,6 +197,7 @@ static int launch(const void *f, dim3 grid, void **args, stream *S)
 	const char *name = "?";
 	for (int k = 0; k < nkernels; k++) if (kernels[k].f == f) name = kernels[k].name;
 	if (strstr(name, "k_unpack")) checkUnpack(name, args);
+	if (strstr(name, "k_mirror") && S->device != current) __atomic_fetch_add(&foreign, 1, __ATOMIC_RELAXED);
 	say("launch", name, (long)grid.x * grid.y * grid.z, S->id);
 	return OK;
 }

@@ -226,3 +226,25 @@ for h in range(2):
     assert n.value == 1 and ms.value > 0
     ok(lib.alis_dev_ghosts(D, h))
 """)
+
+
+def test_whole_syncs_on_two_devices(libs):
+    """Worlds on two GPUs, synced from either of them as the current device: events and streams of one
+    device together, the caller's device left as it was."""
+    run(libs, """
+dev = []
+for d in range(2):
+    ok(rec.hipSetDevice(d))
+    W = ec.ec_world(40, 0, 1)
+    ec.ec_step(W, 1)
+    dev.append(ec.ec_device(W))
+for current in (1, 0):
+    ok(rec.hipSetDevice(current))
+    for D in dev + dev:
+        log = calls(lambda: ok(lib.alis_dev_sync(D, 0, -1, 0, -1, 0, -1)))
+        assert "k_mirror" in kernels(log) and "k_pack" not in kernels(log), log
+        now = I()
+        ok(rec.hipGetDevice(ctypes.byref(now)))
+        assert now.value == current
+assert rec.hipRecForeign() == 0
+""")
