@@ -22,6 +22,7 @@
 #include <cstdint>
 #include <cmath>
 #include <algorithm>
+#include <condition_variable>
 #include <functional>
 #include <list>
 #include <map>
@@ -2890,6 +2891,7 @@ int ghostsEntry(alis_dev_world *D, int h)
 // device's streams only.
 struct MirrorStage {
 	int device = 0;
+	bool taken = false;
 	float *pinned[2 * MIRROR_THREADS] = {};
 	hipEvent_t done[2 * MIRROR_THREADS] = {};
 
@@ -2912,29 +2914,65 @@ struct MirrorStage {
 	}
 };
 
-// One per device, shared by its worlds; one call at a time; given back with the last world.
+// Those of the process: a whole sync takes one of its device for itself, or waits for one, so at most
+// MIRROR_STAGES of a device's syncs run at a time.  The lock is held for the choice alone: commits, releases
+// and other syncs go on meanwhile.  Two, since one sync leaves the link idle between its chunks (syncs a
+// second from two threads, one stage -> two: 64^3 worlds 2680 -> 4120, 160^3 374 -> 433).  Given back with
+// the last world.
+constexpr int MIRROR_STAGES = 2;
 struct MirrorStages {
 	std::mutex lock;
+	std::condition_variable given;
 	std::list<MirrorStage> all;
 	int worlds = 0;
 
-	MirrorStage &of(int device)
+	MirrorStage *take(int device)
 	{
-		for (MirrorStage &s : all) if (s.device == device) return s;
-		all.emplace_back();
-		all.back().device = device;
-		return all.back();
+		std::unique_lock<std::mutex> g(lock);
+		for (;;) {
+			int n = 0;
+			for (MirrorStage &s : all) {
+				if (s.device != device) continue;
+				if (!s.taken) {
+					s.taken = true;
+					return &s;
+				}
+				n++;
+			}
+			if (n < MIRROR_STAGES) {
+				all.emplace_back();
+				all.back().device = device, all.back().taken = true;
+				return &all.back();
+			}
+			given.wait(g);
+		}
+	}
+	void give(MirrorStage *s)
+	{
+		{
+			std::lock_guard<std::mutex> g(lock);
+			s->taken = false;
+		}
+		given.notify_all();
 	}
 	void hold(int n)
 	{
-		std::lock_guard<std::mutex> g(lock);
-		worlds += n;
-		if (worlds) return;
-		for (MirrorStage &s : all) s.clear();
-		all.clear();
+		std::list<MirrorStage> old;         // (none is taken: a sync's own world is counted)
+		{
+			std::lock_guard<std::mutex> g(lock);
+			worlds += n;
+			if (!worlds) old.swap(all);
+		}
+		for (MirrorStage &s : old) s.clear();
 	}
 };
 MirrorStages g_mirror;
+
+struct MirrorTaken {
+	MirrorStage *const s;
+	explicit MirrorTaken(int device) : s(g_mirror.take(device)) {}
+	~MirrorTaken() { g_mirror.give(s); }
+};
 
 // The calling thread's current device while this lives.
 struct OnDevice {
@@ -2986,7 +3024,6 @@ template<class T>
 int mirrorAll(alis_dev_world *D, bool &done)
 {
 	done = false;
-	std::lock_guard<std::mutex> guard(g_mirror.lock);
 	const alis_dev_world_desc *W = &D->W;
 	std::vector<MirrorSeg<T>> seg;
 	std::vector<MirrorHost> out;
@@ -3022,7 +3059,8 @@ int mirrorAll(alis_dev_world *D, bool &done)
 	const int threads = (int)std::min<long>(std::min<long>(MIRROR_THREADS, std::max(1u, std::thread::hardware_concurrency())), chunks);
 	const OnDevice here(D->device);
 	HIPCHECK(here.err);
-	MirrorStage &stage = g_mirror.of(D->device);
+	const MirrorTaken mine(D->device);
+	MirrorStage &stage = *mine.s;
 	if (!stage.ready(threads, chunks)) return 0;
 	const size_t table = seg.size() * sizeof(MirrorSeg<T>);
 	if (ensureScratch(D, (long)((table + sizeof(double) - 1) / sizeof(double)))) return -1;
@@ -3052,7 +3090,11 @@ int mirrorAll(alis_dev_world *D, bool &done)
 	work(0, threads);
 	for (int t = alone; alone && t < threads; t++) work(t, threads);
 	for (std::thread &t : pool) t.join();
-	for (hipError_t e : err) if (e != hipSuccess) return fail("copy to the host arrays", e);
+	for (hipError_t e : err)
+		if (e != hipSuccess) {
+			(void)hipStreamSynchronize(D->st);     // no kernel writes to the stage once it is given back
+			return fail("copy to the host arrays", e);
+		}
 	done = true;
 	return 0;
 }

@@ -248,3 +248,32 @@ for current in (1, 0):
         assert now.value == current
 assert rec.hipRecForeign() == 0
 """)
+
+
+def test_commits_syncs_and_releases_beside_a_whole_sync(libs):
+    """While one thread waits inside a whole sync, another commits, steps, syncs and releases a world."""
+    run(libs, """
+import time
+A = ec.ec_world(64, 0, 1)
+ec.ec_step(A, 1)
+dA = ec.ec_device(A)
+rec.hipRecHold()
+first = threading.Thread(target=lambda: ok(lib.alis_dev_sync(dA, 0, -1, 0, -1, 0, -1)))
+first.start()
+while not rec.hipRecWaiting():
+    time.sleep(0.01)
+
+def other():
+    B = V(ec.ec_world(40, 0, 1))
+    ec.ec_step(B, 1)
+    ok(lib.alis_dev_sync(ec.ec_device(B), 0, -1, 0, -1, 0, -1))
+    ec.ec_free(B)
+
+second = threading.Thread(target=other, daemon=True)
+second.start()
+second.join(20)
+late = second.is_alive()
+rec.hipRecLetGo()
+first.join()
+assert not late
+""")
