@@ -30,7 +30,7 @@ static pthread_cond_t changed = PTHREAD_COND_INITIALIZER;
 
 static char *text;
 static size_t used, room;
-static int nstreams, waiting, nevents, npinned;
+static int nstreams, waiting, nevents, npinned, pinnedNow;
 static long outside, foreign;
 
 static void say(const char *what, const char *name, long n, int s)
@@ -49,7 +49,8 @@ void hipRecClear(void) { if (text) text[used = 0] = 0; }
 long hipRecOutside(void) { return outside; }
 long hipRecForeign(void) { return foreign; }
 int hipRecStreamOf(void *s) { return ((stream *)s)->id; }
-int hipRecPinned(void) { return npinned; }
+int hipRecPinned(void) { return npinned; }              /* pinned allocations made, and held now */
+int hipRecPinnedNow(void) { return pinnedNow; }
 
 /* The next wait for an event blocks until hipRecLetGo (once): hipRecWaiting tells that one does. */
 static int hold;
@@ -93,8 +94,8 @@ int hipFree(void *p)
 	return OK;
 }
 
-int hipHostMalloc(void **p, size_t n, unsigned flags) { (void)flags; *p = calloc(1, n); npinned++; return OK; }
-int hipHostFree(void *p) { free(p); return OK; }
+int hipHostMalloc(void **p, size_t n, unsigned flags) { (void)flags; *p = calloc(1, n); npinned++, pinnedNow++; return OK; }
+int hipHostFree(void *p) { free(p); pinnedNow--; return OK; }
 int hipMemcpyAsync(void *dst, const void *src, size_t n, int kind, void *s) { (void)kind, (void)s; memcpy(dst, src, n); return OK; }
 int hipMemsetAsync(void *dst, int v, size_t n, void *s) { (void)s; memset(dst, v, n); return OK; }
 

@@ -277,3 +277,28 @@ rec.hipRecLetGo()
 first.join()
 assert not late
 """)
+
+
+@pytest.mark.parametrize("sphere", [0, 1])
+def test_worlds_one_after_another_share_the_staging(libs, sphere):
+    """A program that solves one world after another pays for the pinned chunks of its whole syncs once;
+    worlds that pass without a whole sync give them back."""
+    run(libs, f"""
+def solve(sync):
+    W = V(ec.ec_world(64, 0, {sphere}))
+    ec.ec_step(W, 1)
+    if sync:
+        ok(lib.alis_dev_sync(ec.ec_device(W), 0, -1, 0, -1, 0, -1))
+    before = rec.hipRecPinned()
+    ec.ec_free(W)
+    return before
+
+first = solve(True)
+assert first > 0
+for _ in range(3):
+    assert solve(True) == first         # (allocated so far: nothing new)
+for _ in range(2):
+    solve(False)
+assert rec.hipRecPinnedNow() == 0
+assert solve(True) == 2 * first
+""")
