@@ -1810,16 +1810,25 @@ int zSamples(alis_dev_world *D, PhsZ<T> *zs, std::vector<DevPhaser *> &owners, b
 	return n;
 }
 
+// Whether strips recorded for half step h read an auxiliary world that steps on another stream.
+bool stripsBeside(const alis_dev_world *D, int h)
+{
+	for (size_t s = 0; s < D->tf.size(); s++)
+		if (((D->pendStrips[h] >> s) & 1u) && D->tf[s].aux->st != D->st) return true;
+	return false;
+}
+
 // What the curl of half step h makes of its end: 1 the copies along z that it can, 2 and the strips
-// and sources.
-int curlMakes(const alis_dev_world *D, int h) { return D->addsInCurl[h] ? 2 : 1; }
+// and sources.  An auxiliary world on another stream steps beside the curl, so its strips stay out of it
+// and only the end waits for that world (us a step, curl after it -> beside it: two TF/SF boxes in 200^3
+// 213 -> 161, oblique incidence on a 160^3 Bloch cell 224 -> 165, on 128^3 with PML 143 -> 103).
+int curlMakes(const alis_dev_world *D, int h) { return D->addsInCurl[h] && !stripsBeside(D, h) ? 2 : 1; }
 
 // The additive operations of part m that this half step's curl applies.
 template<class T>
-AddArgs<T> addArgs(const alis_dev_world *D, int h, int m, bool whole)
+AddArgs<T> addArgs(const alis_dev_world *D, int h, int m)
 {
 	AddArgs<T> a{};
-	if (!whole || !D->addsInCurl[h]) return a;
 	a.add = (const StepAdd<T> *)D->addTab[m][h], a.at = (const unsigned long long *)D->addTile[m][h];
 	for (size_t u = 0; u < D->adds[m][h].size(); u++) {
 		const alis_dev_world::AddRef &r = D->adds[m][h][u];
@@ -1830,11 +1839,10 @@ AddArgs<T> addArgs(const alis_dev_world *D, int h, int m, bool whole)
 	return a;
 }
 
-// whole: the launch also does what it can of the end of the half step (curlMakes), and the rest of
-// that program follows.
+// made: what the launch also does of the end of the half step (curlMakes), whose rest follows, or 0.
 // x: an auxiliary world's share of the launch, or null.
 template<class T>
-int coreHalf(alis_dev_world *D, int h, bool whole = false, const AuxCurl<T> *x = nullptr)
+int coreHalf(alis_dev_world *D, int h, int made = 0, const AuxCurl<T> *x = nullptr)
 {
 	dropPresamples(D);
 	hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1846,8 +1854,8 @@ int coreHalf(alis_dev_world *D, int h, bool whole = false, const AuxCurl<T> *x =
 	std::vector<DevPhaser *> sampled;
 	for (int m = 0; m <= D->cplx; m++) {
 		HalfArgs<T> a = halfArgs<T>(D, h, m);
-		if (!whole || m < D->cplx) a.ends = 0;
-		const AddArgs<T> adds = addArgs<T>(D, h, m, whole);
+		if (!made || m < D->cplx) a.ends = 0;
+		const AddArgs<T> adds = made == 2 ? addArgs<T>(D, h, m) : AddArgs<T>{};
 		ZFaces<T> z{};
 		const bool aux = x && m == 0;
 		const dim3 grid(a.tiles, a.ni + (aux ? 1 : 0)), block(CURL_WG);
@@ -2402,12 +2410,11 @@ int postWaiting(alis_dev_world *D)
 	return rc;
 }
 
-// The end of half step h after a whole curl.  E's ghost copies wait for H's where they are all that is
+// The end of half step h after a curl that made `made` of it.  E's ghost copies wait for H's where they are all that is
 // left of E's program: 40^3 dipole, 4 launches a step -> 3.
 template<class T>
-int endHalf(alis_dev_world *D, int h, const PostArgs<T> *x)
+int endHalf(alis_dev_world *D, int h, int made, const PostArgs<T> *x)
 {
-	const int made = curlMakes(D, h);
 	const bool alone = D->tf.empty() || (D->tf.size() == 1 && (!D->tf[0].aux || D->tf[0].aux->st == D->st));   // (released: null)
 	if (h == 0 && made == 2 && !x && !D->isAux && alone) {
 		size_t programs = 0;
@@ -2445,7 +2452,7 @@ int foldedHalf(alis_dev_world *D, int h)
 		x.part[m] = halfArgs<T>(A, h, m);
 		if (m < A->cplx) x.part[m].ends = 0;
 	}
-	for (int m = 0; m <= A->cplx; m++) x.adds[m] = addArgs<T>(A, h, m, true);
+	for (int m = 0; m <= A->cplx; m++) x.adds[m] = addArgs<T>(A, h, m);
 	PostArgs<T> last = postArgs<T>(A, h);               // (its sources are in x.adds)
 	// its copies: in the curl launch too, but for a last program of many cells
 	PostArgs<T> *rest = nullptr;
@@ -2462,8 +2469,9 @@ int foldedHalf(alis_dev_world *D, int h)
 	}
 	if (!D->postBuilt && buildPost<T>(D)) return -1;
 	if (rest && postWaiting<T>(D)) return -1;
-	if (coreHalf<T>(D, h, true, &x)) return -1;
-	return endHalf<T>(D, h, rest);
+	const int made = curlMakes(D, h);
+	if (coreHalf<T>(D, h, made, &x)) return -1;
+	return endHalf<T>(D, h, made, rest);
 }
 
 // made: what the curl has done of it (curlMakes), or 0.  x: an auxiliary world's launch to take along, or null.
@@ -2874,9 +2882,10 @@ int ghostsEntry(alis_dev_world *D, int h)
 	if (D->pendMain == 1 + h && !D->pendFold) {
 		D->pendMain = 0;
 		if (!D->postBuilt && buildPost<T>(D)) return -1;
-		// the strips read the auxiliary worlds' fields in the curl
-		if (waitForAux(D, D->pendStrips[h]) || coreHalf<T>(D, h, true)) return -1;
-		return endHalf<T>(D, h, nullptr);
+		const int made = curlMakes(D, h);
+		// (where the curl makes the strips, the auxiliary worlds they read must have made their half step)
+		if ((made == 2 && waitForAux(D, D->pendStrips[h])) || coreHalf<T>(D, h, made)) return -1;
+		return endHalf<T>(D, h, made, nullptr);
 	}
 	if (h == 1 && D->pendH == 1) {
 		D->pendH = 2;

@@ -302,3 +302,23 @@ for _ in range(2):
 assert rec.hipRecPinnedNow() == 0
 assert solve(True) == 2 * first
 """)
+
+
+@pytest.mark.parametrize("percent", [25, 60])
+def test_auxiliary_worlds_step_beside_the_curl(libs, percent):
+    """Auxiliary worlds on streams of their own (two TF/SF boxes): the main world's curl is launched before its
+    stream waits for them, and the launch that applies their strips after."""
+    run(libs, f"""
+W = ec.ec_boxes(64, 2, 0, {percent})
+ec.ec_step(W, 2)
+log = calls(ec.ec_step, W, 2)
+main = max((c for c in log if c[0] == "launch" and c[1].startswith("k_curl")), key=lambda c: c[3])[4]
+seen = []
+for c in log:
+    if c[0] == "wait" and c[1] == main:
+        seen.append("w")
+    elif c[0] == "launch" and c[4] == main:
+        seen.append(c[1][2])
+order = "".join(seen)
+assert re.fullmatch("(c(w+)p)+", order) and order.count("c") == 4, order
+""")
