@@ -26,6 +26,16 @@ world ec_boxes(int cells, int boxes, int sphere, int percent)
 	return W;
 }
 
+/* A focused beam: a source with a phase per cell, of `steps` steps. */
+world ec_beam(int cells, int steps)
+{
+	world W = ec_boxes(cells, 0, 0, 60);
+	removeSources(W);
+	focusedBeam(W, W->Dom, Ex, 0, 0, 0, 180, Sine, 600, 3, 1.5);
+	for (source S = W->SE; S; S = S->S) S->N = steps;
+	return W;
+}
+
 world ec_world(int cells, int boxes, int sphere) { return ec_boxes(cells, boxes, sphere, 60); }
 void ec_step(world W, int n) { for (int s = 0; s < n; s++) updateE(W), updateH(W); }
 void ec_free(world W) { deleteWorld(W); }
@@ -65,3 +75,16 @@ int ec_commit_below(world W, int below)
 	if (!rc) alis_dev_release(D);
 	return rc;
 }
+
+/* The real part of one field array of W as alis_dev_read_field gives it: the values, or 0 for too small a
+ * buffer. */
+long ec_field(world W, int h, int axis, double *out, long room)
+{
+	const long n = (long)(W->iNUM + 2) * (W->jNUM + 2) * (W->kNUM + 2);
+	if (n > room) return 0;
+	alisFatal("read", alis_dev_read_field(W->dev, h, 0, axis, out));
+	return n;
+}
+
+/* W[0..n-1] together. */
+void ec_step_many(world *W, int n, int steps) { for (int s = 0; s < steps; s++) updateWorldsE(W, n), updateWorldsH(W, n); }

@@ -18,7 +18,7 @@ ec = ctypes.CDLL(sys.argv[1] + "/engine_client.so")
 rec.hipRecLog.restype = lib.alis_dev_error.restype = ctypes.c_char_p
 rec.hipRecOutside.restype = ctypes.c_long
 rec.hipRecStreamOf.argtypes = [V]
-ec.ec_world.restype = ec.ec_boxes.restype = ec.ec_device.restype = ec.ec_aux.restype = V
+ec.ec_world.restype = ec.ec_boxes.restype = ec.ec_beam.restype = ec.ec_device.restype = ec.ec_aux.restype = V
 ec.ec_step.argtypes = ec.ec_aux.argtypes = ec.ec_commit_below.argtypes = [V, I]
 ec.ec_device.argtypes = ec.ec_free.argtypes = ec.ec_disown.argtypes = [V]
 lib.alis_dev_core.argtypes = lib.alis_dev_ghosts.argtypes = [V, I]
@@ -321,4 +321,28 @@ for c in log:
         seen.append(c[1][2])
 order = "".join(seen)
 assert re.fullmatch("(c(w+)p)+", order) and order.count("c") == 4, order
+""")
+
+
+@pytest.mark.parametrize("shared", [False, True])
+def test_core_runs_while_the_host_evaluates_waves(libs, shared):
+    """A source with per-cell waves: the E core is launched at its call, before the host evaluates them for the
+    end of the half step; without such waves, or once they have ended, it waits for that call."""
+    run(libs, f"""
+shared = {shared}
+W = [V(ec.ec_beam(40, 4)) for _ in range(2)]
+for w in W:
+    ec.ec_step(w, 2)
+dev = [ec.ec_device(w) for w in W]
+B = batch(dev) if shared else None
+curl = "k_curl_batch" if shared else "k_curl"
+core = lambda h: ok(lib.alis_dev_batch_core(B, h) if shared else lib.alis_dev_core(dev[0], h))
+end = lambda h: ok(lib.alis_dev_batch_post(B, h) if shared else lib.alis_dev_ghosts(dev[0], h))
+for waves in (True, False):              # (the second step here records none)
+    assert kernels(calls(core, 0)) == ([curl] if waves else [])
+    assert (curl in kernels(calls(end, 0))) == (not waves)
+    assert kernels(calls(core, 1)) == []
+    assert curl in kernels(calls(end, 1))[0]
+if shared:
+    lib.alis_dev_batch_release(B)
 """)

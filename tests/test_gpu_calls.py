@@ -1,6 +1,9 @@
 """Batches of Bloch worlds (complex fields, CPML along z) in other ways than updateWorldsE/H: FP32 fields
 bit for bit the CPU oracle's, after enough steps that the fields reach the ends of z."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -74,3 +77,44 @@ def _ends_apart(e, B, dev):
 def test_half_steps_of_single_and_shared_calls(program):
     got, ref = _fields("hip", program), _fields("oracle", program)
     assert np.abs(ref).max() > 0 and np.array_equal(got, ref)
+
+
+BEAMS = r'''
+import ctypes, sys
+import numpy as np
+V, I = ctypes.c_void_p, ctypes.c_int
+ctypes.CDLL(sys.argv[2], mode=ctypes.RTLD_GLOBAL)
+ec = ctypes.CDLL(sys.argv[1])
+ec.ec_beam.restype, ec.ec_field.restype = V, ctypes.c_long
+ec.ec_step.argtypes, ec.ec_step_many.argtypes = [V, I], [V, I, I]
+ec.ec_field.argtypes = [V, I, I, V, ctypes.c_long]
+W = (V * 2)(*[ec.ec_beam(n, 20) for n in (40, 43)])
+if int(sys.argv[4]):
+    ec.ec_step_many(W, 2, 45)
+else:
+    for w in W:
+        ec.ec_step(w, 45)
+out, buf = [], np.zeros(200000)
+for w in W:
+    for h in range(2):
+        for a in range(3):
+            n = ec.ec_field(w, h, a, buf.ctypes.data, buf.size)
+            assert n > 0
+            out.append(buf[:n].copy())
+np.save(sys.argv[3], np.concatenate(out))
+'''
+
+
+@pytest.mark.parametrize("shared", [0, 1])
+def test_waves_per_cell(tmp_path, shared):
+    """Focused beams, whose core runs at its call while the source is on and waits once it has ended."""
+    client = tmp_path / "engine_client.so"
+    subprocess.run(["gcc", "-O1", "-std=gnu99", "-shared", "-fPIC", f"-I{ROOT / 'include'}", "-o", str(client),
+                    str(ROOT / "tests" / "engine_client.c")], check=True)
+    got = {}
+    for kind in LIBS:
+        print(f"[gpu] two beams, {kind}, together: {shared}", flush=True)
+        subprocess.run([sys.executable, "-c", BEAMS, str(client), str(LIBS[kind][1]), str(tmp_path / f"{kind}.npy"), str(shared)],
+                       check=True, timeout=100, env={**os.environ, "ALIS_PRECISION": "fp32"})
+        got[kind] = np.load(tmp_path / f"{kind}.npy")
+    assert np.abs(got["oracle"]).max() > 0 and np.array_equal(got["hip"], got["oracle"])
