@@ -202,14 +202,16 @@ constexpr int MAXCHAIN = 24;    // copies per launch
 constexpr int MAXPOST = 48;     // operations per launch
 constexpr int POST_WG = 64;     // threads per workgroup of k_post: one wavefront (64 k-point worlds:
                                 // H program 84 -> 79 us, E 35 -> 31 us against 256)
-constexpr int POST_U = 4, POST_BLK = POST_WG * POST_U;   // cells per thread, per workgroup
+constexpr int POST_U = 4;       // most cells per thread of a piece
+constexpr long POST_WAVES = 256 * 32;   // wavefronts that the chip holds at a time
 
 struct PostPiece {
 	int kind;                   // OP_COPY, or OP_STRIP for an additive piece
 	int n;                      // operations in list
 	int si, sj, sk;             // copy piece: base cell - cell
 	Box b;                      // the cells
-	long off;                   // first cell in the launch (a multiple of POST_BLK)
+	int u;                      // cells per thread: POST_U, or 1 (additive pieces, see buildPieces)
+	int wg;                     // its first workgroup in the launch
 	unsigned rk, rj;            // 2^32 over the cells along k, along j (recip32)
 	unsigned char list[MAXPOST];// operation indices (copy piece: its chain, last copy first)
 };
@@ -263,8 +265,12 @@ __device__ __forceinline__ int divBy(int t, int d, unsigned r)
 // dependent loads (piece, operation, cell) where a search of the pieces added about seven
 // (measured with 256-thread workgroups: 64 k-point worlds' H program 95 -> 84 us; 256^3
 // nanoblock H program 17.5 -> 16.1 us).  That chain is what bounds it: piece and operation come
-// through the scalar cache, and a thread takes POST_U cells, whose loads are in flight together
-// (256^3 H program with its current update 23 -> 18 us, 64 spheres 42 -> 36, 6 worlds 32 -> 27).
+// through the scalar cache, and a thread takes POST_U cells of a copy piece, whose loads are in flight
+// together (400x400x200, 165 000 threads 8.5 -> 6.6 us).  An additive piece is a chain of its own per cell
+// (1/eps and auxiliary value per operation), so a thread takes one where the chip then still holds all
+// wavefronts (with POST_U: strips of 256^3 6.2 -> 9.0 us, with 64 spheres 8.6 -> 11.8, of 6 worlds 7.0 ->
+// 12.1; 9.0 -> 9.8, 32.8 -> 32.4 and 14.1 -> 13.1 where the launch holds copies and the current update too),
+// and POST_U beyond (645 000 cells of 400x400x200: one 40.6, POST_U 39.7, and the curl after it 274, 271).
 // tid: the thread's place in the workgroup; ADDS: pieces may be additive.
 template<class T, bool ADDS = true, class A>
 __device__ __forceinline__ void postCells(const A &a, const PostOp<T> *allOps, const PostPiece *pieces, int blk, int tid)
@@ -272,21 +278,24 @@ __device__ __forceinline__ void postCells(const A &a, const PostOp<T> *allOps, c
 	const auto &P = uniform(pieces)[blk];
 	const auto *const ops = uniform(allOps);
 	const int nk = P.b.k1 - P.b.k0 + 1, nj = P.b.j1 - P.b.j0 + 1, count = (P.b.i1 - P.b.i0 + 1) * nj * nk;
-	const int t0 = blk * POST_BLK + tid - (int)P.off;
 	const auto &o = ops[P.list[0]];
 	T *const F = o.F, *const G = o.G;
-	int i[POST_U], j[POST_U], k[POST_U];
-	long d[POST_U];
-	T f[POST_U], g[POST_U];
-#pragma unroll
-	for (int u = 0; u < POST_U; u++) {
-		// cells beyond the piece repeat its last one's loads and store nothing
-		const int t = min(t0 + u * POST_WG, count - 1), r = divBy(t, nk, P.rk), di = divBy(r, nj, P.rj);
-		i[u] = P.b.i0 + di, j[u] = P.b.j0 + r - di * nj, k[u] = P.b.k0 + t - r * nk;
-		d[u] = layAt(o.LF, i[u], j[u], k[u]);
-	}
+	auto place = [&](int t, int &i, int &j, int &k) {
+		const int r = divBy(t, nk, P.rk), di = divBy(r, nj, P.rj);
+		i = P.b.i0 + di, j = P.b.j0 + r - di * nj, k = P.b.k0 + t - r * nk;
+		return layAt(o.LF, i, j, k);
+	};
 	if (P.kind == OP_COPY) {
+		const int t0 = (blk - P.wg) * POST_WG * POST_U + tid;
 		const long off = layAt(o.LF, P.si, P.sj, P.sk) - layAt(o.LF, 0, 0, 0);
+		long d[POST_U];
+		T f[POST_U], g[POST_U];
+#pragma unroll
+		for (int u = 0; u < POST_U; u++) {
+			// cells beyond the piece repeat its last one's loads and store nothing
+			int i, j, k;
+			d[u] = place(min(t0 + u * POST_WG, count - 1), i, j, k);
+		}
 #pragma unroll
 		for (int u = 0; u < POST_U; u++) f[u] = glb(F)[d[u] + off], g[u] = G ? glb(G)[d[u] + off] : T(0);
 		for (int x = P.n - 1; x >= 0; x--) {
@@ -308,22 +317,33 @@ __device__ __forceinline__ void postCells(const A &a, const PostOp<T> *allOps, c
 		return;
 	}
 	if constexpr (ADDS) {
-		bool on = false;
-		for (int x = 0; x < P.n; x++) {
-			const auto &r = ops[P.list[x]];
-			if (!opOn(a, r)) continue;
-			if (!on)
+		auto add = [&](auto cells) {
+			constexpr int U = decltype(cells)::value;
+			const int t0 = (blk - P.wg) * POST_WG * U + tid;
+			int i[U], j[U], k[U];
+			long d[U];
+			T f[U];
 #pragma unroll
-				for (int u = 0; u < POST_U; u++) f[u] = glb(F)[d[u]];
-			on = true;
-			const T wave = r.kind == OP_SOURCE ? a.wave[r.slot] : T(0);
+			for (int u = 0; u < U; u++) d[u] = place(min(t0 + u * POST_WG, count - 1), i[u], j[u], k[u]);
+			bool on = false;
+			for (int x = 0; x < P.n; x++) {
+				const auto &r = ops[P.list[x]];
+				if (!opOn(a, r)) continue;
+				if (!on)
 #pragma unroll
-			for (int u = 0; u < POST_U; u++) f[u] = addTo<T>(r, f[u], i[u], j[u], k[u], wave);
-		}
-		if (!on) return;
+					for (int u = 0; u < U; u++) f[u] = glb(F)[d[u]];
+				on = true;
+				const T wave = r.kind == OP_SOURCE ? a.wave[r.slot] : T(0);
 #pragma unroll
-		for (int u = 0; u < POST_U; u++)
-			if (t0 + u * POST_WG < count) glb(F)[d[u]] = f[u];
+				for (int u = 0; u < U; u++) f[u] = addTo<T>(r, f[u], i[u], j[u], k[u], wave);
+			}
+			if (!on) return;
+#pragma unroll
+			for (int u = 0; u < U; u++)
+				if (t0 + u * POST_WG < count) glb(F)[d[u]] = f[u];
+		};
+		if (P.u == 1) add(std::integral_constant<int, 1>{});
+		else add(std::integral_constant<int, POST_U>{});
 	}
 }
 
@@ -945,10 +965,9 @@ struct DevSrc {
 
 struct PostSeg {
 	void *ops = nullptr;        // PostOp<T>[] in device memory
-	void *pieces = nullptr;     // PostPiece[total / POST_BLK] in device memory: each workgroup's
-	                            //  piece
-	long total = 0;             // cells (a multiple of POST_BLK)
-	// the cells stand in this order: copies, strips and sources (up to `rest`), and the copies that the
+	void *pieces = nullptr;     // PostPiece[total] in device memory: each workgroup's piece
+	long total = 0;             // workgroups
+	// these stand in this order: copies, strips and sources (up to `rest`), and the copies that the
 	// curl can make (see rowCopyOf); bare: the first alone
 	long rest = 0, bare = 0;
 };
@@ -1332,6 +1351,8 @@ bool cellWork(const std::vector<PostOp<T>> &v, int nadd, int p, int i, int j, in
 	return true;
 }
 
+long workgroups(const PostPiece &P) { return (P.b.count() + POST_WG * P.u - 1) / (POST_WG * P.u); }
+
 // Compile a launch's program into pieces: per operation, the cells of its box labelled by
 // their work, then grown greedily into boxes of equal work (along k, then j, then i).
 template<class T>
@@ -1389,11 +1410,17 @@ void buildPieces(const std::vector<PostOp<T>> &v, int nadd, std::vector<PostPiec
 					P.n = (int)K.size() - 4;
 					for (int u = 0; u < P.n; u++) P.list[u] = (unsigned char)K[4 + u];
 					P.b = Box{b.i0 + di, b.i0 + di1, b.j0 + dj, b.j0 + dj1, b.k0 + dk, b.k0 + dk1};
-					P.off = total;
 					P.rk = recip32(P.b.k1 - P.b.k0 + 1), P.rj = recip32(P.b.j1 - P.b.j0 + 1);
-					total += (P.b.count() + POST_BLK - 1) / POST_BLK * POST_BLK;
 					out.push_back(P);
 				}
+	}
+	// An additive piece takes one cell per thread while the chip holds all its launch's wavefronts at once.
+	long add = 0;
+	for (const PostPiece &P : out) if (P.kind != OP_COPY) add += P.b.count();
+	for (PostPiece &P : out) {
+		P.u = P.kind != OP_COPY && add <= POST_WAVES * POST_WG ? 1 : POST_U;
+		P.wg = (int)total;
+		total += workgroups(P);
 	}
 }
 
@@ -2058,22 +2085,24 @@ int postSegment(alis_dev_world *D, const std::vector<PostOp<T>> &v, int nadd, st
 			back.push_back(part(P, b));
 			for (const Box &x : outsideParts(P.b, b)) front.push_back(part(P, x));
 		}
-		long off = 0;
-		auto place = [&](PostPiece &P) { P.off = off, off += (P.b.count() + POST_BLK - 1) / POST_BLK * POST_BLK; };
+		long wg = 0;
+		auto place = [&](PostPiece &P) { P.wg = (int)wg, wg += workgroups(P); };
 		for (PostPiece &P : front) place(P);
-		seg.bare = off;
+		seg.bare = wg;
 		for (PostPiece &P : middle) place(P);
-		seg.rest = off;
+		seg.rest = wg;
 		for (PostPiece &P : back) place(P);
-		seg.total = off;
+		seg.total = wg;
 		pieces = front;
 		pieces.insert(pieces.end(), middle.begin(), middle.end());
 		pieces.insert(pieces.end(), back.begin(), back.end());
 	}
-	if (seg.total >= (1L << 31)) return fail("end-of-half-step launch over 2^31 threads");
-	std::vector<PostPiece> perBlock(seg.total / POST_BLK);
+	long cells = 0;
+	for (const PostPiece &P : pieces) cells += workgroups(P) * POST_WG * P.u;
+	if (cells >= (1L << 31)) return fail("end-of-half-step launch over 2^31 cells");
+	std::vector<PostPiece> perBlock(seg.total);
 	for (const PostPiece &P : pieces)
-		for (long b = P.off / POST_BLK; b < (P.off + P.b.count() + POST_BLK - 1) / POST_BLK; b++) perBlock[b] = P;
+		for (long b = P.wg; b < P.wg + workgroups(P); b++) perBlock[b] = P;
 	if (devAlloc(D, &seg.ops, v.size() * sizeof(PostOp<T>))) return -1;
 	if (devAlloc(D, &seg.pieces, perBlock.size() * sizeof(PostPiece))) return -1;
 	HIPCHECK(hipMemcpyAsync(seg.ops, v.data(), v.size() * sizeof(PostOp<T>), hipMemcpyHostToDevice, D->st));
@@ -2393,7 +2422,7 @@ int foldsAux(alis_dev_world *D, bool &on)
 			if (!A->addsInCurl[h]) return 0;
 			if (A->post[h].size() > (size_t)AUX_SEGS) return 0;
 			for (size_t g = 0; g + 1 < A->post[h].size(); g++)
-				if (A->post[h][g].bare > AUX_CELLS) return 0;
+				if (A->post[h][g].bare > AUX_WGS) return 0;
 		}
 		if (joinStream(A, D)) return -1;
 		D->foldState = 1;
@@ -2439,7 +2468,7 @@ int endHalf(alis_dev_world *D, int h, int made, const PostArgs<T> *x)
 	if (h == 1 && D->pendPost && !x) {
 		PostArgs<T> e{};
 		for (const PostSeg &G : D->post[0])
-			if (G.bare) e.ops = (const PostOp<T> *)G.ops, e.pieces = (const PostPiece *)G.pieces, e.post = (int)(G.bare / POST_BLK);
+			if (G.bare) e.ops = (const PostOp<T> *)G.ops, e.pieces = (const PostPiece *)G.pieces, e.post = (int)G.bare;
 		D->pendPost = false;
 		return postHalf<T>(D, 1, made, &e);
 	}
@@ -2470,13 +2499,13 @@ int foldedHalf(alis_dev_world *D, int h)
 	for (size_t g = 0; g < A->post[h].size(); g++) {
 		const PostSeg &G = A->post[h][g];
 		if (!G.bare) continue;
-		if (g + 1 == A->post[h].size() && G.bare > AUX_CELLS) {
+		if (g + 1 == A->post[h].size() && G.bare > AUX_WGS) {
 			last.ops = (const PostOp<T> *)G.ops, last.pieces = (const PostPiece *)G.pieces;
-			last.post = (int)(G.bare / POST_BLK), rest = &last;
+			last.post = (int)G.bare, rest = &last;
 			break;
 		}
 		x.seg[x.segs].ops = (const PostOp<T> *)G.ops, x.seg[x.segs].pieces = (const PostPiece *)G.pieces;
-		x.seg[x.segs++].n = (int)(G.bare / POST_BLK);
+		x.seg[x.segs++].n = (int)G.bare;
 	}
 	if (!D->postBuilt && buildPost<T>(D)) return -1;
 	if (rest && postWaiting<T>(D)) return -1;
@@ -2503,14 +2532,14 @@ int postHalf(alis_dev_world *D, int h, int made, const PostArgs<T> *x)
 	for (size_t s = 0; s < D->tf.size(); s++) bind = bind || sideStream(s);
 	if (bind && !D->halfDone) HIPCHECK(hipEventCreateWithFlags(&D->halfDone, hipEventDisableTiming));
 	int last = -1;
-	auto cells = [&](const PostSeg &G) { return made == 2 ? G.bare : made ? G.rest : G.total; };
-	for (int g = 0; g < (int)D->post[h].size(); g++) if (cells(D->post[h][g])) last = g;
+	auto groups = [&](const PostSeg &G) { return made == 2 ? G.bare : made ? G.rest : G.total; };
+	for (int g = 0; g < (int)D->post[h].size(); g++) if (groups(D->post[h][g])) last = g;
 	for (int g = 0; g <= last; g++) {
 		const PostSeg &G = D->post[h][g];
-		if (!cells(G)) continue;
+		if (!groups(G)) continue;
 		a.ops = (const PostOp<T> *)G.ops;
 		a.pieces = (const PostPiece *)G.pieces;
-		a.post = (int)(cells(G) / POST_BLK);
+		a.post = (int)groups(G);
 		unsigned blocks = a.post;
 		if (g == last && h == 1 && D->pendAde) a.ade = objArgs<T>(D), blocks += objBlocks(D), D->pendAde = false;
 		if (g == last && x) launchEv(k_post_aux<T>, dim3(blocks + x->post), dim3(POST_WG), 0, D->st, nullptr, bind ? D->halfDone : nullptr, a, *x, (int)blocks);
@@ -2775,7 +2804,7 @@ int fusedStep(alis_dev_world *D)
 	for (const PostSeg &G : D->copies) {
 		a.ops = (const PostOp<T> *)G.ops;
 		a.pieces = (const PostPiece *)G.pieces;
-		a.post = (int)(G.total / POST_BLK);
+		a.post = (int)G.total;
 		unsigned blocks = a.post;
 		a.ade = ObjArgs<T>{};
 		if (D->pendAde) a.ade = objArgs<T>(D), blocks += objBlocks(D), D->pendAde = false;
@@ -3536,7 +3565,7 @@ int batchBuildPost(alis_dev_batch *B, bool copied)
 			for (int w = 0; w < (int)B->W.size(); w++) {
 				alis_dev_world *D = B->W[w];
 				if (r >= D->post[h].size()) continue;
-				long blocks = (copied ? D->post[h][r].rest : D->post[h][r].total) / POST_BLK;
+				long blocks = copied ? D->post[h][r].rest : D->post[h][r].total;
 				// the current update runs with a world's last H launch
 				if (h == 1 && r + 1 == D->post[h].size()) blocks += objBlocks(D);
 				if (!blocks) continue;
@@ -3630,7 +3659,7 @@ int batchPostArgs(alis_dev_batch *B, int h, bool whole, bool copied)
 			memset(&a[e], 0, sizeof(PostArgs<T>));
 			a[e].ops = (const PostOp<T> *)g.ops;
 			a[e].pieces = (const PostPiece *)g.pieces;
-			a[e].post = (int)((copied ? g.rest : g.total) / POST_BLK);
+			a[e].post = (int)(copied ? g.rest : g.total);
 			if (h == 1 && R.seg[e] + 1 == (int)D->post[h].size() && (whole ? D->objWgs > 0 : D->pendAde)) a[e].ade = objArgs<T>(D);
 			a[e].strips = D->pendStrips[h];
 			for (size_t w = 0; w < D->pendSrc[h].size(); w++) a[e].src[w] = D->pendSrc[h][w];

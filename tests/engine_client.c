@@ -88,3 +88,17 @@ long ec_field(world W, int h, int axis, double *out, long room)
 
 /* W[0..n-1] together. */
 void ec_step_many(world *W, int n, int steps) { for (int s = 0; s < steps; s++) updateWorldsE(W, n), updateWorldsH(W, n); }
+
+/* cells x cells x 4 nodes, periodic, with a uniform source over the whole upper plane and a dipole: more
+ * cells of strips and sources in one launch than the chip holds wavefronts' lanes, from 725 cells on. */
+world ec_plane(int cells)
+{
+	const float dx = 10, e = dx * cells / 2;
+	dom D = {{-e, e}, {-e, e}, {0, 3 * dx}};
+	res R = {5, {dx}, {1240}};
+	sur S = {{PBC}, {PBC}, {PBC}};
+	world W = createWorld(D, R, S, "");
+	focusedBeam(W, W->Dom, Ex, 0, 0, 0, 0, Sine, 600, 3);
+	pointDipole(W, Ez, 3 * dx, -5 * dx, dx, Pulse, 600, 240);
+	return W;
+}

@@ -346,3 +346,16 @@ for waves in (True, False):              # (the second step here records none)
 if shared:
     lib.alis_dev_batch_release(B)
 """)
+
+
+def test_strips_take_a_cell_per_thread(libs):
+    """The strips of two TF/SF boxes of 14 x 28 x 28 cells at the end of the E half step: two components on
+    each face, about 12500 cells, a wavefront (64 threads) to as many of them."""
+    run(libs, """
+W = ec.ec_boxes(64, 2, 0, 60)
+ec.ec_step(W, 2)
+log = calls(ec.ec_step, W, 1)
+main = max((c for c in log if c[0] == "launch" and c[1].startswith("k_curl")), key=lambda c: c[3])[4]
+post = [c[3] for c in log if c[0] == "launch" and c[4] == main and c[1].startswith("k_post")]
+assert len(post) == 2 and post[0] >= 12500 * 0.9 / 64, post
+""")

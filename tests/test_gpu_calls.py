@@ -85,16 +85,18 @@ import numpy as np
 V, I = ctypes.c_void_p, ctypes.c_int
 ctypes.CDLL(sys.argv[2], mode=ctypes.RTLD_GLOBAL)
 ec = ctypes.CDLL(sys.argv[1])
-ec.ec_beam.restype, ec.ec_field.restype = V, ctypes.c_long
+ec.ec_beam.restype = ec.ec_plane.restype = V
+ec.ec_field.restype = ctypes.c_long
 ec.ec_step.argtypes, ec.ec_step_many.argtypes = [V, I], [V, I, I]
 ec.ec_field.argtypes = [V, I, I, V, ctypes.c_long]
-W = (V * 2)(*[ec.ec_beam(n, 20) for n in (40, 43)])
-if int(sys.argv[4]):
+mode = sys.argv[4]
+W = (V * 1)(ec.ec_plane(730)) if mode == "plane" else (V * 2)(*[ec.ec_beam(n, 20) for n in (40, 43)])
+if mode == "together":
     ec.ec_step_many(W, 2, 45)
 else:
     for w in W:
-        ec.ec_step(w, 45)
-out, buf = [], np.zeros(200000)
+        ec.ec_step(w, 6 if mode == "plane" else 45)
+out, buf = [], np.zeros(4000000)
 for w in W:
     for h in range(2):
         for a in range(3):
@@ -105,16 +107,17 @@ np.save(sys.argv[3], np.concatenate(out))
 '''
 
 
-@pytest.mark.parametrize("shared", [0, 1])
-def test_waves_per_cell(tmp_path, shared):
-    """Focused beams, whose core runs at its call while the source is on and waits once it has ended."""
+@pytest.mark.parametrize("mode", ["alone", "together", "plane"])
+def test_sources_of_many_cells(tmp_path, mode):
+    """Focused beams, whose core runs at its call while the source is on and waits once it has ended; a uniform
+    source over a plane of 731 x 731 cells, which takes four cells per thread."""
     client = tmp_path / "engine_client.so"
     subprocess.run(["gcc", "-O1", "-std=gnu99", "-shared", "-fPIC", f"-I{ROOT / 'include'}", "-o", str(client),
                     str(ROOT / "tests" / "engine_client.c")], check=True)
     got = {}
     for kind in LIBS:
-        print(f"[gpu] two beams, {kind}, together: {shared}", flush=True)
-        subprocess.run([sys.executable, "-c", BEAMS, str(client), str(LIBS[kind][1]), str(tmp_path / f"{kind}.npy"), str(shared)],
+        print(f"[gpu] {mode}, {kind}", flush=True)
+        subprocess.run([sys.executable, "-c", BEAMS, str(client), str(LIBS[kind][1]), str(tmp_path / f"{kind}.npy"), mode],
                        check=True, timeout=100, env={**os.environ, "ALIS_PRECISION": "fp32"})
         got[kind] = np.load(tmp_path / f"{kind}.npy")
     assert np.abs(got["oracle"]).max() > 0 and np.array_equal(got["hip"], got["oracle"])
