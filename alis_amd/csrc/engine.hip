@@ -347,17 +347,19 @@ __device__ __forceinline__ void postCells(const A &a, const PostOp<T> *allOps, c
 	}
 }
 
-template<class T, class A>
+// ADE: the workgroups after those of the program run a current update (which takes more registers than the
+// program).
+template<class T, bool ADE, class A>
 __device__ __forceinline__ void postBlock(const A &a, int blk)
 {
-	if (blk < a.post) postCells<T>(a, a.ops, a.pieces, blk, (int)threadIdx.x);
-	else if (a.ade.blocks) adeBlock<T>(a.ade, blk - a.post);
+	if (!ADE || blk < a.post) postCells<T>(a, a.ops, a.pieces, blk, (int)threadIdx.x);
+	else adeBlock<T>(a.ade, blk - a.post);
 }
 
-template<class T>
+template<class T, bool ADE>
 __global__ __launch_bounds__(POST_WG) void k_post(PostArgs<T> a)
 {
-	postBlock<T>(a, (int)blockIdx.x);
+	postBlock<T, ADE>(a, (int)blockIdx.x);
 }
 
 // Several worlds' programs in one launch: entry e owns workgroups [start[e], start[e+1]).
@@ -366,7 +368,7 @@ __global__ __launch_bounds__(POST_WG) void k_post_batch(const PostArgs<T> *__res
 {
 	const int b = (int)blockIdx.x;
 	const int e = batchEntry(start, n, b);
-	postBlock<T>(uniform(args)[e], b - uniform(start)[e]);
+	postBlock<T, false>(uniform(args)[e], b - uniform(start)[e]);
 }
 
 #include "step_kernel.inc"
@@ -1090,7 +1092,9 @@ struct alis_dev_world {
 	void *stepArgs = nullptr;   // StepArgs<T>[2 parts][2 sets]: k_step's arguments per current set
 	void *objStart = nullptr, *objOver = nullptr;   // tables of the objects' launches (ObjArgs)
 	int objWgs = 0;             // workgroups of one component of one part
-	bool pendAde = false;       // the current update of the last H core is still to run
+	bool pendAde = false;       // the current update of the last H core is still to run: beside the
+	                            //  end of its half step (updateBeside), with the next E core, or
+	                            //  before anything that needs it (flushAde)
 	struct AddRef { int kind, slot; };
 	std::vector<AddRef> adds[2][2];   // [part][half]: the additive operations of the curl's lists
 	// their tables on the device (StepAdd<T>; bits per plane, and per workgroup of a curl launch)
@@ -1742,6 +1746,51 @@ ObjArgs<T> objArgs(const alis_dev_world *D)
 
 int objBlocks(const alis_dev_world *D) { return D->objWgs * 3 * (1 + D->cplx); }
 
+// Whether D's current update runs beside the end of the H half step (in its launch, a few workgroups
+// more) and not with the next E half step: where the objects take at most a workgroup per compute unit,
+// so that both are bound by latency alone.  Before E and the end of H, us a step, beside it and with E:
+// scatterer of 128^3 (192 workgroups) 4.4 + 5.4 and 5.6 + 4.9; of 256^3 (1578) 5.7 + 9.2 and 7.8 + 6.2, 64
+// spheres (13 641) 17.5 + 32.3 and 34.0 + 7.5.
+bool updateBeside(const alis_dev_world *D) { return objBlocks(D) <= 256; }
+
+// The current update of the last H core, where no launch took it along.
+template<class T>
+int flushAde(alis_dev_world *D)
+{
+	if (!D->pendAde) return 0;
+	D->pendAde = false;
+	k_ade<T><<<objBlocks(D), OBJ_WG, 0, D->st>>>(objArgs<T>(D));
+	HIPCHECK(hipGetLastError());
+	return 0;
+}
+
+// The bytes of D that a step passes over, but for CPML and 1/eps: its fields, its objects' arrays.
+long stepBytes(const alis_dev_world *D)
+{
+	long n = 6L * (1 + D->cplx) * D->fsize;
+	for (const DevObj &O : D->obj) n += 3 * O.n * (1 + (1 + D->cplx) * (2L * O.NK - O.NJ));
+	return n * (long)D->esz;
+}
+
+// Objects' arrays bypass the cache (256 MiB, the last level) where a step passes over more than it holds
+// with what else there is.  Worlds by their MiB, us a step cached and past the cache: 64 spheres in 200^3
+// (290) 33 and 37 a launch, metal 160^3 (190) 113 and 115, 4/5 of 200^3 (280) 167 and 168; metal 200^3 (370)
+// 202 and 196, dielectric with a pole pair 200^3 (460) 247 and 223, metal 256^3 (770) 431 and 376.
+constexpr long OBJECTS_NT = 320L << 20;
+
+// What D's objects do before the E curl.
+template<class T>
+int objectsBeforeE(alis_dev_world *D)
+{
+	if (!D->objWgs) return 0;
+	if (!D->pendAde) k_currents<T><<<objBlocks(D), OBJ_WG, 0, D->st>>>(objArgs<T>(D));
+	else if (stepBytes(D) > OBJECTS_NT) k_objects<T, true><<<objBlocks(D), OBJ_WG, 0, D->st>>>(objArgs<T>(D));
+	else k_objects<T, false><<<objBlocks(D), OBJ_WG, 0, D->st>>>(objArgs<T>(D));
+	D->pendAde = false;
+	HIPCHECK(hipGetLastError());
+	return 0;
+}
+
 // Make D use the stream of `to` (reference counted; the last user destroys a stream).
 int joinStream(alis_dev_world *D, alis_dev_world *to)
 {
@@ -1888,7 +1937,7 @@ int coreHalf(alis_dev_world *D, int h, int made = 0, const AuxCurl<T> *x = nullp
 		ZFaces<T> z{};
 		const bool aux = x && m == 0;
 		const dim3 grid(a.tiles, a.ni + (aux ? 1 : 0)), block(CURL_WG);
-		if (h == 0 && m == 0 && D->objWgs) k_currents<T><<<objBlocks(D), OBJ_WG, 0, D->st>>>(objArgs<T>(D));
+		if (m == 0 && (h == 0 ? objectsBeforeE<T>(D) : flushAde<T>(D))) return -1;
 		if (h == 1 && m == 0) z.n = zSamples<T>(D, z.z, sampled, false);   // phasers sample part 0
 		hipEvent_t s0 = m == 0 ? e0 : nullptr, s1 = m == D->cplx ? e1 : nullptr;
 #define CURL(H, C, Z) (aux && adds.on ? launchEv(k_curl_aux<T, H, C, Z, true>, grid, block, 0, D->st, s0, s1, a, *x, adds, z) : \
@@ -1901,7 +1950,7 @@ int coreHalf(alis_dev_world *D, int h, int made = 0, const AuxCurl<T> *x = nullp
 		else CURL(1, 0, false);
 #undef CURL
 	}
-	if (h == 1 && D->objWgs) D->pendAde = true;   // with the end of the half step (or flushStep)
+	if (h == 1) D->pendAde = D->objWgs > 0;
 	if (e1) {
 		D->evPairs[h].push_back(e0);
 		D->evPairs[h].push_back(e1);
@@ -2354,7 +2403,7 @@ int buildCopies(alis_dev_world *D)
 	return 0;
 }
 
-int flushE(alis_dev_world *D);
+int flushFields(alis_dev_world *D);
 
 // Make D's stream wait for the last half step of the auxiliary worlds (on other streams) whose
 // strips apply.
@@ -2363,7 +2412,7 @@ int waitForAux(alis_dev_world *D, unsigned strips)
 	for (size_t s = 0; s < D->tf.size(); s++) {
 		alis_dev_world *X = D->tf[s].aux;
 		if (!((strips >> s) & 1u)) continue;
-		if ((X->pendMain || X->pendPost) && flushE(X)) return -1;
+		if ((X->pendMain || X->pendPost) && flushFields(X)) return -1;
 		if (X->st == D->st) continue;
 		if (!X->halfDone) {
 			HIPCHECK(hipEventCreateWithFlags(&X->halfDone, hipEventDisableTiming));
@@ -2371,17 +2420,6 @@ int waitForAux(alis_dev_world *D, unsigned strips)
 		}
 		HIPCHECK(hipStreamWaitEvent(D->st, X->halfDone, 0));
 	}
-	return 0;
-}
-
-// The current update of the last H core, where no end-of-half-step launch took it along.
-template<class T>
-int flushAde(alis_dev_world *D)
-{
-	if (!D->pendAde) return 0;
-	D->pendAde = false;
-	k_ade<T><<<objBlocks(D), OBJ_WG, 0, D->st>>>(objArgs<T>(D));
-	HIPCHECK(hipGetLastError());
 	return 0;
 }
 
@@ -2541,15 +2579,15 @@ int postHalf(alis_dev_world *D, int h, int made, const PostArgs<T> *x)
 		a.pieces = (const PostPiece *)G.pieces;
 		a.post = (int)groups(G);
 		unsigned blocks = a.post;
-		if (g == last && h == 1 && D->pendAde) a.ade = objArgs<T>(D), blocks += objBlocks(D), D->pendAde = false;
-		if (g == last && x) launchEv(k_post_aux<T>, dim3(blocks + x->post), dim3(POST_WG), 0, D->st, nullptr, bind ? D->halfDone : nullptr, a, *x, (int)blocks);
-		else if (g == last) launchEv(k_post<T>, dim3(blocks), dim3(POST_WG), 0, D->st, nullptr, bind ? D->halfDone : nullptr, a);
-		else k_post<T><<<blocks, POST_WG, 0, D->st>>>(a);
+		if (g == last && h == 1 && D->pendAde && updateBeside(D)) a.ade = objArgs<T>(D), blocks += objBlocks(D), D->pendAde = false;
+		const bool ade = blocks > (unsigned)a.post;
+		if (g == last && x) launchEv(ade ? k_post_aux<T, true> : k_post_aux<T, false>, dim3(blocks + x->post), dim3(POST_WG), 0, D->st, nullptr, bind ? D->halfDone : nullptr, a, *x, (int)blocks);
+		else if (g == last) launchEv(ade ? k_post<T, true> : k_post<T, false>, dim3(blocks), dim3(POST_WG), 0, D->st, nullptr, bind ? D->halfDone : nullptr, a);
+		else k_post<T, false><<<blocks, POST_WG, 0, D->st>>>(a);
 		HIPCHECK(hipGetLastError());
 	}
-	if (last < 0 && flushAde<T>(D)) return -1;
 	if (last < 0 && x) {
-		k_post<T><<<x->post, POST_WG, 0, D->st>>>(*x);
+		k_post<T, false><<<x->post, POST_WG, 0, D->st>>>(*x);
 		HIPCHECK(hipGetLastError());
 	}
 	if (last < 0 && bind) HIPCHECK(hipEventRecord(D->halfDone, D->st));
@@ -2761,7 +2799,7 @@ int fusedStep(alis_dev_world *D)
 	for (size_t s = 0; s < D->tf.size(); s++) side = side || (((strips >> s) & 1u) && D->tf[s].aux->st != D->st);
 	if (side && !D->halfDone) HIPCHECK(hipEventCreateWithFlags(&D->halfDone, hipEventDisableTiming));
 	// the objects' currents, into the set that this step replaces
-	if (D->objWgs) k_currents<T><<<objBlocks(D), OBJ_WG, 0, D->st>>>(objArgs<T>(D));
+	if (objectsBeforeE<T>(D)) return -1;
 	const StepShape z = stepShape(D);
 	const dim3 grid((unsigned)z.blocks), block(STEP_THREADS);
 	const size_t lds = z.lds;
@@ -2805,13 +2843,9 @@ int fusedStep(alis_dev_world *D)
 		a.ops = (const PostOp<T> *)G.ops;
 		a.pieces = (const PostPiece *)G.pieces;
 		a.post = (int)G.total;
-		unsigned blocks = a.post;
-		a.ade = ObjArgs<T>{};
-		if (D->pendAde) a.ade = objArgs<T>(D), blocks += objBlocks(D), D->pendAde = false;
-		k_post<T><<<blocks, POST_WG, 0, D->st>>>(a);
+		k_post<T, false><<<a.post, POST_WG, 0, D->st>>>(a);
 		HIPCHECK(hipGetLastError());
 	}
-	if (flushAde<T>(D)) return -1;
 	forgetRecorded(D, 0), forgetRecorded(D, 1);
 	for (size_t s = 0; side && s < D->tf.size(); s++)
 		if (((strips >> s) & 1u) && D->tf[s].aux->st != D->st) HIPCHECK(hipStreamWaitEvent(D->tf[s].aux->st, D->halfDone, 0));
@@ -2834,8 +2868,7 @@ int auxHalves(alis_dev_world *D)
 
 int batchFlush(alis_dev_batch *B);
 
-// Whether a part of D's half step waits for a later call (other than the objects' current update, which an
-// H program takes along).
+// Whether a part of D's half step waits for a later call (other than the objects' current update).
 bool halfWaits(const alis_dev_world *D)
 {
 	return D->pendE || D->pendH || D->pendCore || D->pendMain || D->pendPost || D->pendBatch;
@@ -2856,22 +2889,29 @@ int flushStep(alis_dev_world *D)
 		const bool core = A && A->pendCore, ghosts = A && A->pendGhosts;
 		D->pendMain = 0, D->pendFold = false;
 		if (A) A->pendCore = A->pendGhosts = 0;
-		if (coreHalf<T>(D, h) || flushAde<T>(D)) return -1;
+		if (coreHalf<T>(D, h)) return -1;
 		if (core && coreHalf<T>(A, h)) return -1;
 		return ghosts ? postHalf<T>(A, h) : 0;
 	}
 	const int p = D->pendE;
-	if (!p) return flushAde<T>(D);
+	if (!p) return 0;
 	D->pendE = 0;
 	if (coreHalf<T>(D, 0)) return -1;
 	if (p >= 2 && postHalf<T>(D, 0)) return -1;
-	if (p >= 3 && (coreHalf<T>(D, 1) || flushAde<T>(D))) return -1;
+	if (p >= 3 && coreHalf<T>(D, 1)) return -1;
 	return auxHalves<T>(D);
 }
 
-int flushE(alis_dev_world *D)
+int flushFields(alis_dev_world *D)
 {
 	return D->fp64 ? flushStep<double>(D) : flushStep<float>(D);
+}
+
+// And the current update of D's objects: for calls that read the currents, or change E.
+int flushE(alis_dev_world *D)
+{
+	if (flushFields(D)) return -1;
+	return D->fp64 ? flushAde<double>(D) : flushAde<float>(D);
 }
 
 template<class T>
@@ -2933,7 +2973,7 @@ int ghostsEntry(alis_dev_world *D, int h)
 		D->pendH = 2;
 		return 0;
 	}
-	if ((h == 0 || halfWaits(D)) && flushStep<T>(D)) return -1;   // (an H program takes its current update along)
+	if ((halfWaits(D) && flushStep<T>(D)) || (h == 0 && flushAde<T>(D))) return -1;     // (it changes E)
 	return postHalf<T>(D, h);
 }
 
@@ -3434,6 +3474,7 @@ struct alis_dev_batch {
 	std::vector<CurlClass> curlClass[2];
 	void *objArgs = nullptr, *objStart = nullptr;   // ObjArgs<T>[] of the worlds with objects
 	int objEntries = 0, objBlocks = 0;
+	long bytes = 0;             // that a step of its worlds passes over (stepBytes)
 	int pend = 0;               // 1 + h: the core of half step h waits for its post
 	// ALIS_BATCH_PAIRS=0 with Bloch worlds: their parts are entries of one launch, side by side, and a
 	// ghost copy between the parts reads and writes both, so the curls make none
@@ -3538,6 +3579,7 @@ int batchBuildObjects(alis_dev_batch *B)
 	std::vector<ObjArgs<T>> args;
 	std::vector<int> start;
 	for (alis_dev_world *D : B->W) {
+		B->bytes += stepBytes(D);
 		if (!D->objWgs) continue;
 		args.push_back(objArgs<T>(D));
 		start.push_back(B->objBlocks);
@@ -3566,8 +3608,6 @@ int batchBuildPost(alis_dev_batch *B, bool copied)
 				alis_dev_world *D = B->W[w];
 				if (r >= D->post[h].size()) continue;
 				long blocks = copied ? D->post[h][r].rest : D->post[h][r].total;
-				// the current update runs with a world's last H launch
-				if (h == 1 && r + 1 == D->post[h].size()) blocks += objBlocks(D);
 				if (!blocks) continue;
 				R.world.push_back(w), R.seg.push_back((int)r);
 				start.push_back((int)R.blocks);
@@ -3605,15 +3645,24 @@ int batchCore(alis_dev_batch *B, int h, bool copies, const FetchArgs &next = Fet
 	alis_dev_world *D0 = B->W[0];
 	for (alis_dev_world *W : B->W) {
 		dropPresamples(W);
-		if (flushStep<T>(W)) return -1;
-		if (h == 1) W->pendAde = W->objWgs > 0;   // with the end of the half step (or flushStep)
+		if (flushStep<T>(W) || (h == 1 && flushAde<T>(W))) return -1;
+		if (h == 1) W->pendAde = W->objWgs > 0;
 	}
 	hipEvent_t e0 = nullptr, e1 = nullptr;
 	if (D0->timing) {
 		if (timingEvents(D0, e0, e1)) return -1;
 	}
 	if (h == 0 && B->objEntries) {
-		k_currents_batch<T><<<B->objBlocks, OBJ_WG, 0, B->st>>>((const ObjArgs<T> *)B->objArgs, (const int *)B->objStart, B->objEntries);
+		// with the current update where no world's has been made apart
+		const bool update = std::all_of(B->W.begin(), B->W.end(), [](const alis_dev_world *W) { return !W->objWgs || W->pendAde; });
+		for (alis_dev_world *W : B->W) {
+			if (!update && flushAde<T>(W)) return -1;
+			W->pendAde = false;
+		}
+		const ObjArgs<T> *args = (const ObjArgs<T> *)B->objArgs;
+		if (!update) k_currents_batch<T><<<B->objBlocks, OBJ_WG, 0, B->st>>>(args, (const int *)B->objStart, B->objEntries);
+		else if (B->bytes > OBJECTS_NT) k_objects_batch<T, true><<<B->objBlocks, OBJ_WG, 0, B->st>>>(args, (const int *)B->objStart, B->objEntries);
+		else k_objects_batch<T, false><<<B->objBlocks, OBJ_WG, 0, B->st>>>(args, (const int *)B->objStart, B->objEntries);
 		HIPCHECK(hipGetLastError());
 	}
 	const std::vector<alis_dev_batch::CurlClass> &cls = B->curlClass[h];
@@ -3642,10 +3691,9 @@ int batchCore(alis_dev_batch *B, int h, bool copies, const FetchArgs &next = Fet
 	return 0;
 }
 
-// The arguments of the end of half step h into pinned memory; whole: the current update of H is one of
-// them although its core is still to come; copied: the curl makes the copies that it can.
+// The arguments of the end of half step h into pinned memory; copied: the curl makes the copies that it can.
 template<class T>
-int batchPostArgs(alis_dev_batch *B, int h, bool whole, bool copied)
+int batchPostArgs(alis_dev_batch *B, int h, bool copied)
 {
 	if (batchPrograms<T>(B) || (!B->postReady[copied] && batchBuildPost<T>(B, copied))) return -1;
 	if (!B->postBytes[copied][h]) return 0;
@@ -3660,7 +3708,6 @@ int batchPostArgs(alis_dev_batch *B, int h, bool whole, bool copied)
 			a[e].ops = (const PostOp<T> *)g.ops;
 			a[e].pieces = (const PostPiece *)g.pieces;
 			a[e].post = (int)(copied ? g.rest : g.total);
-			if (h == 1 && R.seg[e] + 1 == (int)D->post[h].size() && (whole ? D->objWgs > 0 : D->pendAde)) a[e].ade = objArgs<T>(D);
 			a[e].strips = D->pendStrips[h];
 			for (size_t w = 0; w < D->pendSrc[h].size(); w++) a[e].src[w] = D->pendSrc[h][w];
 			for (size_t q = 0; q < D->pendWave[h].size(); q++) a[e].wave[q] = (T)D->pendWave[h][q];
@@ -3674,7 +3721,8 @@ template<class T>
 int batchPost(alis_dev_batch *B, int h, bool whole)
 {
 	const bool copied = whole && !B->apart;
-	if (batchPostArgs<T>(B, h, whole, copied)) return -1;
+	for (alis_dev_world *W : B->W) if (h == 0 && !whole && flushAde<T>(W)) return -1;     // (it changes E)
+	if (batchPostArgs<T>(B, h, copied)) return -1;
 	const size_t bytes = B->postBytes[copied][h];
 	if (whole) {
 		FetchArgs next{};
@@ -3686,11 +3734,8 @@ int batchPost(alis_dev_batch *B, int h, bool whole)
 		if (R.world.empty()) continue;
 		k_post_batch<T><<<R.blocks, POST_WG, 0, B->st>>>((const PostArgs<T> *)R.args, (const int *)R.start, (int)R.world.size());
 		HIPCHECK(hipGetLastError());
-		for (size_t e = 0; e < R.world.size(); e++)
-			if (h == 1 && ((const PostArgs<T> *)R.pinned)[e].ade.blocks) B->W[R.world[e]]->pendAde = false;
 	}
 	for (alis_dev_world *D : B->W) {
-		if (h == 1 && flushAde<T>(D)) return -1;     // a world without an H program
 		forgetRecorded(D, h);
 	}
 	return 0;
@@ -3703,7 +3748,6 @@ int batchFlush(alis_dev_batch *B)
 	B->pend = 0;
 	for (alis_dev_world *W : B->W) W->pendBatch = nullptr;
 	if (B->fp64 ? batchCore<double>(B, h, false) : batchCore<float>(B, h, false)) return -1;
-	for (alis_dev_world *W : B->W) if (B->fp64 ? flushAde<double>(W) : flushAde<float>(W)) return -1;
 	return 0;
 }
 
@@ -3899,7 +3943,7 @@ void gatherWorld(alis_dev_world *D, const Box &box, int mask, std::vector<Gather
 
 int alis_dev_sync_boxes(alis_dev_world *const *D, const int *box, int n)
 {
-	for (int e = 0; e < n; e++) if (flushE(D[e])) return -1;
+	for (int e = 0; e < n; e++) if (box[7 * e + 6] & ALIS_DEV_PROBE_CURRENTS ? flushE(D[e]) : flushFields(D[e])) return -1;
 	if (n < 1) return 0;
 	std::vector<GatherSeg> seg;
 	std::vector<GatherHost> out;
@@ -3963,7 +4007,7 @@ int alis_dev_sync_boxes(alis_dev_world *const *D, const int *box, int n)
 
 int alis_dev_read_field(alis_dev_world *D, int h, int m, int axis, double *out)
 {
-	if (flushE(D)) return -1;
+	if (flushFields(D)) return -1;
 	if (m > D->cplx || h < 0 || h > 1 || axis < 0 || axis > 2) return fail("no such field array");
 	return D->fp64 ? readField<double>(D, h, m, axis, out) : readField<float>(D, h, m, axis, out);
 }
@@ -3979,7 +4023,7 @@ int alis_dev_write_field(alis_dev_world *D, int h, int m, int axis, const double
 
 int alis_dev_phaser_add(alis_dev_world *D, const alis_dev_phaser_desc *P, int *id)
 {
-	if (flushE(D)) return -1;
+	if (flushFields(D)) return -1;
 	DevPhaser Q;
 	Q.nf = P->nf;
 	Q.iMin = P->iMin, Q.iMax = P->iMax, Q.jMin = P->jMin, Q.jMax = P->jMax, Q.kMin = P->kMin, Q.kMax = P->kMax;
@@ -4045,7 +4089,7 @@ int alis_dev_phaser_add(alis_dev_world *D, const alis_dev_phaser_desc *P, int *i
 
 int alis_dev_phaser_update(alis_dev_world *D, int id, int q0, int nq, const double *expE, const double *expH)
 {
-	if (flushE(D)) return -1;
+	if (flushFields(D)) return -1;
 	if (id < 0 || id >= (int)D->phs.size() || !D->phs[id].live) return fail("no such phaser");
 	DevPhaser &P = D->phs[id];
 	if (q0 < 0 || nq < 0 || q0 + nq > P.nf) return fail("phaser frequency range out of bounds");
@@ -4057,7 +4101,7 @@ int alis_dev_phaser_update(alis_dev_world *D, int id, int q0, int nq, const doub
 int alis_dev_phaser_update_many(alis_dev_world *const *D, const int *id, const int *q0, const int *nq,
                                 const double *const *expE, const double *const *expH, int n)
 {
-	for (int e = 0; e < n; e++) if (flushE(D[e])) return -1;
+	for (int e = 0; e < n; e++) if (flushFields(D[e])) return -1;
 	if (n < 1) return 0;
 	for (int e = 0; e < n; e++) {
 		if (id[e] < 0 || id[e] >= (int)D[e]->phs.size() || !D[e]->phs[id[e]].live) return fail("no such phaser");
@@ -4080,7 +4124,7 @@ long alis_dev_phaser_size(alis_dev_world *D, int id)
 
 int alis_dev_phaser_read(alis_dev_world *D, int id, double *out, long n)
 {
-	if (flushE(D)) return -1;
+	if (flushFields(D)) return -1;
 	long need = alis_dev_phaser_size(D, id);
 	if (need < 0 || n < need) return fail("phaser read buffer too small");
 	DevPhaser &P = D->phs[id];
@@ -4183,7 +4227,7 @@ int fluxScratch(alis_dev_world *D, double **out)
 int alis_dev_phaser_flux_sums(alis_dev_world *D, int id, int q, int nterm, const int *terms,
                               const double *w, long nw, double *out, long nout)
 {
-	if (flushE(D)) return -1;
+	if (flushFields(D)) return -1;
 	FluxPlan F;
 	if (fluxPlan(D, id, q, 1, nterm, terms, nw, nout, F)) return -1;
 	if (ensureScratch(D, F.doubles)) return -1;
@@ -4193,7 +4237,7 @@ int alis_dev_phaser_flux_sums(alis_dev_world *D, int id, int q, int nterm, const
 int alis_dev_phaser_flux_sums_range(alis_dev_world *D, int id, int q0, int nq, int nterm, const int *terms,
                                     const double *w, long nw, double *out, long nout)
 {
-	if (flushE(D)) return -1;
+	if (flushFields(D)) return -1;
 	FluxPlan F;
 	if (fluxPlan(D, id, q0, nq, nterm, terms, nw, nout, F)) return -1;
 	if (ensureScratch(D, F.doubles)) return -1;
@@ -4203,7 +4247,7 @@ int alis_dev_phaser_flux_sums_range(alis_dev_world *D, int id, int q0, int nq, i
 int alis_dev_phaser_flux_sums_noalloc(alis_dev_world *D, int id, int q, int nterm, const int *terms,
                                       const double *w, long nw, double *out, long nout)
 {
-	if (flushE(D)) return -1;
+	if (flushFields(D)) return -1;
 	FluxPlan F;
 	if (fluxPlan(D, id, q, 1, nterm, terms, nw, nout, F)) return -1;
 	if (F.doubles > FLUX_SCRATCH_DOUBLES)
@@ -4216,7 +4260,7 @@ int alis_dev_phaser_flux_sums_noalloc(alis_dev_world *D, int id, int q, int nter
 
 int alis_dev_phaser_sync(alis_dev_world *D, int id)
 {
-	if (flushE(D)) return -1;
+	if (flushFields(D)) return -1;
 	long need = alis_dev_phaser_size(D, id);
 	if (need < 0) return fail("no such phaser");
 	DevPhaser &Q = D->phs[id];
@@ -4641,7 +4685,7 @@ int alis_dev_farfield(alis_dev_world *D, int id, int q, const alis_dev_ff_geom *
 
 int alis_dev_batch_create(alis_dev_world *const *D, int n, alis_dev_batch **out)
 {
-	for (int w = 0; w < n; w++) if (flushE(D[w])) return -1;
+	for (int w = 0; w < n; w++) if (flushFields(D[w])) return -1;
 	*out = nullptr;
 	if (n < 1) return fail("empty batch");
 	alis_dev_batch *B = new alis_dev_batch;
@@ -4679,7 +4723,7 @@ int alis_dev_batch_core(alis_dev_batch *B, int h)
 {
 	if (h < 0 || h > 1) return fail("no such half step");
 	if (batchStream(B)) return -1;
-	for (alis_dev_world *W : B->W) if (flushE(W)) return -1;
+	for (alis_dev_world *W : B->W) if (flushFields(W)) return -1;
 	for (alis_dev_world *W : B->W) if (W->lastCells[h]) return B->fp64 ? batchCore<double>(B, h, false) : batchCore<float>(B, h, false);
 	B->pend = 1 + h;
 	for (alis_dev_world *W : B->W) W->pendBatch = B;
@@ -4696,7 +4740,7 @@ int alis_dev_batch_post(alis_dev_batch *B, int h)
 		for (alis_dev_world *W : B->W) W->pendBatch = nullptr;
 	}
 	else
-		for (alis_dev_world *W : B->W) if (halfWaits(W) && flushE(W)) return -1;
+		for (alis_dev_world *W : B->W) if (halfWaits(W) && flushFields(W)) return -1;
 	return B->fp64 ? batchPost<double>(B, h, whole) : batchPost<float>(B, h, whole);
 }
 
@@ -4777,7 +4821,7 @@ int absorption(alis_dev_world *D, int n, const Box &b, const double *dzE, const 
 
 int alis_dev_plane_sums(alis_dev_world *D, int nterm, const int *terms, const double *w, long nw, double *out, long nout)
 {
-	if (flushE(D)) return -1;
+	if (flushFields(D)) return -1;
 	if (nterm < 1 || nw < 1 || nout < 1) return fail("plane sums: no terms or no buffers");
 	return D->fp64 ? planeSums<double>(D, nterm, terms, w, nw, out, nout) : planeSums<float>(D, nterm, terms, w, nw, out, nout);
 }
@@ -4894,7 +4938,7 @@ void alis_dev_spectrum_release(alis_dev_spectrum *S)
 
 int alis_dev_three_wave(alis_dev_world *S, alis_dev_world *P1, alis_dev_world *P2, int n, const float *d, float alt)
 {
-	if (flushE(S) || flushE(P1) || flushE(P2)) return -1;
+	if (flushE(S) || flushFields(P1) || flushFields(P2)) return -1;
 	dropPresamples(S);
 	if (S == P1 || S == P2) return fail("three-wave coupling: the signal world is one of the pumps");
 	for (alis_dev_world *P : {P1, P2})
@@ -4965,7 +5009,7 @@ int alis_dev_timing(alis_dev_world *D, int enable)
 int alis_dev_timing_read(alis_dev_world *D, int h, double *ms, long *launches)
 {
 	if (h < 0 || h > 2) return fail("no such timed launch");
-	if (flushE(D)) return -1;
+	if (flushFields(D)) return -1;
 	HIPCHECK(hipStreamSynchronize(D->st));
 	auto &v = D->evPairs[h];
 	for (size_t a = 0; a + 1 < v.size(); a += 2) {

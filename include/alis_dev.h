@@ -104,8 +104,10 @@ void alis_dev_release(alis_dev_world *D);
  * both halves in one pass over the grid (k_step, strips and sources included) followed by the
  * ghost copies; the results are those of the separate half steps, bit for bit.
  * Otherwise the core waits for the alis_dev_ghosts of its half step, whose work its launch shares
- * (ghost copies, sources, the half step of a small TF/SF auxiliary world), and E's last ghost
- * copies may wait for H's.  Errors of what waits come from the call that runs it.
+ * (ghost copies, sources, the half step of a small TF/SF auxiliary world), E's last ghost
+ * copies may wait for H's, and the current update of an H core for the next E core, which passes over the
+ * same values.  A core whose source has per-cell waves is launched at its call, and runs while the
+ * caller evaluates those.  Errors of what waits come from the call that runs it.
  * Any other call on the world (or on a world that reads it) first completes what is deferred
  * the separate way. */
 int alis_dev_core(alis_dev_world *D, int h);

@@ -5,7 +5,7 @@
 #include "alis.h"
 #include "../alis_amd/host/internal.h"
 
-/* percent: the boxes' edges, of the domain's. */
+/* sphere: its radius in 4 cells, 0 for none; percent: the boxes' edges, of the domain's. */
 world ec_boxes(int cells, int boxes, int sphere, int percent)
 {
 	const float half = 0.01f * percent;
@@ -15,7 +15,8 @@ world ec_boxes(int cells, int boxes, int sphere, int percent)
 	sur S = {{PML}, {PML}, {PML}, {8}};
 	world W = createWorld(D, R, S, "");
 	matter Gold = {{1.5}, {{9, 0.07}, {2.6, 0.3, 0.5}, {3.5, 0.6, 0.8}}};
-	object Sphere = {Ball, {{-4 * dx, 4 * dx}, {-4 * dx, 4 * dx}, {-4 * dx, 4 * dx}}};
+	const float r = 4 * sphere * dx;
+	object Sphere = {Ball, {{-r, r}, {-r, r}, {-r, r}}};
 	if (sphere) putObjects(W, Gold, Sphere, Air);
 	for (int b = 0; b < boxes; b++) {
 		const float x = -0.8f * e + 1.6f * e * b / boxes;
@@ -101,4 +102,26 @@ world ec_plane(int cells)
 	focusedBeam(W, W->Dom, Ex, 0, 0, 0, 0, Sine, 600, 3);
 	pointDipole(W, Ez, 3 * dx, -5 * dx, dx, Pulse, 600, 240);
 	return W;
+}
+
+/* Overlapping dispersive objects of one, three and two poles around a point dipole, 10 scale cells wide. */
+world ec_objects(int cells, int scale)
+{
+	world W = ec_boxes(cells, 0, 0, 60);
+	matter Gold = {{1.5}, {{9, 0.07}, {2.6, 0.3, 0.5}, {3.5, 0.6, 0.8}}}, Metal = {{1}, {{9, 0.07}}}, Glass = {{2}, {{2.6, 0.3, 0.5}, {3.1, 0.2, 0.4}}};
+	const float s = scale;
+	object A = {Box, {{-83 * s, 21 * s}, {-55 * s, 47 * s}, {-71 * s, 33 * s}}}, B = {Ball, {{-50 * s, 60 * s}, {-50 * s, 60 * s}, {-47 * s, 63 * s}}},
+	       C = {Box, {{-15 * s, 75 * s}, {-90 * s, 25 * s}, {-15 * s, 95 * s}}};
+	putObjects(W, Metal, A, Gold, B, Glass, C, Air);
+	return W;
+}
+
+/* n worlds stepped together, or one by one (together 0), their currents read after every third step. */
+void ec_step_read(world *W, int n, int steps, int together)
+{
+	for (int s = 0; s < steps; s++) {
+		if (together) updateWorldsE(W, n), updateWorldsH(W, n);
+		else for (int a = 0; a < n; a++) updateE(W[a]), updateH(W[a]);
+		if (s % 3 == 2) alisFatal("sync", alis_dev_sync(W[s % n]->dev, 0, -1, 0, -1, 0, -1));
+	}
 }

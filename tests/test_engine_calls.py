@@ -359,3 +359,40 @@ main = max((c for c in log if c[0] == "launch" and c[1].startswith("k_curl")), k
 post = [c[3] for c in log if c[0] == "launch" and c[4] == main and c[1].startswith("k_post")]
 assert len(post) == 2 and post[0] >= 12500 * 0.9 / 64, post
 """)
+
+
+@pytest.mark.parametrize("shared", [False, True])
+def test_objects_are_passed_over_once_a_step(libs, shared):
+    """Objects of more than a workgroup per compute unit: the current update of an H half step runs with what the objects do before the next E curl, in one
+    launch; apart from it only where a call in between reads the currents or changes E."""
+    run(libs, f"""
+shared = {shared}
+W = [V(ec.ec_world(64, 0, 5)) for _ in range(2)]
+for w in W:
+    ec.ec_step(w, 2)
+dev = [ec.ec_device(w) for w in W]
+B = batch(dev) if shared else None
+both = "k_objects_batch" if shared else "k_objects"           # (update and currents)
+currents = "k_currents_batch" if shared else "k_currents"
+core = lambda h: ok(lib.alis_dev_batch_core(B, h) if shared else lib.alis_dev_core(dev[0], h))
+end = lambda h: ok(lib.alis_dev_batch_post(B, h) if shared else lib.alis_dev_ghosts(dev[0], h))
+half = lambda h: (core(h), end(h))
+objects = lambda k: [n for n in k if n in ("k_ade", both, currents)]
+read = lambda d: ok(lib.alis_dev_read_field(V(d), 0, 0, 2, buf))
+buf = (ctypes.c_double * 400000)()
+lib.alis_dev_read_field.argtypes = [V, I, I, I, V]
+half(0), half(1)
+for between in ("nothing", "fields", "currents", "ghosts"):
+    assert objects(kernels(calls(half, 0))) == [both], between
+    assert objects(kernels(calls(half, 1))) == [], between
+    if between == "fields":              # (the fields do not depend on it)
+        assert objects(kernels(calls(read, dev[0]))) == []
+    if between == "currents":
+        assert objects(kernels(calls(lambda: ok(lib.alis_dev_sync(dev[0], 0, -1, 0, -1, 0, -1))))) == ["k_ade"]
+        apart = objects(kernels(calls(half, 0)))
+        assert apart == (["k_ade", currents] if shared else [currents])
+        half(1)
+    if between == "ghosts":              # E's ghost copies without a core
+        k = objects(kernels(calls(end, 0)))
+        assert k == ["k_ade"] * (2 if shared else 1), k
+""")

@@ -79,19 +79,21 @@ def test_half_steps_of_single_and_shared_calls(program):
     assert np.abs(ref).max() > 0 and np.array_equal(got, ref)
 
 
-BEAMS = r'''
+WORLDS_OF = r'''
 import ctypes, sys
 import numpy as np
 V, I = ctypes.c_void_p, ctypes.c_int
 ctypes.CDLL(sys.argv[2], mode=ctypes.RTLD_GLOBAL)
 ec = ctypes.CDLL(sys.argv[1])
-ec.ec_beam.restype = ec.ec_plane.restype = V
+ec.ec_beam.restype = ec.ec_plane.restype = ec.ec_objects.restype = V
 ec.ec_field.restype = ctypes.c_long
-ec.ec_step.argtypes, ec.ec_step_many.argtypes = [V, I], [V, I, I]
+ec.ec_step.argtypes, ec.ec_step_many.argtypes, ec.ec_step_read.argtypes = [V, I], [V, I, I], [V, I, I, I]
 ec.ec_field.argtypes = [V, I, I, V, ctypes.c_long]
 mode = sys.argv[4]
-W = (V * 1)(ec.ec_plane(730)) if mode == "plane" else (V * 2)(*[ec.ec_beam(n, 20) for n in (40, 43)])
-if mode == "together":
+W = (V * 1)(ec.ec_plane(730)) if mode == "plane" else (V * 2)(*[ec.ec_objects(2 * n if "large" in mode else n, 3 if "large" in mode else 1) if "objects" in mode else ec.ec_beam(n, 20) for n in (40, 43)])
+if "objects" in mode:
+    ec.ec_step_read(W, 2, 31, "together" in mode)
+elif mode == "together":
     ec.ec_step_many(W, 2, 45)
 else:
     for w in W:
@@ -114,10 +116,31 @@ def test_sources_of_many_cells(tmp_path, mode):
     client = tmp_path / "engine_client.so"
     subprocess.run(["gcc", "-O1", "-std=gnu99", "-shared", "-fPIC", f"-I{ROOT / 'include'}", "-o", str(client),
                     str(ROOT / "tests" / "engine_client.c")], check=True)
+    _compare(client, tmp_path, mode, "fp32")
+
+
+@pytest.mark.parametrize("mode", ["objects", "objects together", "large objects", "large objects together"])
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+def test_current_updates_apart_and_with_the_next_step(tmp_path, mode, precision):
+    """Overlapping objects: the current update runs beside the end of the H half step (small ones), with the
+    next E half step, or by itself where the currents are read before."""
+    client = tmp_path / "engine_client.so"
+    subprocess.run(["gcc", "-O1", "-std=gnu99", "-shared", "-fPIC", f"-I{ROOT / 'include'}", "-o", str(client),
+                    str(ROOT / "tests" / "engine_client.c")], check=True)
+    _compare(client, tmp_path, mode, precision)
+
+
+def _compare(client, tmp_path, mode, precision):
+    """FP32 bit for bit, FP64 to 1e-12 of the largest value (the bound the parity scenarios have)."""
     got = {}
     for kind in LIBS:
-        print(f"[gpu] {mode}, {kind}", flush=True)
-        subprocess.run([sys.executable, "-c", BEAMS, str(client), str(LIBS[kind][1]), str(tmp_path / f"{kind}.npy"), mode],
-                       check=True, timeout=100, env={**os.environ, "ALIS_PRECISION": "fp32"})
+        print(f"[gpu] {mode}, {kind}, {precision}", flush=True)
+        subprocess.run([sys.executable, "-c", WORLDS_OF, str(client), str(LIBS[kind][1]), str(tmp_path / f"{kind}.npy"), mode],
+                       check=True, timeout=100, env={**os.environ, "ALIS_PRECISION": precision})
         got[kind] = np.load(tmp_path / f"{kind}.npy")
-    assert np.abs(got["oracle"]).max() > 0 and np.array_equal(got["hip"], got["oracle"])
+    big = np.abs(got["oracle"]).max()
+    assert big > 0
+    if precision == "fp32":
+        assert np.array_equal(got["hip"], got["oracle"])
+    else:
+        assert np.abs(got["hip"] - got["oracle"]).max() <= 1e-12 * big
