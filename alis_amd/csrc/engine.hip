@@ -3,10 +3,10 @@
 //
 // Layout in HBM.  Every field component is its own array over
 // [iMIN-1..iMAX+1] x [jMIN-1..jMAX+1] x [kMIN-1..kMAX+1] (ghost layer included), z
-// contiguous, each (i,j) row padded to a multiple of 128 bytes and shifted so that k = kMIN
-// starts on a 128-byte boundary: a 64-lane wavefront reading 64 consecutive k touches
-// exactly two cache lines.  CPML slabs normal to x and y use the same padded rows; slabs
-// normal to z, ADE currents and fill factors are compact over their boxes.
+// contiguous, in rows of whole quads (16 bytes) that lie end to end: k = kMIN starts on a quad,
+// and the ghost below a row is the last value of the row before (fieldLayout).  CPML slabs
+// normal to x and y use the same rows; slabs normal to z, ADE currents and fill factors cover
+// their boxes, widened to the grid's quads (quadLayout).
 //
 // Arithmetic.  Kernels keep the reference's operation order per cell (curl, then the CPML
 // slabs in face order xMin,yMin,zMin,xMax,yMax,zMax; ADE scaling, then -J per pole; strips
@@ -1092,6 +1092,7 @@ struct alis_dev_world {
 	void *stepArgs = nullptr;   // StepArgs<T>[2 parts][2 sets]: k_step's arguments per current set
 	void *objStart = nullptr, *objOver = nullptr;   // tables of the objects' launches (ObjArgs)
 	int objWgs = 0;             // workgroups of one component of one part
+	long stepBytes = 0;         // that a step passes over, but for CPML and 1/eps: fields, objects' arrays
 	bool pendAde = false;       // the current update of the last H core is still to run: beside the
 	                            //  end of its half step (updateBeside), with the next E core, or
 	                            //  before anything that needs it (flushAde)
@@ -1428,11 +1429,11 @@ void buildPieces(const std::vector<PostOp<T>> &v, int nadd, std::vector<PostPiec
 	}
 }
 
-// 1/eps per row segment of k_curl's tiles (64 cells along k): (x, y, z, 1) when every cell
-// of the segment holds the same triple (bit patterns), else zeros.  A wavefront of the E
-// curl covers one segment: on a uniform one it takes 1/eps from this table instead of
-// reading three arrays (most segments of a world lie inside one material; the values, and
-// so the results, are the same).
+// 1/eps per row segment (64 cells along k): (x, y, z, 1) when every cell of the segment holds the
+// same triple (bit patterns), else zeros.  A lane of the E curl looks up the segment of its own
+// quad, and on a uniform one takes 1/eps from this table instead of reading three arrays (most
+// segments of a world lie inside one material; the values, and so the results, are the same).
+// A wavefront covers 64 quads, across row ends, and may hold both kinds.
 template<class T>
 int rowSegments(alis_dev_world *D)
 {
@@ -1459,7 +1460,10 @@ int rowSegments(alis_dev_world *D)
 				else mixedCells += k1 - k0 + 1;
 			}
 	// a table that spares the arrays in under a quarter of the cells (rows that all cross
-	// material boundaries) only adds its own reads: the curl then reads the arrays alone
+	// material boundaries) only adds its own reads: the curl then reads the arrays alone.  E curl with
+	// the arrays over that with the table, 128^3 to 256^3, FP32 and FP64, mixed cells in one half of
+	// the world or spread over it: 1.05-1.09 at one half, 1.01-1.04 at three quarters, 1.00-1.02 at
+	// nine tenths, 0.98-1.00 where all are mixed
 	const double cells = (double)D->iNUM * D->jNUM * D->kNUM;
 	(void)uniform;
 	if (mixedCells > 0.75 * cells) return 0;
@@ -1509,6 +1513,7 @@ int commitWorld(alis_dev_world *D)
 	const alis_dev_world_desc *W = &D->W;
 	D->L = fieldLayout(D);
 	D->fsize = (long)(D->iNUM + 2) * D->L.si + 2 * D->L.koff;
+	D->stepBytes = 6L * (1 + D->cplx) * D->fsize * (long)sizeof(T);
 	const Box fb = fieldBox(D);
 
 	for (int h = 0; h < 2; h++)
@@ -1638,7 +1643,10 @@ int commitWorld(alis_dev_world *D)
 	}
 	if (!D->obj.empty()) {
 		std::vector<int> start, over(2 * D->obj.size() + 1);
-		for (const DevObj &O : D->obj) start.push_back(D->objWgs), D->objWgs += (int)blocksFor(O.n / Quads<T>::N, OBJ_WG);
+		for (const DevObj &O : D->obj) {
+			start.push_back(D->objWgs), D->objWgs += (int)blocksFor(O.n / Quads<T>::N, OBJ_WG);
+			D->stepBytes += 3 * O.n * (1 + (1 + D->cplx) * (2L * O.NK - O.NJ)) * (long)sizeof(T);
+		}
 		for (size_t n = 0; n < D->obj.size(); n++)
 			for (size_t q = 0; q <= D->obj.size(); q++) {
 				if (q == 0) over[2 * n] = (int)over.size();
@@ -1764,14 +1772,6 @@ int flushAde(alis_dev_world *D)
 	return 0;
 }
 
-// The bytes of D that a step passes over, but for CPML and 1/eps: its fields, its objects' arrays.
-long stepBytes(const alis_dev_world *D)
-{
-	long n = 6L * (1 + D->cplx) * D->fsize;
-	for (const DevObj &O : D->obj) n += 3 * O.n * (1 + (1 + D->cplx) * (2L * O.NK - O.NJ));
-	return n * (long)D->esz;
-}
-
 // Objects' arrays bypass the cache (256 MiB, the last level) where a step passes over more than it holds
 // with what else there is.  Worlds by their MiB, us a step cached and past the cache: 64 spheres in 200^3
 // (290) 33 and 37 a launch, metal 160^3 (190) 113 and 115, 4/5 of 200^3 (280) 167 and 168; metal 200^3 (370)
@@ -1784,7 +1784,7 @@ int objectsBeforeE(alis_dev_world *D)
 {
 	if (!D->objWgs) return 0;
 	if (!D->pendAde) k_currents<T><<<objBlocks(D), OBJ_WG, 0, D->st>>>(objArgs<T>(D));
-	else if (stepBytes(D) > OBJECTS_NT) k_objects<T, true><<<objBlocks(D), OBJ_WG, 0, D->st>>>(objArgs<T>(D));
+	else if (D->stepBytes > OBJECTS_NT) k_objects<T, true><<<objBlocks(D), OBJ_WG, 0, D->st>>>(objArgs<T>(D));
 	else k_objects<T, false><<<objBlocks(D), OBJ_WG, 0, D->st>>>(objArgs<T>(D));
 	D->pendAde = false;
 	HIPCHECK(hipGetLastError());
@@ -3579,7 +3579,7 @@ int batchBuildObjects(alis_dev_batch *B)
 	std::vector<ObjArgs<T>> args;
 	std::vector<int> start;
 	for (alis_dev_world *D : B->W) {
-		B->bytes += stepBytes(D);
+		B->bytes += D->stepBytes;
 		if (!D->objWgs) continue;
 		args.push_back(objArgs<T>(D));
 		start.push_back(B->objBlocks);
@@ -3817,8 +3817,9 @@ int alis_dev_link_tfsf(alis_dev_world *D, int s, alis_dev_world *aux)
 	D->postBuilt = D->postBuiltAlt = false;
 	D->fuseState = 0, D->foldState = 0, D->stepArgs = nullptr;
 	aux->isAux = true, aux->mainOf = D;
-	// The auxiliary world keeps its own stream, so its half steps run beside the main
-	// world's curl launches; postHalf orders its strips against them with events.
+	// A small auxiliary world steps inside D's launches, on D's stream (foldsAux).  Any other keeps
+	// its own, and its half steps run beside D's curl launches; postHalf orders its strips against
+	// them with events.
 	return 0;
 }
 

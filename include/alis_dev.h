@@ -287,7 +287,9 @@ int alis_dev_synchronize(alis_dev_world *D);
 
 /* Timing of the curl kernels with device events on the world's stream: enable (resets the
  * totals) or disable, then read total milliseconds and launch count per half (h = 0 E,
- * 1 H) or of the fused step kernel (h = 2, see alis_dev_core). */
+ * 1 H) or of the fused step kernel (h = 2, see alis_dev_core).  What dispersive objects do before
+ * the E curl and after H (their currents and current updates) are launches of their own and not
+ * in these times. */
 int alis_dev_timing(alis_dev_world *D, int enable);
 int alis_dev_timing_read(alis_dev_world *D, int h, double *ms, long *launches);
 
