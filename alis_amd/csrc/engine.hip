@@ -362,7 +362,12 @@ __global__ __launch_bounds__(POST_WG) void k_post(PostArgs<T> a)
 	postBlock<T, ADE>(a, (int)blockIdx.x);
 }
 
-// Several worlds' programs in one launch: entry e owns workgroups [start[e], start[e+1]).
+// Several worlds' programs in one launch: entry e owns workgroups [start[e], start[e+1]).  Launched with
+// POST_BATCH_LDS bytes of LDS that it does not use: they keep 20 workgroups on a compute unit where its
+// registers allow 32, which at ghost copies of many worlds take lines from each other before they are
+// whole (64 Bloch worlds 30.0 -> 24.5 us, 32 of them and six other worlds the same either way; 10 workgroups
+// 26.3, and the six 6.4 -> 8.3).
+constexpr size_t POST_BATCH_LDS = 8192;
 template<class T>
 __global__ __launch_bounds__(POST_WG) void k_post_batch(const PostArgs<T> *__restrict__ args, const int *__restrict__ start, int n)
 {
@@ -3732,7 +3737,7 @@ int batchPost(alis_dev_batch *B, int h, bool whole)
 	else if (bytes) fetchArgs(B->postArgs[copied][h], B->postPinned[copied][h], bytes, B->st, B->postDone[copied][h]);
 	for (alis_dev_batch::Round &R : B->rounds[copied][h]) {
 		if (R.world.empty()) continue;
-		k_post_batch<T><<<R.blocks, POST_WG, 0, B->st>>>((const PostArgs<T> *)R.args, (const int *)R.start, (int)R.world.size());
+		k_post_batch<T><<<R.blocks, POST_WG, POST_BATCH_LDS, B->st>>>((const PostArgs<T> *)R.args, (const int *)R.start, (int)R.world.size());
 		HIPCHECK(hipGetLastError());
 	}
 	for (alis_dev_world *D : B->W) {
